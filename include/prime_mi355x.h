@@ -265,10 +265,11 @@ size_t prime_delta_prefill_workspace_size(int B, int H, int L, unsigned flags);
  *                  forward's clamp [1e-5, 1]
  *   dstate_in    : fp32 [B, H, D, 2D] or NULL
  *   workspace    : prime_delta_prefill_backward_workspace_size(B, H, L, D, chunk)
- *                  bytes (the state entering every chunk, recomputed in fp32;
- *                  outside D = 64 with chunk 64 also one chunk's token states
- *                  per (sequence, head), recomputed chunk by chunk for the
- *                  reverse pass)
+ *                  bytes (per chunk its transfer record, the state entering it
+ *                  and the state's adjoint, in fp32, for as many (sequence,
+ *                  head) pairs as 8 GiB hold and at least one; outside D = 64
+ *                  with chunk 64 the state entering every chunk and one
+ *                  chunk's token states per (sequence, head))
  * fp32 arithmetic throughout.
  */
 size_t prime_delta_prefill_backward_workspace_size(int B, int H, int L, int D, int chunk);

@@ -1252,8 +1252,7 @@ int prime_delta_prefill(const prime_tensor_t *q, const prime_tensor_t *k, const 
 size_t prime_delta_prefill_backward_workspace_size(int B, int H, int L, int D, int chunk) {
     if (B <= 0 || H <= 0 || L <= 0 || D < 1 || D > prime::kDeltaGenMaxD || chunk <= 0) return 0;
     if (delta_generic(D, chunk)) return prime::delta_gen_backward_ws_bytes(B, H, L, D, chunk);
-    const size_t NC = (static_cast<size_t>(L) + prime::kDeltaChunk - 1) / prime::kDeltaChunk;
-    return static_cast<size_t>(B) * H * NC * prime::kDeltaStateBytes;
+    return prime::delta_backward_ws_bytes(B, H, L);
 }
 
 int prime_delta_prefill_backward(const prime_tensor_t *q, const prime_tensor_t *k, const prime_tensor_t *v,

@@ -24,7 +24,7 @@
 //   R0 [8 fb][4 dv][64 lanes]   R0^T accumulator tiles (4 floats per lane)
 //   Y0 [4 dv][4 tb][64 lanes]   Y0^T accumulator tiles
 
-#include "prefill_common.h"
+#include "delta_f32_common.h"
 
 namespace prime {
 namespace {
@@ -40,15 +40,6 @@ static_assert(kFSC + 16 <= static_cast<int>(kDeltaRecBytesF32), "record layout")
 constexpr int kPF = kP + 4;        // phi / psi rows: 16-byte reads of 16 rows fall on distinct bank quads
 constexpr int kPN = kC + 4;        // N, A rows
 constexpr int kPX = 3 * kD + 16;   // X rows: scalar reads of 4 rows x 16 columns meet no bank twice
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
-__device__ __forceinline__ f32x4 ld4(const uint8_t *p) { return *reinterpret_cast<const f32x4 *>(p); }
-__device__ __forceinline__ void st4(float *p, f32x4 v) { *reinterpret_cast<f32x4 *>(p) = v; }
-__device__ __forceinline__ void st4(uint8_t *p, f32x4 v) { *reinterpret_cast<f32x4 *>(p) = v; }
 
 }  // namespace
 
@@ -142,8 +133,8 @@ __global__ __launch_bounds__(256, 1) void delta_prep_f32_kernel(const DeltaArgs 
 
     // ---- N and A (:203-218, :248-250) on the 10 lower 16x16 tiles; wave w takes tiles w, w+4, w+8
     for (int ti = wave; ti < 10; ti += 4) {
-        const int ib = ti < 1 ? 0 : ti < 3 ? 1 : ti < 6 ? 2 : 3;
-        const int jb = ti - ib * (ib + 1) / 2;
+        int ib, jb;
+        lower_tile(ti, ib, jb);
         const float *pa = &sPhi[16 * ib + c16][32 * g];
         const float *sa = &sPsi[16 * ib + c16][32 * g];
         const float *pb = &sPhi[16 * jb + c16][32 * g];
@@ -169,13 +160,9 @@ __global__ __launch_bounds__(256, 1) void delta_prep_f32_kernel(const DeltaArgs 
     }
     __syncthreads();
 
-    // ---- solve T X = [V | diag(e^cum) Phi] (:242-245): thread = one of 192 columns,
-    // forward substitution in registers, each row's sum in four partial sums.
-    // The empty asm statements keep the compiler from hoisting all row reads
-    // to the top or sinking a row's arithmetic to its last use (either spills).
+    // ---- solve T X = [V | diag(e^cum) Phi] (:242-245): thread = one of 192 columns
     if (tid < kD + kP) {
         const int col = tid;
-        const float *nbase = &sN[0][0];
         float x[kC];
         if (col < kD) {
             const float *vp = vf + b * a.v_sb + hk * a.v_sh + col;
@@ -188,22 +175,7 @@ __global__ __launch_bounds__(256, 1) void delta_prep_f32_kernel(const DeltaArgs 
 #pragma unroll
             for (int i = 0; i < kC; ++i) x[i] = sEc[i] * sPhi[i][col - kD];
         }
-#pragma unroll
-        for (int i = 1; i < kC; ++i) {
-            int ro = i * kPN;
-            asm volatile("" : "+v"(ro));
-            float acc[4] = {x[i], 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < i; j += 4) {
-                const f32x4 n4 = ld4(nbase + ro + j);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (j + e < i) acc[e] -= n4[e] * x[j + e];
-            }
-            float r = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            asm volatile("" : "+v"(r));
-            x[i] = r;
-        }
+        solve_unit_lower<kPN>(&sN[0][0], x);
 #pragma unroll
         for (int i = 0; i < kC; ++i) sX[i][col] = x[i];
     }

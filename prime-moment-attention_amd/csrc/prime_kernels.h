@@ -310,7 +310,8 @@ hipError_t launch_generic_backward(const GenericArgs &a, hipStream_t stream);
 
 // Backward of the delta-rule prefill (delta_bwd.hip): q, k, v, dy strided
 // [B, H(kv), L, D]; gradients fp32 contiguous, dk / dv per query head
-// ([B, H, L, D]); ws = [B*H][chunks][D*2D] fp32 (the state entering each chunk).
+// ([B, H, L, D]); ws holds, for a group of sequences, each chunk's record, the
+// state entering it and the state's adjoint.
 struct DeltaBwdArgs {
     const void *q, *k, *v, *dy;
     int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, dy_sb, dy_sh, dy_sl;
@@ -323,9 +324,11 @@ struct DeltaBwdArgs {
     float *dq, *dk, *dv;        // [B, H, L, D]
     float *dbeta, *dalpha;      // [B, H, L]
     float *dstate_in;           // [B, H, D, 2D] or null
-    float *ws;
+    float *ws;                  // delta_backward_ws_bytes
+    int seq0;                   // first (sequence, head) of the group in the workspace
 };
-hipError_t launch_delta_backward(const DeltaBwdArgs &a, hipStream_t stream);
+size_t delta_backward_ws_bytes(int B, int H, int L);
+hipError_t launch_delta_backward(DeltaBwdArgs a, hipStream_t stream);
 
 // The delta rule at head dims up to 64 and any chunk size (delta_gen.hip):
 // one wavefront per (sequence, head), the recurrence token by token.

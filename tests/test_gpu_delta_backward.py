@@ -71,6 +71,39 @@ def test_delta_backward_matches_fp64_autograd(B, H, Hkv, L, bound, dtype):
         assert _rel(g, r) < TOL, (name, _rel(g, r))
 
 
+@pytest.mark.parametrize("L,bound", [(63, 25.0), (64, 0.0), (65, 1.0), (128, 25.0), (191, 1.0), (321, 1.5)])
+def test_delta_backward_chunk_edges(L, bound):
+    """One to six chunks (the chains take chunks in pairs), lengths around a
+    chunk's end, no clamp, a clamp that holds in every chunk."""
+    args = _case(2, 2, 2, L, 40 + L, torch.float32)
+    to = lambda t: t.to(dev()).contiguous()
+    q, k, v, beta, alpha, s0, dy, ds = args
+    got = _lib.delta_prefill_backward(*(to(t) for t in (q, k, v, beta, alpha)), 0.9995, 1e-5, bound, to(s0), to(dy),
+                                      to(ds))
+    torch.cuda.synchronize()
+    ref = _reference(q, k, v, beta, alpha, s0, dy, ds, bound)
+    for name, g, r in zip(("q", "k", "v", "beta", "alpha", "state"), got, ref):
+        assert _rel(g, r) < 1e-5, (name, _rel(g, r))  # fp32 sums of up to 128 products a contraction
+
+
+def test_delta_backward_sequence_groups():
+    """More sequences than one workspace group holds: the later group's results
+    equal those of a call with its sequences alone."""
+    H, L = 120, 3
+    B = 235  # 28200 (sequence, head) pairs; 8 GiB hold about 27000 of one chunk each
+    per = _lib.delta_backward_workspace_size(1, 1, L)
+    assert _lib.delta_backward_workspace_size(B, H, L) < per * B * H
+    q, k, v, beta, alpha, s0, dy, ds = (t.to(dev()).contiguous() for t in _case(B, H, H, L, 9, torch.float32))
+    got = _lib.delta_prefill_backward(q, k, v, beta, alpha, 0.9995, 1e-5, 2.0, s0, dy, ds)
+    cut = B - 12
+    for sel in (slice(0, 2), slice(cut, B)):
+        part = _lib.delta_prefill_backward(*(t[sel].contiguous() for t in (q, k, v, beta, alpha)), 0.9995, 1e-5, 2.0,
+                                           s0[sel].contiguous(), dy[sel].contiguous(), ds[sel].contiguous())
+        torch.cuda.synchronize()
+        for g, r in zip(got, part):
+            assert torch.equal(g[sel], r)
+
+
 def test_delta_backward_without_state_gradient_inputs():
     """No incoming state and no gradient on the final state: the adjoint starts
     at zero, dstate_in is not produced."""
