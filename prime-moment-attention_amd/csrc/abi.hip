@@ -126,6 +126,8 @@ int generic_args(prime::GenericArgs &a, const prime_tensor_t *q, const prime_ten
     a.B = B; a.H = H; a.group = H / H_kv; a.L = L; a.D = D;
     a.decay = decay; a.eps = eps;
     a.dense_clamp = (flags & PRIME_FLAG_DENSE_CLAMP) ? 1 : 0;
+    a.G = 1;
+    a.cps = (L + 63) / 64;
     if (state_in) {
         a.s0i = state_in->s0; a.s1i = state_in->s1; a.s2i = state_in->s2;
         a.k0i = state_in->k0; a.k1i = state_in->k1; a.k2i = state_in->k2;
@@ -135,6 +137,24 @@ int generic_args(prime::GenericArgs &a, const prime_tensor_t *q, const prime_ten
         a.k0o = state_out->k0; a.k1o = state_out->k1; a.k2o = state_out->k2;
     }
     return PRIME_OK;
+}
+
+// The backward's per-token scratch at the start of the workspace, and the dense
+// clamp's incoming-K correction: behind it where the workspace holds it, else in
+// the incoming state's adjoint itself (which the dk/dv pass writes last).
+void generic_bwd_scratch(prime::GenericArgs &a, void *workspace, size_t workspace_bytes, size_t token_bytes) {
+    a.inv_den = static_cast<float *>(workspace);
+    a.g_den = a.inv_den + static_cast<size_t>(a.B) * a.H * a.L;
+    if (workspace_bytes >= token_bytes + static_cast<size_t>(a.B) * a.H * prime::kBwdCorr * sizeof(float)) {
+        a.kc1 = reinterpret_cast<float *>(static_cast<char *>(workspace) + token_bytes);
+        a.kc2 = a.kc1 + prime::kD;
+        a.kc0 = a.kc2 + prime::kD;
+        a.kc_s = a.kc0_s = prime::kBwdCorr;
+    } else {
+        a.kc1 = a.dki1; a.kc2 = a.dki2; a.kc0 = a.dki0;
+        a.kc_s = a.D;
+        a.kc0_s = 1;
+    }
 }
 
 int generic_norm(prime::GenericArgs &a, const prime_qk_norm_t *norm) {
@@ -562,7 +582,7 @@ static int prefill_impl(const prime_tensor_t *q, const prime_tensor_t *k, const 
         (selective && !k_scale))
         return fail(PRIME_ERR_INVALID_ARG, "prefill: null argument");
     if (D != prime::kD) {
-        // head dims below 64: one wavefront per (sequence, head), chunk size irrelevant
+        // head dims below 64: fp32 chunks of 64 tokens, whatever the chunk size asked for
         if (chunk <= 0) return fail(PRIME_ERR_INVALID_ARG, "bad chunk %d", chunk);
         if (selective && flags) return fail(PRIME_ERR_INVALID_ARG, "the selective form takes no flags");
         if (!valid_dtype(y->dtype)) return fail(PRIME_ERR_UNSUPPORTED_DTYPE, "unsupported y dtype");
@@ -836,7 +856,7 @@ int prime_chunked_prefill_backward(const prime_tensor_t *q, const prime_tensor_t
         !dk->data || !dv->data || !decay || !workspace)
         return fail(PRIME_ERR_INVALID_ARG, "prime_chunked_prefill_backward: null argument");
     if (D != prime::kD) {
-        // head dims below 64: the generic reverse pass (workspace: the per-token
+        // head dims below 64: the fp32 chunk passes (workspace: the per-token
         // denominators, as the 64 path's minimum)
         if (H_kv != H)
             return fail(PRIME_ERR_INVALID_ARG, "backward takes k/v with one head per query head (H_kv=%d, H=%d)",
@@ -866,8 +886,8 @@ int prime_chunked_prefill_backward(const prime_tensor_t *q, const prime_tensor_t
             g.dsi0 = dstate_in->s0; g.dsi1 = dstate_in->s1; g.dsi2 = dstate_in->s2;
             g.dki0 = dstate_in->k0; g.dki1 = dstate_in->k1; g.dki2 = dstate_in->k2;
         }
-        g.ws = static_cast<float *>(workspace);
-        return check_hip(prime::launch_generic_backward(g, static_cast<hipStream_t>(stream)), "backward launch");
+        generic_bwd_scratch(g, workspace, workspace_bytes, bwd_token_bytes(B, H, L));
+        return check_hip(prime::launch_chunk_f32_backward(g, static_cast<hipStream_t>(stream)), "backward launch");
     }
     if (B <= 0 || H <= 0 || L <= 0) return fail(PRIME_ERR_INVALID_ARG, "bad sizes B=%d H=%d L=%d", B, H, L);
     if (H_kv != H)
@@ -953,7 +973,7 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
         !dk->data || !dv->data || !log_decay || !k_scale || !d_log_decay || !d_k_scale || !workspace)
         return fail(PRIME_ERR_INVALID_ARG, "prime_selective_prefill_backward: null argument");
     if (D != prime::kD) {
-        // head dims below 64: the generic reverse pass in its selective form
+        // head dims below 64: the fp32 chunk passes in their selective form
         if (H_kv != H)
             return fail(PRIME_ERR_INVALID_ARG, "backward takes k/v with one head per query head (H_kv=%d, H=%d)",
                         H_kv, H);
@@ -986,11 +1006,12 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
             g.dsi0 = dstate_in->s0; g.dsi1 = dstate_in->s1; g.dsi2 = dstate_in->s2;
             g.dki0 = dstate_in->k0; g.dki1 = dstate_in->k1; g.dki2 = dstate_in->k2;
         }
-        g.ws = static_cast<float *>(workspace);
+        generic_bwd_scratch(g, workspace, bwd_token_bytes(B, H, L), bwd_token_bytes(B, H, L));
         g.pq = reinterpret_cast<float *>(static_cast<char *>(workspace) + bwd_token_bytes(B, H, L));
+        g.fin = g.pq + static_cast<size_t>(B) * H * L;
         g.dlogd = d_log_decay;
         g.dkscale = d_k_scale;
-        return check_hip(prime::launch_generic_backward(g, static_cast<hipStream_t>(stream)), "backward launch");
+        return check_hip(prime::launch_chunk_f32_backward(g, static_cast<hipStream_t>(stream)), "backward launch");
     }
     if (B <= 0 || H <= 0 || L <= 0) return fail(PRIME_ERR_INVALID_ARG, "bad sizes B=%d H=%d L=%d", B, H, L);
     if (H_kv != H)

@@ -261,7 +261,8 @@ struct DeltaArgs {
     int first, last;            // window is the first / last of the call
 };
 
-// Head dims below 64 (generic_d.hip): one wavefront per (sequence, head).
+// Head dims below 64: one token (generic_d.hip, one wavefront per (sequence,
+// head)) and several (chunk_f32.hip).
 struct GenericArgs {
     const void *q, *k, *v;
     int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
@@ -288,7 +289,15 @@ struct GenericArgs {
     int dt_g;
     int64_t g_sb, g_sh, g_sl;
     float *dsi0, *dsi1, *dsi2, *dki0, *dki1, *dki2;  // adjoint of the incoming state or null
-    float *ws;                                        // [B*H][L][2]
+    float *inv_den, *g_den;                           // [B*H][L]: 1/D and the denominator's adjoint
+    // the dense clamp's share of the incoming K adjoint (dq pass to dk/dv pass), per
+    // sequence at strides kc_s and kc0_s: features q, q*q, and the constant
+    float *kc1, *kc2, *kc0;
+    int64_t kc_s, kc0_s;
+    // segments per sequence (D = 64) of cps chunks, their slots, and the dk/dv
+    // pass's per-segment totals (selective: decay suffix sum, key scale's adjoint)
+    int G, cps;
+    float *slots, *seg_tot;
     // selective form: a decay per token, k weighted by k_scale[h] (beta), S2
     // and K2 carrying the 1/2; decays from log_decay [B*H][L] (natural log), or
     // for one token (the decode step) from decay_bh [B*H] or the step-size
@@ -303,10 +312,13 @@ struct GenericArgs {
     float *dlogd;    // backward: [B*H][L], the log decays' adjoint
     float *dkscale;  // backward: [B*H], beta's adjoint per sequence
     float *pq;       // backward scratch: [B*H][L]
+    float *fin;      // backward scratch: [B*H], <dstate_out, state_out>
 };
+using ChunkF32Args = GenericArgs;
 constexpr int kGenericMaxD = 63;
-hipError_t launch_generic_prefill(const GenericArgs &a, hipStream_t stream);
-hipError_t launch_generic_backward(const GenericArgs &a, hipStream_t stream);
+hipError_t launch_generic_prefill(GenericArgs a, hipStream_t stream);
+hipError_t launch_chunk_f32_prefill(const ChunkF32Args &a, hipStream_t stream);
+hipError_t launch_chunk_f32_backward(const ChunkF32Args &a, hipStream_t stream);
 
 // Backward of the delta-rule prefill (delta_bwd.hip): q, k, v, dy strided
 // [B, H(kv), L, D]; gradients fp32 contiguous, dk / dv per query head

@@ -1,0 +1,114 @@
+"""GPU parity of the fp32 chunk kernels (chunk_f32.hip) where they can go wrong:
+head dims at the edges of the padded widths 16, 32 and 64, lengths around a
+chunk's end and the one-token kernel's line, rows at any alignment and in mixed
+dtypes, and decays of 0.  Against the float64 oracle; 2e-5 of each tensor's
+largest value: fp32 sums of a few hundred products at 6e-8 each."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from prime_moment_attention import _lib
+
+from gpu_util import dev, random_state, state_to_dev, state_to_np, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-5
+
+
+def _close(x, r, name):
+    e = np.abs(np.asarray(x, np.float64).reshape(np.shape(r)) - r).max() / max(np.abs(r).max(), 1e-300)
+    assert e < TOL, f"{name}: {e:.2e}"
+
+
+def _case(B, H, L, D, seed):
+    rng = np.random.default_rng(seed)
+    q, k, v = O.make_inputs((B, H, L, D), seed=seed, bf16=False)
+    lam = rng.uniform(0.98, 0.9999, H).astype(np.float32)
+    return q, k, v, lam, rng
+
+
+@pytest.mark.parametrize("D,L", [(1, 2), (15, 63), (16, 64), (17, 65), (31, 129), (32, 128), (33, 127), (63, 66)])
+def test_chunk_f32_prefill_and_backward_edges(D, L):
+    B, H = 2, 2
+    BH = B * H
+    q, k, v, lam, rng = _case(B, H, L, D, 100 + D)
+    st0 = random_state(BH, D, 7)
+    dy = rng.standard_normal((B, H, L, D)).astype(np.float32)
+    ds = tuple(0.1 * rng.standard_normal(x.shape) for x in O.zero_state(BH, D))
+    flat = [x.reshape(BH, L, D) for x in (q, k, v)]
+    lam_bh = np.tile(lam.astype(np.float64), B)
+    yo, so = O.chunked(*flat, lam_bh, eps=1.0, chunk=64, state=st0)
+    ref = O.recurrent_vjp(*flat, lam_bh, dy.reshape(BH, L, D), eps=1.0, state=st0, dstate=ds)
+    print(f"[chunk f32] D={D} L={L}", flush=True)
+    tq, tk, tv, tl, tdy = (to_dev(x) for x in (q, k, v, lam, dy))
+    st_in = state_to_dev(st0, B, H, D)
+    y, st = torch.empty_like(tq), _lib.new_state(B, H, D, dev())
+    _lib.chunked_prefill(tq, tk, tv, tl, 1.0, 64, st_in, y, st)
+    g = [torch.empty_like(tq) for _ in range(3)]
+    dsi = _lib.new_state(B, H, D, dev())
+    _lib.chunked_prefill_backward(tq, tk, tv, tl, 1.0, st_in, tdy, state_to_dev(ds, B, H, D), *g, dsi)
+    torch.cuda.synchronize()
+    _close(to_np(y), yo.reshape(y.shape), "y")
+    for n, x, r in zip("S0 S1 S2 K0 K1 K2".split(), state_to_np(st, BH, D), so):
+        _close(x, r, n)
+    for n, x, r in zip(("dq", "dk", "dv"), g, ref[:3]):
+        _close(to_np(x), r, n)
+    for n, x, r in zip("S0 S1 S2 K0 K1 K2".split(), state_to_np(dsi, BH, D), ref[3]):
+        _close(x, r, "d" + n)
+
+
+def test_chunk_f32_any_alignment_and_mixed_dtypes():
+    """Rows that start on odd elements, q fp32, k bf16, v fp16, grouped heads:
+    the same values as contiguous fp32 rows."""
+    B, H, Hkv, L, D = 2, 4, 2, 70, 24
+    g = torch.Generator().manual_seed(3)
+    big = [torch.randn(B, h, L, D + 5, generator=g) * 0.3 for h in (H, Hkv, Hkv)]
+    views = [t.to(dev(), dt)[..., 3:3 + D] for t, dt in zip(big, (torch.float32, torch.bfloat16, torch.float16))]
+    lam = torch.full((H,), 0.99, device=dev())
+    out = []
+    for q, k, v in (views, [t.float().contiguous() for t in views]):
+        y, st = torch.empty(B, H, L, D, device=dev()), _lib.new_state(B, H, D, dev())
+        _lib.chunked_prefill(q, k, v, lam, 1.0, 64, None, y, st)
+        out.append((y, *st))
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+def test_chunk_f32_zero_decay():
+    """A decay of 0 (and a log decay of -inf) keeps each token alone: y is v
+    over the clamped score of its own key."""
+    B, H, L, D = 1, 2, 70, 32
+    q, k, v, _, _ = _case(B, H, L, D, 5)
+    score = 1 + (q * k).sum(-1) + 0.5 * (q * q * k * k).sum(-1)
+    want = v * (score / np.maximum(score, 1.0))[..., None]
+    t = [to_dev(x) for x in (q, k, v)]
+    y, y2 = torch.empty_like(t[0]), torch.empty_like(t[0])
+    _lib.chunked_prefill(*t, torch.zeros(H, device=dev()), 1.0, 64, None, y, _lib.new_state(B, H, D, dev()))
+    ninf = torch.full((B, H, L), -float("inf"), device=dev())
+    _lib.selective_prefill(*t, ninf, torch.ones(H, device=dev()), 1.0, None, y2, _lib.new_state(B, H, D, dev()))
+    torch.cuda.synchronize()
+    _close(to_np(y), want, "y")
+    _close(to_np(y2), want, "selective y")
+
+
+@pytest.mark.parametrize("D", [32, 63])
+def test_chunk_f32_dense_clamp_backward_scratch(D):
+    """The dense clamp's correction in the workspace or, where a caller gives the
+    per-token scratch alone, in the incoming state's adjoint: the same result."""
+    B, H, L = 1, 2, 90
+    q, k, v, lam, rng = _case(B, H, L, D, 11)
+    st = state_to_dev(random_state(B * H, D, 12), B, H, D)
+    t = [to_dev(x) for x in (q, k, v)]
+    dy = to_dev(rng.standard_normal(q.shape).astype(np.float32))
+    out = []
+    small = (B * H * L * 8 + 255) // 256 * 256
+    for size in (_lib.backward_workspace_size(B, H, L), small):
+        g, dsi = [torch.empty_like(t[0]) for _ in range(3)], _lib.new_state(B, H, D, dev())
+        _lib.chunked_prefill_backward(*t, to_dev(lam), 2.5, st, dy, None, *g, dsi, flags=1,
+                                      workspace=torch.empty(size, dtype=torch.uint8, device=dev()))
+        out.append((*g, *dsi))
+    torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
