@@ -21,9 +21,9 @@
  *
  * Head dim: D = 64 runs the MFMA chunk kernels; the base and selective forms
  * (prefill, decode step, backward, QK-norm) also take 1 <= D <= 63 (the
- * reference's own tests use 32 and 16), run token by token in one wavefront
- * per (sequence, head) with no row-alignment requirement and no workspace
- * beyond the backward's per-token records.  The delta rule takes D <= 64
+ * reference's own tests use 32 and 16), run in fp32 chunks (one token: one
+ * wavefront per (sequence, head)) with no row-alignment requirement and no
+ * workspace beyond the backward's per-token records.  The delta rule takes D <= 64
  * with any chunk (documented at prime_delta_prefill).  prime_accumulate and
  * the split decode readout/update take D = 64 only.
  */
@@ -561,7 +561,7 @@ int prime_accumulate_noalloc(const prime_tensor_t *k, const prime_tensor_t *v, i
  * the call's own tokens, the outer one the incoming state's term (without a
  * state the two clamps are the same).  BF16 inputs run on bf16 MFMA operands (fp32
  * accumulation); F32 inputs run fp32 passes (fp32 MFMA operands throughout,
- * one workgroup per sequence, as the reference differentiates in fp32).
+ * as the reference differentiates in fp32).
  * workspace (16-byte aligned): at least B*H*L*8 bytes (per-token
  * denominators; rounded up to 256), plus B*H*528 bytes for
  * PRIME_FLAG_DENSE_CLAMP with a state; with prime_chunked_prefill_backward_workspace_size()
@@ -582,7 +582,7 @@ size_t prime_chunked_prefill_backward_workspace_size(int B, int H, int L);
  * prime_selective_prefill_backward: the adjoint of prime_selective_prefill
  * (torch autograd through selective.py:414-440, and through the step branch
  * :384-409 for a call with an incoming state), F32 q/k/v (convert bf16 inputs
- * first; the passes are the fp32 backward's, one workgroup per sequence).
+ * first; the passes are the fp32 backward's).
  * Inputs as for prime_selective_prefill: log_decay fp32 [B,H,L] (log lambda_t,
  * contiguous), k_scale fp32 [H] (beta; the key enters as beta k), state_in in
  * the selective convention (S2, K2 carry the 1/2), or NULL; dy; dstate_out
@@ -594,7 +594,10 @@ size_t prime_chunked_prefill_backward_workspace_size(int B, int H, int L);
  * features [1, q, q*q] and [1, beta k, beta^2 k*k/2], plus
  * <dstate_out, state_out>), d_k_scale fp32 [B,H] (the adjoint of k_scale per
  * sequence: sum over the batch for the [H] parameter).  H_kv == H.
- * workspace (16-byte aligned): prime_selective_prefill_backward_workspace_size.
+ * workspace (16-byte aligned): at least B*H*L*12 bytes (the first 8 of each
+ * rounded up to 256 in all) and B*H*4; with
+ * prime_selective_prefill_backward_workspace_size() bytes few long sequences
+ * run in segments, as above.
  */
 int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor_t *k, const prime_tensor_t *v,
                                      int B, int H, int H_kv, int L, int D, const float *log_decay,

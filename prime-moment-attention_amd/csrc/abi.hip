@@ -954,11 +954,28 @@ int prime_chunked_prefill_backward(const prime_tensor_t *q, const prime_tensor_t
     return check_hip(prime::launch_prefill_backward(a, static_cast<hipStream_t>(stream)), "backward launch");
 }
 
-size_t prime_selective_prefill_backward_workspace_size(int B, int H, int L) {
-    if (B <= 0 || H <= 0 || L <= 0) return 0;
-    // the per-token denominators (8 bytes), the query-side decay terms (4), one float per sequence
+namespace {
+// the per-token denominators (8 bytes), the query-side decay terms (4), one float per sequence
+size_t sel_bwd_min_bytes(int B, int H, int L) {
     return bwd_token_bytes(B, H, L) + static_cast<size_t>(B) * H * L * sizeof(float) +
            static_cast<size_t>(B) * H * sizeof(float);
+}
+// with segments: then, on a slot boundary, their slots and two floats a segment
+size_t sel_bwd_slots_at(int B, int H, int L) {
+    return (sel_bwd_min_bytes(B, H, L) + 255) & ~static_cast<size_t>(255);
+}
+size_t sel_bwd_segment_bytes(int B, int H, int L, int G) {
+    return G > 1 ? sel_bwd_slots_at(B, H, L) +
+                       static_cast<size_t>(B) * H * G * (prime::kWsStride + 2) * sizeof(float)
+                 : sel_bwd_min_bytes(B, H, L);
+}
+}  // namespace
+
+size_t prime_selective_prefill_backward_workspace_size(int B, int H, int L) {
+    if (B <= 0 || H <= 0 || L <= 0) return 0;
+    int G, cps;
+    prime::plan_backward_segments(B * H, L, &G, &cps, 1);
+    return sel_bwd_segment_bytes(B, H, L, G);
 }
 
 int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor_t *k, const prime_tensor_t *v,
@@ -984,9 +1001,9 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
             dk->stride_l != dq->stride_l || dv->stride_l != dq->stride_l)
             return fail(PRIME_ERR_INVALID_ARG, "dq, dk and dv must share dtype and strides");
         if (B > 0 && H > 0 && L > 0 &&
-            (workspace_bytes < prime_selective_prefill_backward_workspace_size(B, H, L) || !aligned16(workspace)))
+            (workspace_bytes < sel_bwd_min_bytes(B, H, L) || !aligned16(workspace)))
             return fail(PRIME_ERR_INVALID_ARG, "workspace of %zu bytes (16-byte aligned) is below the %zu needed",
-                        workspace_bytes, prime_selective_prefill_backward_workspace_size(B, H, L));
+                        workspace_bytes, sel_bwd_min_bytes(B, H, L));
         prime::GenericArgs g{};
         int rc;
         if ((rc = generic_args(g, q, k, v, B, H, H_kv, L, D, nullptr, eps, 0u, state_in, nullptr)) ||
@@ -1028,7 +1045,7 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
         return fail(PRIME_ERR_INVALID_ARG, "dq, dk and dv must share dtype and strides");
     if (!rows_aligned(q, true) || !rows_aligned(k, true) || !rows_aligned(v, true) || !rows_aligned(dy, true))
         return fail(PRIME_ERR_MISALIGNED, "q/k/v/dy rows must start on 16-byte boundaries");
-    const size_t need = prime_selective_prefill_backward_workspace_size(B, H, L);
+    const size_t need = sel_bwd_min_bytes(B, H, L);
     if (workspace_bytes < need || !aligned16(workspace))
         return fail(PRIME_ERR_INVALID_ARG, "workspace of %zu bytes (16-byte aligned) is below the %zu needed",
                     workspace_bytes, need);
@@ -1063,8 +1080,15 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
     a.g_den = a.inv_den + ntok;
     a.pq = reinterpret_cast<float *>(static_cast<char *>(workspace) + bwd_token_bytes(B, H, L));
     a.fin = a.pq + ntok;
-    a.G = 1;
-    a.cps = (L + 63) / 64;
+    prime::plan_backward_segments(B * H, L, &a.G, &a.cps, 1);
+    if (a.G > 1 && workspace_bytes < sel_bwd_segment_bytes(B, H, L, a.G)) {
+        a.G = 1;  // one segment per sequence in the workspace given
+        a.cps = (L + 63) / 64;
+    }
+    if (a.G > 1) {
+        a.ws = reinterpret_cast<float *>(static_cast<char *>(workspace) + sel_bwd_slots_at(B, H, L));
+        a.seg_tot = a.ws + static_cast<size_t>(B) * H * a.G * prime::kWsStride;
+    }
     a.logd = log_decay; a.kscale = k_scale; a.dlogd = d_log_decay; a.dkscale = d_k_scale;
     return check_hip(prime::launch_prefill_backward_f32(a, static_cast<hipStream_t>(stream)), "backward launch");
 }

@@ -37,10 +37,12 @@
 // - the next chunk's rows are loaded into registers a chunk ahead;
 // - the denominators and the moments of a value that is always 1 (Kf, K0) and S0 are
 //   VALU sums spread over all 1024 threads, beside the MFMA units;
-// - LDS pitches are 20 modulo 64 dwords where an array is read both as 16 rows x 4
-//   columns and as 4 rows x 16 columns by a wave (no bank twice in 32 lanes either
-//   way), 4 modulo 64 where only the former occurs.
-// Measured at D = 32, 8 sequences of 256 tokens: prefill 25 us, backward 71 us, against
+// - the products with the carried state run beside the score tiles of their phase, the
+//   products with a and da in the next;
+// - LDS pitches by the way each array is read (Dim).
+// Measured at D = 64, 96 sequences of 1000 tokens: dq pass 119 us, dk/dv 117, dual 47
+// (8 waves, nothing loaded ahead, 2 segments: 187, 206, 72); a chunk is 16-18 us of which
+// its MFMAs are 8.4.  At D = 32, 8 sequences of 256 tokens: prefill 25 us, backward 71 us, against
 // 934 and 3580 us for one wavefront per sequence running the recurrence token by token
 // (one token costs the same either way, so a single token keeps that kernel).
 
@@ -63,10 +65,13 @@ struct Dim {
     static constexpr int FP = 2 * DP;              // features
     static constexpr int ND = DP / 16;             // 16-wide blocks of a head row
     static constexpr int NE = kC * DP / kT;        // elements of a row array per thread
-    static constexpr int PB = DP == 64 ? 84 : DP == 32 ? 36 : 20;  // read both ways
-    static constexpr int PP = DP == 64 ? 68 : DP == 32 ? 36 : 20;  // 16 rows x 4 columns only
+    // LDS pitches by how a wave reads the array (64 banks): 16 rows x 4 columns, 4
+    // rows x 16 columns, or both ways (then 4 x 16 meets 12 banks twice)
+    static constexpr int PR = DP == 64 ? 68 : DP == 32 ? 36 : 20;
+    static constexpr int PC = DP == 64 ? 80 : DP == 32 ? 48 : 16;
+    static constexpr int PB = DP == 64 ? 84 : DP == 32 ? 36 : 20;
 };
-constexpr int kPA = kC + 4, kPAt = kC + 20;  // a / da rows, read by rows (dq) or by columns (dk/dv)
+constexpr int kPA = kC + 4, kPAt = kC + 16;  // a / da rows, read by rows (dq) or by columns (dk/dv)
 
 // sum over the 16 lanes of a row of lanes, in each of them
 __device__ __forceinline__ float sum16(float x) {
@@ -76,25 +81,73 @@ __device__ __forceinline__ float sum16(float x) {
     return x + xor_lane<8>(x);
 }
 
+// n batches of B k-steps: the next batch's LDS reads go out before this batch's
+// MFMAs (left alone the compiler reads a whole unrolled loop's operands first and
+// waits for them with the matrix cores idle).
+template <int B, class T, class L, class M>
+__device__ __forceinline__ void pipe(int n, L load, M mul) {
+    T cur[B];
+#pragma unroll
+    for (int e = 0; e < B; ++e) cur[e] = load(e);
+    for (int b = 1; b < n; ++b) {
+        T nxt[B];
+#pragma unroll
+        for (int e = 0; e < B; ++e) nxt[e] = load(b * B + e);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < B; ++e) mul(cur[e]);
+#pragma unroll
+        for (int e = 0; e < B; ++e) cur[e] = nxt[e];
+    }
+#pragma unroll
+    for (int e = 0; e < B; ++e) mul(cur[e]);
+}
+struct Op2 {
+    float a, b;
+};
+struct Op3 {
+    float a, b, c;
+};
+struct OpV {
+    f32x4 a, b;
+};
+
 // lower 16x16 tile t (0..9) -> (row block, column block)
 __device__ __forceinline__ void lower_tile(int t, int &ib, int &jb) {
     ib = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
     jb = t - ib * (ib + 1) / 2;
 }
 
-// NE consecutive elements of a row from column d0, zero past D or when !valid
+// NE consecutive elements of a row from column d0 as stored, from clamped addresses:
+// nothing is masked or converted here, so that no wait sits between a load and the
+// work it is to hide behind (a select on the loaded value cost half the dq pass).
 template <int DP, bool VEC>
-__device__ __forceinline__ void load_elems(const void *p, int dt, int64_t row, int d0, int D, bool valid,
-                                           float (&o)[Dim<DP>::NE]) {
+__device__ __forceinline__ void load_raw(const void *p, int dt, int64_t row, int d0, int D,
+                                         uint32_t (&o)[Dim<DP>::NE]) {
     constexpr int NE = Dim<DP>::NE;
     if constexpr (VEC) {
         static_assert(NE == 4, "vector rows are 64 wide");
-        const f32x4 x = valid ? ld4(static_cast<const float *>(p) + row + d0) : f32x4{0.f, 0.f, 0.f, 0.f};
+        const u32x4 x = *reinterpret_cast<const u32x4 *>(static_cast<const float *>(p) + row + d0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[e] = x[e];
+    } else if (dt == PRIME_F32) {
+#pragma unroll
+        for (int e = 0; e < NE; ++e) o[e] = static_cast<const uint32_t *>(p)[row + min(d0 + e, D - 1)];
     } else {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) o[e] = valid && d0 + e < D ? load_elem(p, row + d0 + e, dt) : 0.f;
+        for (int e = 0; e < NE; ++e) o[e] = static_cast<const uint16_t *>(p)[row + min(d0 + e, D - 1)];
+    }
+}
+// ... and as fp32, zero past D or when !valid
+template <int DP, bool VEC>
+__device__ __forceinline__ void to_f32(const uint32_t (&r)[Dim<DP>::NE], int dt, int d0, int D, bool valid,
+                                       float (&o)[Dim<DP>::NE]) {
+#pragma unroll
+    for (int e = 0; e < Dim<DP>::NE; ++e) {
+        float x = __uint_as_float(r[e]);
+        if (dt == PRIME_BF16) x = __uint_as_float(r[e] << 16);
+        else if (dt == PRIME_F16) x = h16_bits_to_f32(static_cast<uint16_t>(r[e]));
+        o[e] = valid && (VEC || d0 + e < D) ? x : 0.f;
     }
 }
 
@@ -120,32 +173,49 @@ __device__ __forceinline__ void store_out(void *p, int dt, int64_t idx, f32x4 v,
 // A thread's share of a chunk's rows, loaded a chunk ahead
 template <int DP>
 struct Rows {
-    float q[Dim<DP>::NE], k[Dim<DP>::NE], v[Dim<DP>::NE], dy[Dim<DP>::NE];
+    uint32_t q[Dim<DP>::NE], k[Dim<DP>::NE], v[Dim<DP>::NE], dy[Dim<DP>::NE];
     float ld;  // wave 0, selective: the token's log decay
 };
 
+// (the chunk's first row is a scalar address and the row within it is formed from the
+// chunk's length here: no per-thread 64-bit base is carried from chunk to chunk, whose
+// spilled copies would be reloaded between the loads and wait for them)
 template <int DP, bool VEC, bool SEL, bool DY, bool STATE_ONLY = false>
 __device__ __forceinline__ void load_rows(const ChunkF32Args &a, int b, int h, int seq, int c, int tid, Rows<DP> &R) {
-    const int i = tid >> 4, d0 = Dim<DP>::NE * (tid & 15);
-    const int t = c * kC + i;
-    const bool valid = t < a.L;
-    const int64_t tc = valid ? t : 0;
+    const int d0 = Dim<DP>::NE * (tid & 15);
+    const int last = min(kC, a.L - c * kC) - 1;
+    const int64_t i = min(tid >> 4, last), t0 = static_cast<int64_t>(c) * kC;
     const int hk = h / a.group;
-    if constexpr (!STATE_ONLY) load_elems<DP, VEC>(a.q, a.dt_q, b * a.q_sb + h * a.q_sh + tc * a.q_sl, d0, a.D, valid, R.q);
-    load_elems<DP, VEC>(a.k, a.dt_k, b * a.k_sb + hk * a.k_sh + tc * a.k_sl, d0, a.D, valid, R.k);
-    load_elems<DP, VEC>(a.v, a.dt_v, b * a.v_sb + hk * a.v_sh + tc * a.v_sl, d0, a.D, valid, R.v);
+    auto row0 = [](const void *p, int dt, int64_t off) {
+        return static_cast<const void *>(static_cast<const char *>(p) + off * (dt == PRIME_F32 ? 4 : 2));
+    };
+    if constexpr (!STATE_ONLY)
+        load_raw<DP, VEC>(row0(a.q, a.dt_q, b * a.q_sb + h * a.q_sh + t0 * a.q_sl), a.dt_q, i * a.q_sl, d0, a.D, R.q);
+    load_raw<DP, VEC>(row0(a.k, a.dt_k, b * a.k_sb + hk * a.k_sh + t0 * a.k_sl), a.dt_k, i * a.k_sl, d0, a.D, R.k);
+    load_raw<DP, VEC>(row0(a.v, a.dt_v, b * a.v_sb + hk * a.v_sh + t0 * a.v_sl), a.dt_v, i * a.v_sl, d0, a.D, R.v);
     if constexpr (DY) {
-        const int64_t row = b * a.dy_sb + h * a.dy_sh + tc * a.dy_sl;
-        if (VEC && a.dt_dy == PRIME_F32) load_elems<DP, VEC>(a.dy, PRIME_F32, row, d0, a.D, valid, R.dy);
-        else load_elems<DP, false>(a.dy, a.dt_dy, row, d0, a.D, valid, R.dy);
+        const void *p = row0(a.dy, a.dt_dy, b * a.dy_sb + h * a.dy_sh + t0 * a.dy_sl);
+        if (VEC && a.dt_dy == PRIME_F32) load_raw<DP, VEC>(p, PRIME_F32, i * a.dy_sl, d0, a.D, R.dy);
+        else load_raw<DP, false>(p, a.dt_dy, i * a.dy_sl, d0, a.D, R.dy);
     }
-    if constexpr (SEL) {
-        R.ld = 0.f;
-        if (tid < kWave && c * kC + tid < a.L) {
-            const float x = a.log_decay[static_cast<size_t>(seq) * a.L + c * kC + tid];
-            R.ld = x < -200.f ? -200.f : x;  // (e^-200 is 0 in fp32; -inf would make the differences NaN)
-        }
+    if constexpr (SEL)
+        if (tid < kWave) R.ld = (a.log_decay + static_cast<size_t>(seq) * a.L + t0)[min(tid, last)];
+}
+// the loaded rows in LDS as fp32 (k times kscale), zero past L and D
+template <int DP, bool VEC, bool STATE_ONLY, int PQ, int PK, int PV>
+__device__ __forceinline__ void put_rows(const ChunkF32Args &a, const Rows<DP> &R, int i, int d0, int nv, float kscale,
+                                         float (*sQ)[PQ], float (*sK)[PK], float (*sV)[PV]) {
+    float x[Dim<DP>::NE];
+    if constexpr (!STATE_ONLY) {
+        to_f32<DP, VEC>(R.q, VEC ? PRIME_F32 : a.dt_q, d0, a.D, i < nv, x);
+        put_elems<DP>(sQ, i, d0, x);
     }
+    to_f32<DP, VEC>(R.k, VEC ? PRIME_F32 : a.dt_k, d0, a.D, i < nv, x);
+#pragma unroll
+    for (int e = 0; e < Dim<DP>::NE; ++e) x[e] *= kscale;
+    put_elems<DP>(sK, i, d0, x);
+    to_f32<DP, VEC>(R.v, VEC ? PRIME_F32 : a.dt_v, d0, a.D, i < nv, x);
+    put_elems<DP>(sV, i, d0, x);
 }
 
 // The chunk's decays: sEc[i] = e_i, sW[j] = w_j (0 past L), and e_63, sum w in
@@ -155,7 +225,9 @@ __device__ __forceinline__ void put_decays(int nv, int lane, float ld, const flo
                                            float *sW, float *sSc) {
     float e, w, e63;
     if constexpr (SEL) {
-        const float cum = wave_prefix_sum(ld);
+        // (e^-200 is 0 in fp32; -inf would make the differences NaN)
+        const float x = lane < nv ? (ld < -200.f ? -200.f : ld) : 0.f;
+        const float cum = wave_prefix_sum(x);
         const float cend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum), 63));
         sCum[lane] = cum;
         e = expf(cum);
@@ -188,15 +260,14 @@ __device__ __forceinline__ f32x4 score_tile(int ib, int jb, int g, int c16, cons
     const float *pa = &sQ[16 * ib + c16][DP / 4 * g];
     const float *pb = &sK[16 * jb + c16][DP / 4 * g];
     f32x4 p = {0.f, 0.f, 0.f, 0.f}, p2 = {0.f, 0.f, 0.f, 0.f};
+    pipe<1, OpV>(DP / 16, [&](int q4) { return OpV{ld4(pa + 4 * q4), ld4(pb + 4 * q4)}; },
+                 [&](const OpV &o) {
 #pragma unroll
-    for (int q4 = 0; q4 < DP / 16; ++q4) {
-        const f32x4 x = ld4(pa + 4 * q4), z = ld4(pb + 4 * q4);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            p = mfma4(x[r], z[r], p);
-            p2 = mfma4(x[r] * x[r], 0.5f * (z[r] * z[r]), p2);
-        }
-    }
+                     for (int r = 0; r < 4; ++r) {
+                         p = mfma4(o.a[r], o.b[r], p);
+                         p2 = mfma4(o.a[r] * o.a[r], 0.5f * (o.b[r] * o.b[r]), p2);
+                     }
+                 });
     return p + p2;
 }
 
@@ -223,8 +294,12 @@ __device__ __forceinline__ f32x4 dscore_tile(int w, int nv, int g, int c16, cons
     int ib, jb;
     lower_tile(w, ib, jb);
     f32x4 p = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int s = 0; s < DP / 4; ++s) p = mfma4(sG[16 * ib + c16][4 * s + g], sV[16 * jb + c16][4 * s + g], p);
+#pragma unroll
+    for (int q4 = 0; q4 < DP / 16; ++q4) {
+        const f32x4 x = ld4(&sG[16 * ib + c16][DP / 4 * g + 4 * q4]), z = ld4(&sV[16 * jb + c16][DP / 4 * g + 4 * q4]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p = mfma4(x[r], z[r], p);
+    }
     const int j = 16 * jb + c16;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -345,13 +420,13 @@ __device__ __forceinline__ void advance(Carry<DP> &C, float second, float e63, f
     if (has_unit<DP>(u)) {
         f32x4 x = C.m[0] * e63, y = C.m[1] * e63;
         const int fc = 16 * (u / ND) + c16, xc = 16 * (u % ND) + c16;
-#pragma unroll 8
-        for (int s = 0; s < 16; ++s) {
-            const int j = 4 * s + g;
-            const float f = sR[j][fc], vv = sWt[j] * sX[j][xc];
-            x = mfma4(f, vv, x);
-            y = mfma4(second * (f * f), vv, y);
-        }
+        pipe<4, Op3>(
+            4, [&](int s) { return Op3{sR[4 * s + g][fc], sWt[4 * s + g], sX[4 * s + g][xc]}; },
+            [&](const Op3 &o) {
+                const float vv = o.b * o.c;
+                x = mfma4(o.a, vv, x);
+                y = mfma4(second * (o.a * o.a), vv, y);
+            });
         C.m[0] = x;
         C.m[1] = y;
     }
@@ -395,23 +470,31 @@ __device__ __forceinline__ float k_readout(int i, int part, const float (*sQ)[PQ
     return rd;
 }
 
-// num^T tile of (token block tb, value block dv): the chunk's values and the state's
-template <int DP, int PQ, int PV, int PA, int PM>
-__device__ __forceinline__ f32x4 num_tile(int tb, int dv, int g, int c16, float ec, const float (*sQ)[PQ],
-                                          const float (*sV)[PV], const float (*sA)[PA], const float (*sM)[PM],
-                                          const float *sS0) {
+// num^T tile of (token block tb, value block dv): the state's part (needs no scores) ...
+template <int DP, int PQ, int PM>
+__device__ __forceinline__ f32x4 num_state(int tb, int dv, int g, int c16, float ec, const float (*sQ)[PQ],
+                                           const float (*sM)[PM], const float *sS0) {
     const int tok = 16 * tb + c16;
     f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < 4 * (tb + 1); ++s)  // a is zero above token 16 tb + 15
-        x = mfma4(sV[4 * s + g][16 * dv + c16], sA[tok][4 * s + g], x);
-#pragma unroll 8
-    for (int s = 0; s < DP / 4; ++s) {
-        const float q = sQ[tok][4 * s + g], eq = ec * q;
-        x = mfma4(sM[4 * s + g][16 * dv + c16], eq, x);
-        y = mfma4(sM[DP + 4 * s + g][16 * dv + c16], eq * q, y);
-    }
+    pipe<4, Op3>(
+        DP / 16,
+        [&](int s) { return Op3{sQ[tok][4 * s + g], sM[4 * s + g][16 * dv + c16], sM[DP + 4 * s + g][16 * dv + c16]}; },
+        [&](const Op3 &o) {
+            const float eq = ec * o.a;
+            x = mfma4(o.b, eq, x);
+            y = mfma4(o.c, eq * o.a, y);
+        });
 #pragma unroll
     for (int r = 0; r < 4; ++r) x[r] += y[r] + ec * sS0[16 * dv + 4 * g + r];
+    return x;
+}
+// ... and the chunk's values (a is zero above token 16 tb + 15)
+template <int PV, int PA>
+__device__ __forceinline__ f32x4 num_values(int tb, int dv, int g, int c16, const float (*sV)[PV],
+                                            const float (*sA)[PA], f32x4 x) {
+    const int tok = 16 * tb + c16;
+    pipe<4, Op2>(tb + 1, [&](int s) { return Op2{sV[4 * s + g][16 * dv + c16], sA[tok][4 * s + g]}; },
+                 [&](const Op2 &o) { x = mfma4(o.a, o.b, x); });
     return x;
 }
 
@@ -420,15 +503,15 @@ __device__ __forceinline__ f32x4 num_tile(int tb, int dv, int g, int c16, float 
 // ---------------------------------------------------------------------------
 // Prefill.  DIN: the dense branch's double clamp with an incoming state (the
 // call's own K moments are carried from zero, the incoming ones kept apart);
-// VEC: D = 64 fp32 rows on 16-byte boundaries; STATE_ONLY (selective, D = 64):
-// a segment's state from zero and its log decay, into its slot.
+// VEC: D = 64 fp32 rows on 16-byte boundaries; STATE_ONLY (D = 64): a segment's
+// state from zero (selective: and its log decay) into its slot.
 // ---------------------------------------------------------------------------
 template <int DP, bool DIN, bool SEL, bool VEC, bool STATE_ONLY>
 __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32Args a) {
     using K = Dim<DP>;
-    __shared__ __attribute__((aligned(16))) float sQ[STATE_ONLY ? 1 : kC][K::PP];
-    __shared__ __attribute__((aligned(16))) float sK[kC][K::PB];
-    __shared__ __attribute__((aligned(16))) float sV[kC][K::PB];
+    __shared__ __attribute__((aligned(16))) float sQ[STATE_ONLY ? 1 : kC][K::PR];
+    __shared__ __attribute__((aligned(16))) float sK[kC][K::PC];
+    __shared__ __attribute__((aligned(16))) float sV[kC][K::PC];
     __shared__ __attribute__((aligned(16))) float sA[STATE_ONLY ? 1 : kC][kPA];
     __shared__ __attribute__((aligned(16))) float sM[STATE_ONLY ? 1 : K::FP][K::PB];
     __shared__ float sKf[K::FP], sKin[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sDen[kC], sSc[2];
@@ -469,20 +552,11 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     if constexpr (!SEL) __syncthreads();  // sPw
     for (int c = c_begin; c < c_end; ++c) {
         const int nv = min(kC, a.L - c * kC);
-        if (SEL && !a.qk_norm) {
-            const float beta = a.k_scale[h];
-#pragma unroll
-            for (int e = 0; e < K::NE; ++e) R.k[e] *= beta;
-        }
-        if constexpr (!STATE_ONLY) {
-            put_elems<DP>(sQ, i, d0, R.q);
-            publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
-        }
-        put_elems<DP>(sK, i, d0, R.k);
-        put_elems<DP>(sV, i, d0, R.v);
+        if constexpr (!STATE_ONLY) publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
+        put_rows<DP, VEC, STATE_ONLY>(a, R, i, d0, nv, SEL && !a.qk_norm ? a.k_scale[h] : 1.0f, sQ, sK, sV);
         if (w == 0) {
             put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
-            if (STATE_ONLY) seg_ld += wave_sum(R.ld);
+            if (SEL && STATE_ONLY) seg_ld += wave_sum(lane < nv ? R.ld : 0.f);
         }
         __syncthreads();
         if constexpr (!VEC && !STATE_ONLY) {
@@ -501,6 +575,9 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
         if (c + 1 < c_end) load_rows<DP, VEC, SEL, false, STATE_ONLY>(a, b, h, seq, c + 1, tid, R);
         const float e63 = sSc[0], sumw = sSc[1];
         if constexpr (!STATE_ONLY) {
+            const int tb = w / K::ND, dv = w % K::ND, tok = 16 * tb + c16;
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            if (w < 4 * K::ND) acc = num_state<DP>(tb, dv, g, c16, sEc[tok], sQ, sM, sS0);
             if (w < 10) put_scores<DP, SEL>(w, nv, g, c16, sQ, sK, sPw, sCum, sA);
             __syncthreads();
             // ---- denominators, 16 threads a token (only a's lower tiles exist)
@@ -522,9 +599,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
                 }
                 if (part == 0) sDen[i] = den;
             }
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            const int tb = w / K::ND, dv = w % K::ND, tok = 16 * tb + c16;
-            if (w < 4 * K::ND) acc = num_tile<DP>(tb, dv, g, c16, sEc[tok], sQ, sV, sA, sM, sS0);
+            if (w < 4 * K::ND) acc = num_values(tb, dv, g, c16, sV, sA, acc);
             advance<DP>(C, 0.5f, e63, sumw, u, g, c16, tid, sK, sV, sW, sW);
             __syncthreads();
             if (w < 4 * K::ND && tok < nv) {
@@ -541,8 +616,8 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
         }
     }
     if constexpr (STATE_ONLY) {
-        store_carry<DP>(slot_state(slot), a.D, 1.0f, u, g, c16, tid, C);
-        if (tid == 0) slot[kWsDecay] = seg_ld * 1.44269504088896341f;  // log2
+        store_carry<DP>(slot_state(slot), a.D, c2out, u, g, c16, tid, C);
+        if (SEL && tid == 0) slot[kWsDecay] = seg_ld * 1.44269504088896341f;  // log2
         return;
     }
     if (a.s1o && seg == a.G - 1) {
@@ -566,10 +641,10 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
 template <int DP, bool DIN, bool SEL, bool VEC>
 __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args a) {
     using K = Dim<DP>;
-    __shared__ __attribute__((aligned(16))) float sQ[kC][K::PP];
-    __shared__ __attribute__((aligned(16))) float sK[kC][K::PB];
-    __shared__ __attribute__((aligned(16))) float sV[kC][K::PB];
-    __shared__ __attribute__((aligned(16))) float sG[kC][K::PP];  // dy, then g
+    __shared__ __attribute__((aligned(16))) float sQ[kC][K::PR];
+    __shared__ __attribute__((aligned(16))) float sK[kC][K::PC];
+    __shared__ __attribute__((aligned(16))) float sV[kC][K::PC];
+    __shared__ __attribute__((aligned(16))) float sG[kC][K::PR];  // dy, then g
     __shared__ __attribute__((aligned(16))) float sA[kC][kPA];    // a, then da
     __shared__ __attribute__((aligned(16))) float sM[K::FP][K::PB];
     __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sH[kC], sSc[2];
@@ -612,22 +687,18 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
     if constexpr (!SEL) __syncthreads();
     for (int c = c_begin; c < c_end; ++c) {
         const int nv = min(kC, a.L - c * kC);
-        float dyr[K::NE];
-        if constexpr (SEL) {
-            const float beta = a.k_scale[h];
-#pragma unroll
-            for (int e = 0; e < K::NE; ++e) R.k[e] *= beta;
+        {
+            float x[K::NE];
+            to_f32<DP, VEC>(R.dy, a.dt_dy, d0, a.D, i < nv, x);
+            put_elems<DP>(sG, i, d0, x);
         }
-#pragma unroll
-        for (int e = 0; e < K::NE; ++e) dyr[e] = R.dy[e];
-        put_elems<DP>(sQ, i, d0, R.q);
-        put_elems<DP>(sK, i, d0, R.k);
-        put_elems<DP>(sV, i, d0, R.v);
-        put_elems<DP>(sG, i, d0, R.dy);
+        put_rows<DP, VEC, false>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
         publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
         if (w == 0) put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
         __syncthreads();
         if (c + 1 < c_end) load_rows<DP, VEC, SEL, true>(a, b, h, seq, c + 1, tid, R);
+        f32x4 num = {0.f, 0.f, 0.f, 0.f};
+        if (w < 4 * K::ND) num = num_state<DP>(tb, xb, g, c16, sEc[tok], sQ, sM, sS0);
         if (w < 10) put_scores<DP, SEL>(w, nv, g, c16, sQ, sK, sPw, sCum, sA);
         __syncthreads();
         // ---- denominators (16 threads a token, all holding the result) and the dot num . dy
@@ -651,7 +722,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
             }
         }
         if (w < 4 * K::ND) {
-            const f32x4 num = num_tile<DP>(tb, xb, g, c16, sEc[tok], sQ, sV, sA, sM, sS0);
+            num = num_values(tb, xb, g, c16, sV, sA, num);
             const f32x4 dy = ld4(&sG[tok][16 * xb + 4 * g]);
             float dot = (dy[0] * num[0] + dy[1] * num[1]) + (dy[2] * num[2] + dy[3] * num[3]);
             dot = sum_lane32(sum_lane16(dot));
@@ -668,7 +739,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
             const float hout = valid && d1 >= a.eps ? -dot / (D * D) : 0.f;  // the outer clamp's adjoint
             const float hh = den >= a.eps ? hout : 0.f;                      // the call's share (inner clamp)
 #pragma unroll
-            for (int e = 0; e < K::NE; ++e) sG[i][d0 + e] = valid ? dyr[e] / D : 0.f;
+            for (int e = 0; e < K::NE; ++e) sG[i][d0 + e] = valid ? sG[i][d0 + e] / D : 0.f;
             if (part == 0) {
                 sH[i] = hh;
                 if constexpr (DIN) {
@@ -688,6 +759,21 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
         }
         __syncthreads();
         const float e63 = sSc[0], sumw = sSc[1];
+        // ---- dFq (token block tb; feature block xb and its squares): the state's part
+        const float ec = sEc[tok];
+        f32x4 fx = {0.f, 0.f, 0.f, 0.f}, fy = {0.f, 0.f, 0.f, 0.f};
+        if (w < 4 * K::ND) {
+            pipe<4, Op3>(
+                DP / 16,
+                [&](int s) {
+                    return Op3{sG[tok][4 * s + g], sM[16 * xb + c16][4 * s + g], sM[DP + 16 * xb + c16][4 * s + g]};
+                },
+                [&](const Op3 &o) {
+                    const float eg = ec * o.a;
+                    fx = mfma4(o.b, eg, fx);
+                    fy = mfma4(o.c, eg, fy);
+                });
+        }
         if (w < 10) {
             const f32x4 p = dscore_tile<DP, SEL>(w, nv, g, c16, sG, sV, sH, sPw, sCum);
             put_tile(w, g, c16, p, sA);
@@ -706,21 +792,13 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
             corr0 += wave_sum(sDh[lane]);
         }
         __syncthreads();
-        // ---- dFq (token block tb; feature block xb and its squares) -> dq
+        // ---- dFq: the chunk's part -> dq
         if (w < 4 * K::ND) {
-            const float ec = sEc[tok];
-            f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-            for (int s = 0; s < 4 * (tb + 1); ++s) {
-                const float k = sK[4 * s + g][16 * xb + c16], da = sA[tok][4 * s + g];
-                x = mfma4(k, da, x);
-                y = mfma4(0.5f * (k * k), da, y);
-            }
-#pragma unroll 8
-            for (int s = 0; s < DP / 4; ++s) {
-                const float eg = ec * sG[tok][4 * s + g];
-                x = mfma4(sM[16 * xb + c16][4 * s + g], eg, x);
-                y = mfma4(sM[DP + 16 * xb + c16][4 * s + g], eg, y);
-            }
+            pipe<4, Op2>(tb + 1, [&](int s) { return Op2{sK[4 * s + g][16 * xb + c16], sA[tok][4 * s + g]}; },
+                         [&](const Op2 &o) {
+                             fx = mfma4(o.a, o.b, fx);
+                             fy = mfma4(0.5f * (o.a * o.a), o.b, fy);
+                         });
             if (tok < nv) {
                 const int d = 16 * xb + 4 * g;
                 const f32x4 q = ld4(&sQ[tok][d]);
@@ -728,7 +806,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
                 f32x4 dq;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float x1 = x[r] + hh * sKf[d + r], y1 = y[r] + hh * sKf[DP + d + r];
+                    float x1 = fx[r] + hh * sKf[d + r], y1 = fy[r] + hh * sKf[DP + d + r];
                     if constexpr (DIN) {  // the incoming K's denominator term, under the outer clamp only
                         const float hc = ec * sHc[tok];
                         x1 += hc * sKin[d + r];
@@ -792,10 +870,10 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
 template <int DP, bool SEL, bool VEC, bool DUAL>
 __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args a) {
     using K = Dim<DP>;
-    __shared__ __attribute__((aligned(16))) float sQ[kC][K::PB];
-    __shared__ __attribute__((aligned(16))) float sK[kC][K::PP];
-    __shared__ __attribute__((aligned(16))) float sV[kC][K::PP];
-    __shared__ __attribute__((aligned(16))) float sG[kC][K::PB];
+    __shared__ __attribute__((aligned(16))) float sQ[kC][K::PC];
+    __shared__ __attribute__((aligned(16))) float sK[kC][K::PR];
+    __shared__ __attribute__((aligned(16))) float sV[kC][K::PR];
+    __shared__ __attribute__((aligned(16))) float sG[kC][K::PC];
     __shared__ __attribute__((aligned(16))) float sA[kC][kPAt];     // a, then da
     __shared__ __attribute__((aligned(16))) float sM[K::FP][K::PB];  // dM
     __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sH[kC], sEh[kC], sSc[2];
@@ -832,61 +910,81 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
     float dl_carry = SEL && !DUAL && seg == a.G - 1 ? a.fin[seq] : 0.f, dks = 0.f;
     Rows<DP> R;
     float inv = 0.f, hd = 0.f;  // the token's 1/D and h
+    float seg_ld = 0.f;         // (DUAL, selective, wave 0) the segment's log decay
     auto load = [&](int c) {
         load_rows<DP, VEC, SEL, true>(a, b, h, seq, c, tid, R);
-        const int t = c * kC + i;
-        const size_t o = static_cast<size_t>(seq) * a.L + (t < a.L ? t : 0);
-        inv = t < a.L ? a.inv_den[o] : 0.f;
-        hd = t < a.L ? a.g_den[o] : 0.f;
+        const size_t o = static_cast<size_t>(seq) * a.L + c * kC;
+        const int r = min(i, a.L - c * kC - 1);
+        inv = (a.inv_den + o)[r];
+        hd = (a.g_den + o)[r];
     };
     load(c_end - 1);
     if constexpr (!SEL) __syncthreads();
     for (int c = c_end - 1; c >= c_begin; --c) {
         const int nv = min(kC, a.L - c * kC);
-        if constexpr (SEL) {
-            const float beta = a.k_scale[h];
-#pragma unroll
-            for (int e = 0; e < K::NE; ++e) R.k[e] *= beta;
-        }
-        const bool valid = i < nv;
         float gr[K::NE];
+        to_f32<DP, VEC>(R.dy, a.dt_dy, d0, a.D, i < nv, gr);
 #pragma unroll
-        for (int e = 0; e < K::NE; ++e) gr[e] = valid ? R.dy[e] * inv : 0.f;
-        put_elems<DP>(sQ, i, d0, R.q);
-        put_elems<DP>(sK, i, d0, R.k);
-        put_elems<DP>(sV, i, d0, R.v);
+        for (int e = 0; e < K::NE; ++e) gr[e] = i < nv ? gr[e] * inv : 0.f;
         put_elems<DP>(sG, i, d0, gr);
+        put_rows<DP, VEC, false>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
         publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
-        if (part == 0) sH[i] = hd;
-        if (w == 0) put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
+        if (part == 0) sH[i] = i < nv ? hd : 0.f;
+        if (w == 0) {
+            put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
+            if (SEL && DUAL) seg_ld += wave_sum(lane < nv ? R.ld : 0.f);
+        }
         __syncthreads();
         if (c > c_begin) load(c - 1);
         if (tid < kC) sEh[tid] = sEc[tid] * sH[tid];
-        if (!DUAL && w < 10) put_scores<DP, SEL>(w, nv, g, c16, sQ, sK, sPw, sCum, sA);
+        const float wj = sW[tok];
+        // ---- dv^T tile (value block xb, tokens of block jb): the carried adjoint's part, w_j (Fk_j dM + dS0)
+        f32x4 ov = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (!DUAL) {
+            if (w < 4 * K::ND) {
+                f32x4 y = {0.f, 0.f, 0.f, 0.f};
+                pipe<4, Op3>(
+                    DP / 16,
+                    [&](int s) {
+                        return Op3{sK[tok][4 * s + g], sM[4 * s + g][16 * xb + c16], sM[DP + 4 * s + g][16 * xb + c16]};
+                    },
+                    [&](const Op3 &o) {
+                        const float wk = wj * o.a;
+                        ov = mfma4(o.b, wk, ov);
+                        y = mfma4(o.c, 0.5f * (wk * o.a), y);
+                    });
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ov[r] += y[r] + wj * sS0[16 * xb + 4 * g + r];
+            }
+            if (w < 10) put_scores<DP, SEL>(w, nv, g, c16, sQ, sK, sPw, sCum, sA);
+        }
         __syncthreads();
         const float e63 = sSc[0];
         const float k0 = C.k0;  // dK0 of the state leaving the chunk
         f32x4 da = {0.f, 0.f, 0.f, 0.f};
-        const float wj = sW[tok];
+        f32x4 fx = {0.f, 0.f, 0.f, 0.f}, fy = {0.f, 0.f, 0.f, 0.f};
         if constexpr (!DUAL) {
-            // ---- dv^T tile (value block xb, tokens of block jb): sum_i a_ij g_i + w_j (Fk_j dM + dS0)
             if (w < 4 * K::ND) {
-                f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-                for (int s = 4 * jb; s < 16; ++s)  // a_ij = 0 for i < j
-                    x = mfma4(sG[4 * s + g][16 * xb + c16], sA[4 * s + g][tok], x);
-#pragma unroll 8
-                for (int s = 0; s < DP / 4; ++s) {
-                    const float k = sK[tok][4 * s + g], wk = wj * k;
-                    x = mfma4(sM[4 * s + g][16 * xb + c16], wk, x);
-                    y = mfma4(sM[DP + 4 * s + g][16 * xb + c16], 0.5f * (wk * k), y);
-                }
+                // dv: the chunk's part, sum_i a_ij g_i (a_ij = 0 for i < j)
+                pipe<4, Op2>(
+                    4 - jb,
+                    [&](int s) { return Op2{sG[16 * jb + 4 * s + g][16 * xb + c16], sA[16 * jb + 4 * s + g][tok]}; },
+                    [&](const Op2 &o) { ov = mfma4(o.a, o.b, ov); });
                 if (tok < nv) {
                     const int d = 16 * xb + 4 * g;
-                    f32x4 o;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) o[r] = x[r] + y[r] + wj * sS0[d + r];
-                    store_out(a.dv, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, o, a.D - d, VEC);
+                    store_out(a.dv, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, ov, a.D - d, VEC);
                 }
+                // ---- dFk^T tiles (feature block xb and its squares; tokens of block jb): the carried part
+                pipe<4, Op3>(
+                    DP / 16,
+                    [&](int s) {
+                        return Op3{sV[tok][4 * s + g], sM[16 * xb + c16][4 * s + g], sM[DP + 16 * xb + c16][4 * s + g]};
+                    },
+                    [&](const Op3 &o) {
+                        const float wv = wj * o.a;
+                        fx = mfma4(o.b, wv, fx);
+                        fy = mfma4(o.c, wv, fy);
+                    });
             }
             if (w < 10) da = dscore_tile<DP, SEL>(w, nv, g, c16, sG, sV, sH, sPw, sCum);
         }
@@ -900,28 +998,22 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
         if constexpr (!DUAL) {
             if (w < 10) put_tile(w, g, c16, da, sA);
             __syncthreads();
-            // ---- dFk^T tiles (feature block xb and its squares; tokens of block jb) -> dk:
-            //      sum_i da_ij Fq_i + w_j (dM v_j + dKf)
+            // ---- dFk: the chunk's part, sum_i da_ij Fq_i -> dk
             if (w < 4 * K::ND) {
-                f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-                for (int s = 4 * jb; s < 16; ++s) {
-                    const float q = sQ[4 * s + g][16 * xb + c16], d = sA[4 * s + g][tok];
-                    x = mfma4(q, d, x);
-                    y = mfma4(q * q, d, y);
-                }
-#pragma unroll 8
-                for (int s = 0; s < DP / 4; ++s) {
-                    const float wv = wj * sV[tok][4 * s + g];
-                    x = mfma4(sM[16 * xb + c16][4 * s + g], wv, x);
-                    y = mfma4(sM[DP + 16 * xb + c16][4 * s + g], wv, y);
-                }
+                pipe<4, Op2>(
+                    4 - jb,
+                    [&](int s) { return Op2{sQ[16 * jb + 4 * s + g][16 * xb + c16], sA[16 * jb + 4 * s + g][tok]}; },
+                    [&](const Op2 &o) {
+                        fx = mfma4(o.a, o.b, fx);
+                        fy = mfma4(o.a * o.a, o.b, fy);
+                    });
                 const int d = 16 * xb + 4 * g;
                 const f32x4 k = ld4(&sK[tok][d]);
                 f32x4 dk;
                 float pkp = 0.f;  // SEL: sum over this lane's features of Fk . dFk
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float x1 = x[r] + wj * sKf[d + r], y1 = y[r] + wj * sKf[DP + d + r];
+                    const float x1 = fx[r] + wj * sKf[d + r], y1 = fy[r] + wj * sKf[DP + d + r];
                     dk[r] = x1 + k[r] * y1;
                     if constexpr (SEL) pkp += k[r] * x1 + 0.5f * (k[r] * k[r]) * y1;
                 }
@@ -934,11 +1026,12 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
                 if (tok < nv) {
                     if constexpr (SEL) {
                         const float ks = a.k_scale[h];
+                        const void *kp = static_cast<const char *>(a.k) +
+                                         (b * a.k_sb + (h / a.group) * a.k_sh + static_cast<int64_t>(c) * kC * a.k_sl) *
+                                             (a.dt_k == PRIME_F32 ? 4 : 2);
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            if (d + r < a.D)
-                                dks += load_elem(a.k, b * a.k_sb + (h / a.group) * a.k_sh +
-                                                          static_cast<int64_t>(c * kC + tok) * a.k_sl + d + r, a.dt_k) * dk[r];
+                            if (d + r < a.D) dks += load_elem(kp, min(tok, nv - 1) * a.k_sl + d + r, a.dt_k) * dk[r];
                             dk[r] *= ks;
                         }
                     }
@@ -979,6 +1072,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
     }
     if constexpr (DUAL) {
         store_carry<DP>(slot_state(slot), a.D, 1.0f, u, g, c16, tid, C);
+        if (SEL && tid == 0) slot[kWsDecay] = seg_ld * 1.44269504088896341f;  // log2
         return;
     }
     if constexpr (SEL) {  // the key scale's adjoint, this unit's share; the segment's suffix total
@@ -1049,6 +1143,23 @@ void launch_dkv_dp(const ChunkF32Args &a, dim3 grid, hipStream_t s, const TimerE
 
 }  // namespace
 
+// Selective backward in segments: each segment's dk/dv pass left the suffix sums of
+// its own tokens and its totals; every token gets the later segments' totals added,
+// and the key scale's adjoint is summed over the segments.  One workgroup a sequence.
+__global__ __launch_bounds__(256) void chunk_f32_seg_totals_kernel(const ChunkF32Args a) {
+    const int seq = blockIdx.x;
+    const float *tot = a.seg_tot + static_cast<size_t>(seq) * a.G * 2;
+    float ks = 0.f;
+    for (int s = 0; s < a.G; ++s) ks += tot[2 * s + 1];
+    if (threadIdx.x == 0) a.dkscale[seq] = ks;
+    const int T = a.cps * kC;
+    float carry = 0.f;
+    for (int s = a.G - 2; s >= 0; --s) {
+        carry += tot[2 * (s + 1)];
+        for (int t = s * T + threadIdx.x; t < (s + 1) * T; t += 256) a.dlogd[static_cast<size_t>(seq) * a.L + t] += carry;
+    }
+}
+
 hipError_t launch_chunk_f32_prefill(const ChunkF32Args &a, hipStream_t stream) {
     const TimerEvents t = timer_events(PRIME_KERNEL_PREFILL_CHUNKS);
     const dim3 grid(a.B * a.H * a.G);
@@ -1073,6 +1184,110 @@ hipError_t launch_chunk_f32_backward(const ChunkF32Args &a, hipStream_t stream) 
     else if (a.D <= 32) launch_dkv_dp<32, false>(a, grid, stream, t2);
     else launch_dkv_dp<64, false>(a, grid, stream, t2);
     if ((e = hipGetLastError()) != hipSuccess) timer_drop(t2);
+    return e;
+}
+
+// ---------------------------------------------------------------------------
+// D = 64, fp32 rows on 16-byte boundaries: selective PRIME's prefill and both
+// backwards, few long sequences in segments.
+// ---------------------------------------------------------------------------
+namespace {
+
+template <class A>
+void copy_common(ChunkF32Args &o, const A &a) {
+    o.q = a.q; o.k = a.k; o.v = a.v;
+    o.q_sb = a.q_sb; o.q_sh = a.q_sh; o.q_sl = a.q_sl;
+    o.k_sb = a.k_sb; o.k_sh = a.k_sh; o.k_sl = a.k_sl;
+    o.v_sb = a.v_sb; o.v_sh = a.v_sh; o.v_sl = a.v_sl;
+    o.dt_q = o.dt_k = o.dt_v = a.dt_in;
+    o.B = a.B; o.H = a.H; o.L = a.L; o.D = kD; o.group = 1;
+    o.decay = a.decay; o.eps = a.eps;
+    o.s0i = a.s0i; o.s1i = a.s1i; o.s2i = a.s2i; o.k0i = a.k0i; o.k1i = a.k1i; o.k2i = a.k2i;
+    o.G = a.G; o.cps = a.cps; o.slots = a.ws;
+}
+
+// every segment's state from zero, then the state entering each
+hipError_t launch_segment_states(const ChunkF32Args &o, const PrefillArgs &p, hipStream_t stream) {
+    const TimerEvents ta = timer_events(PRIME_KERNEL_PREFILL_SEGMENTS);
+    const dim3 grid(o.B * o.H * (o.G - 1));
+    if (o.selective)
+        hipExtLaunchKernelGGL((chunk_f32_prefill_kernel<64, false, true, true, true>), grid, dim3(kT), 0, stream,
+                              ta.start, ta.stop, 0, o);
+    else
+        hipExtLaunchKernelGGL((chunk_f32_prefill_kernel<64, false, false, true, true>), grid, dim3(kT), 0, stream,
+                              ta.start, ta.stop, 0, o);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return timer_drop(ta), e;
+    return launch_segment_scan(p, stream);
+}
+
+}  // namespace
+
+hipError_t launch_selective_f32(const PrefillArgs &a, hipStream_t stream) {
+    ChunkF32Args o{};
+    copy_common(o, a);
+    o.group = a.group;
+    o.selective = 1;
+    o.log_decay = a.log_decay; o.k_scale = a.k_scale;
+    o.s0o = a.s0o; o.s1o = a.s1o; o.s2o = a.s2o; o.k0o = a.k0o; o.k1o = a.k1o; o.k2o = a.k2o;
+    o.y = a.y; o.dt_y = a.dt_y; o.y_sb = a.y_sb; o.y_sh = a.y_sh; o.y_sl = a.y_sl;
+    hipError_t e;
+    if (a.G > 1 && (e = launch_segment_states(o, a, stream)) != hipSuccess) return e;
+    const TimerEvents t = timer_events(PRIME_KERNEL_PREFILL_CHUNKS);
+    hipExtLaunchKernelGGL((chunk_f32_prefill_kernel<64, false, true, true, false>), dim3(a.B * a.H * a.G), dim3(kT), 0,
+                          stream, t.start, t.stop, 0, o);
+    if ((e = hipGetLastError()) != hipSuccess) timer_drop(t);
+    return e;
+}
+
+hipError_t launch_prefill_backward_f32(const BwdArgs &a, hipStream_t stream) {
+    ChunkF32Args o{};
+    copy_common(o, a);
+    const bool sel = a.logd != nullptr;
+    o.selective = sel;
+    o.log_decay = a.logd; o.k_scale = a.kscale;
+    o.dense_clamp = a.dense_in;
+    o.dy = a.dy; o.dt_dy = a.dt_dy; o.dy_sb = a.dy_sb; o.dy_sh = a.dy_sh; o.dy_sl = a.dy_sl;
+    o.ds0 = a.ds0o; o.ds1 = a.ds1o; o.ds2 = a.ds2o; o.dk0 = a.dk0o; o.dk1 = a.dk1o; o.dk2 = a.dk2o;
+    o.dsi0 = a.ds0i; o.dsi1 = a.ds1i; o.dsi2 = a.ds2i; o.dki0 = a.dk0i; o.dki1 = a.dk1i; o.dki2 = a.dk2i;
+    o.dq = a.dq; o.dk = a.dk; o.dv = a.dv; o.dt_g = a.dt_g; o.g_sb = a.g_sb; o.g_sh = a.g_sh; o.g_sl = a.g_sl;
+    o.inv_den = a.inv_den; o.g_den = a.g_den;
+    o.kc1 = a.kcorr; o.kc2 = a.kcorr + kD; o.kc0 = a.kcorr + 2 * kD;
+    o.kc_s = o.kc0_s = kBwdCorr;
+    o.dlogd = a.dlogd; o.dkscale = a.dkscale; o.pq = a.pq; o.fin = a.fin; o.seg_tot = a.seg_tot;
+    const dim3 grid(a.B * a.H * a.G), block(kT);
+    hipError_t e;
+    if (a.G > 1) {
+        // (in fp32: the states of the prefill's own state-only pass, formed from operands split
+        // into two bf16 parts, put dq 4e-6 from float64 at 8 segments, against 9e-7)
+        PrefillArgs p{};
+        p.B = a.B; p.H = a.H; p.group = 1; p.L = a.L; p.G = a.G; p.cps = a.cps; p.ws = a.ws;
+        p.decay = a.decay; p.log_decay = a.logd;
+        p.s0i = a.s0i; p.s1i = a.s1i; p.s2i = a.s2i; p.k0i = a.k0i; p.k1i = a.k1i; p.k2i = a.k2i;
+        if ((e = launch_segment_states(o, p, stream)) != hipSuccess) return e;
+    }
+    const TimerEvents t1 = timer_events(PRIME_KERNEL_BWD_DQ);
+    launch_dq_dp<64, true>(o, grid, stream, t1);
+    if ((e = hipGetLastError()) != hipSuccess) return timer_drop(t1), e;
+    if (a.G > 1) {
+        // each segment's dual contribution, then the reverse scan (slots now hold dual states)
+        const TimerEvents td = timer_events(PRIME_KERNEL_BWD_DUAL);
+        if (sel)
+            hipExtLaunchKernelGGL((chunk_f32_dkv_kernel<64, true, true, true>), grid, block, 0, stream, td.start, td.stop,
+                                  0, o);
+        else
+            hipExtLaunchKernelGGL((chunk_f32_dkv_kernel<64, false, true, true>), grid, block, 0, stream, td.start,
+                                  td.stop, 0, o);
+        if ((e = hipGetLastError()) != hipSuccess) return timer_drop(td), e;
+        if ((e = launch_bwd_dual_scan(a, stream)) != hipSuccess) return e;
+    }
+    const TimerEvents t2 = timer_events(PRIME_KERNEL_BWD_DKV);
+    launch_dkv_dp<64, true>(o, grid, stream, t2);
+    if ((e = hipGetLastError()) != hipSuccess) return timer_drop(t2), e;
+    if (sel && a.G > 1) {
+        hipLaunchKernelGGL(chunk_f32_seg_totals_kernel, dim3(a.B * a.H), dim3(256), 0, stream, o);
+        e = hipGetLastError();
+    }
     return e;
 }
 

@@ -967,9 +967,12 @@ __global__ __launch_bounds__(256) void bwd_dual_scan_kernel(const BwdArgs a) {
     if (gid >= static_cast<int64_t>(S) * kWsElems) return;
     const int seq = static_cast<int>(gid / kWsElems), e = static_cast<int>(gid % kWsElems);
     const int h = seq % a.H;
-    const double ld = static_cast<double>(a.decay[h]);
-    const float lT = static_cast<float>(pow(ld, static_cast<double>(a.cps) * kC));
-    const float lLast = static_cast<float>(pow(ld, static_cast<double>(a.L - (a.G - 1) * a.cps * kC)));
+    // (selective: segment s's own log2 decay, beside its slot's state)
+    const bool sel = a.logd != nullptr;
+    const double ld = sel ? 1.0 : static_cast<double>(a.decay[h]);
+    const float lT = sel ? 0.f : static_cast<float>(pow(ld, static_cast<double>(a.cps) * kC));
+    const float lLast = sel ? 0.f : static_cast<float>(pow(ld, static_cast<double>(a.L - (a.G - 1) * a.cps * kC)));
+    const float f2 = sel ? 1.0f : 2.0f;  // the kernels' factor on the second-order adjoints
     const size_t so1 = static_cast<size_t>(seq) * kD * kD, so0 = static_cast<size_t>(seq) * kD;
     // the element's place in the reference state, and the factor of this kernel's convention
     const float *src = nullptr;
@@ -977,17 +980,18 @@ __global__ __launch_bounds__(256) void bwd_dual_scan_kernel(const BwdArgs a) {
     size_t off = 0;
     float fac = 1.0f;
     if (e < kWsS2) { src = a.ds1o; dst = a.ds1i; off = so1 + e; }
-    else if (e < kWsS0) { src = a.ds2o; dst = a.ds2i; off = so1 + e - kWsS2; fac = 2.0f; }
+    else if (e < kWsS0) { src = a.ds2o; dst = a.ds2i; off = so1 + e - kWsS2; fac = f2; }
     else if (e < kWsK1) { src = a.ds0o; dst = a.ds0i; off = so0 + e - kWsS0; }
     else if (e < kWsK2) { src = a.dk1o; dst = a.dk1i; off = so0 + e - kWsK1; }
-    else if (e < kWsK0) { src = a.dk2o; dst = a.dk2i; off = so0 + e - kWsK2; fac = 2.0f; }
+    else if (e < kWsK0) { src = a.dk2o; dst = a.dk2i; off = so0 + e - kWsK2; fac = f2; }
     else { src = a.dk0o; dst = a.dk0i; off = seq; }
     float carry = a.ds1o ? fac * src[off] : 0.f;
     float *slot = a.ws + static_cast<size_t>(seq) * a.G * kWsStride + e;
     for (int s = a.G - 1; s >= 0; --s) {
         const float cs = slot[static_cast<size_t>(s) * kWsStride];
+        const float f = sel ? exp2f(slot[static_cast<size_t>(s) * kWsStride + kWsDecay - e]) : s == a.G - 1 ? lLast : lT;
         slot[static_cast<size_t>(s) * kWsStride] = carry;
-        carry = (s == a.G - 1 ? lLast : lT) * carry + cs;
+        carry = f * carry + cs;
     }
     if (a.ds1i) dst[off] = carry / fac;
 }
@@ -1007,18 +1011,21 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
     int g = 1;
     const int cu = device_cus();
     if (S > 0 && S < per_cu * cu) g = min(min(per_cu * cu / S, NC / 8), 64);
-    if (per_cu == 1 && S > 0 && S < cu) {
-        // one workgroup per CU: the passes take (rounds of units over the CUs) x
-        // (chunks per segment) chunk periods; take the fewest, then the fewest
-        // segments (G = 2 leaves a quarter of the CUs idle at 96 sequences,
-        // G = 8 fills three rounds exactly)
-        long best = static_cast<long>(NC);
+    if (per_cu == 1 && S > 0) {
+        // fp32 passes, one workgroup per CU: in periods of a chunk of the dq or dk/dv
+        // pass (16-18 us each), a round of units over the CUs costs 2 a chunk, with
+        // segments 2.6 (the state-only and dual passes) and about 1.2 for the two scans
+        // and their slots' traffic.  96 sequences of 16 chunks: 8 segments 17.6 against 22
+        // with 2; 48 sequences of 13: 5 segments 9.2 against 26 with one.
+        double best = 1.9 * NC * ((S + cu - 1) / cu);  // (segments only where they pay by 5 %)
         g = 1;
-        for (int t = 2; t <= min(NC / 8, 64); ++t) {
-            const long c = (NC + t - 1) / t, rounds = (static_cast<long>(S) * t + cu - 1) / cu;
-            if (rounds * c < best) {
-                best = rounds * c;
-                g = t;
+        for (int t = 2; t <= min(NC, 64); ++t) {
+            const int c = (NC + t - 1) / t, u = (NC + c - 1) / c;
+            const double rounds = static_cast<double>((static_cast<int64_t>(S) * u + cu - 1) / cu);
+            const double cost = 2.6 * rounds * c + 1.2 + 0.001 * S * u;
+            if (cost < best - 1e-9) {
+                best = cost;
+                g = u;
             }
         }
     }
@@ -1033,6 +1040,7 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
 }
 
 hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream) {
+    if (a.dt_in == PRIME_F32) return launch_prefill_backward_f32(a, stream);
     const int S = a.B * a.H;
     hipError_t e;
     if (a.G > 1) {
@@ -1048,7 +1056,6 @@ hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream) {
         f.G = a.G; f.cps = a.cps; f.ws = a.ws; f.states_only = 1;
         if ((e = launch_prefill(f, stream)) != hipSuccess) return e;
     }
-    if (a.dt_in == PRIME_F32) return launch_prefill_backward_f32(a, stream);
     const int units = S * a.G;
     const TimerEvents t1 = timer_events(PRIME_KERNEL_BWD_DQ);
     if (a.dense_in)

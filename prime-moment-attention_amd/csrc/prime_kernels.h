@@ -210,15 +210,16 @@ struct BwdArgs {
     // scale's adjoint per sequence).  Scratch: pq [B*H, L], fin [B*H].
     const float *logd, *kscale;
     float *dlogd, *dkscale, *pq, *fin;
+    float *seg_tot;  // selective, G > 1: scratch [B*H][G][2]
 };
 constexpr int kBwdCorr = 132;  // floats per sequence in BwdArgs::kcorr (128 features, K0, padding)
 
 hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream);
-// fp32 inputs: the fp32 dq and dk/dv passes, one workgroup per sequence (prefill_bwd_f32.hip)
+// fp32 inputs: the fp32 dq and dk/dv passes (chunk_f32.hip)
 hipError_t launch_prefill_backward_f32(const BwdArgs &a, hipStream_t stream);
 // segments per sequence for the backward: enough (sequence, segment) units to
-// fill per_cu workgroups per CU (2 for the bf16 passes, 1 for the fp32 ones),
-// at least 8 chunks per segment
+// fill per_cu workgroups per CU (2 for the bf16 passes, of at least 8 chunks a
+// segment; 1 for the fp32 ones, by their passes' costs)
 void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu = 2);
 // the reverse scan over segments of the backward's dual states (prefill_bwd.hip)
 hipError_t launch_bwd_dual_scan(const BwdArgs &a, hipStream_t stream);
@@ -229,7 +230,7 @@ hipError_t launch_prefill(PrefillArgs a, hipStream_t stream);
 // the scan over a prefill's segments: slot s <- the state entering segment s
 // (prefill.hip)
 hipError_t launch_segment_scan(const PrefillArgs &a, hipStream_t stream);
-// selective form with fp32 inputs: one fp32 kernel over each sequence's chunks (selective_f32.hip)
+// selective form with fp32 inputs (chunk_f32.hip)
 hipError_t launch_selective_f32(const PrefillArgs &a, hipStream_t stream);
 // segments per sequence for the launch plan, given the workspace the caller has
 void plan_segments(int S, int L, bool dense_clamp, size_t ws_bytes, int *G, int *cps);

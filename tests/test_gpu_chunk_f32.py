@@ -10,6 +10,7 @@ import torch
 from oracle import oracle as O
 from prime_moment_attention import _lib
 
+import test_gpu_selective_backward as SB
 from gpu_util import dev, random_state, state_to_dev, state_to_np, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -112,3 +113,48 @@ def test_chunk_f32_dense_clamp_backward_scratch(D):
     torch.cuda.synchronize()
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("L", [65, 130, 64 * 9 + 1])
+def test_chunk_f32_base_backward_segments(L):
+    """Head dim 64 in fp32, few sequences: one segment, two, several of few chunks."""
+    B, H, D = 1, 2, 64
+    q, k, v, lam, rng = _case(B, H, L, D, 50 + L)
+    st0 = random_state(B * H, D, 51)
+    dy = rng.standard_normal(q.shape).astype(np.float32)
+    ds = tuple(0.1 * rng.standard_normal(x.shape) for x in O.zero_state(B * H, D))
+    ref = O.recurrent_vjp(*(x.reshape(B * H, L, D) for x in (q, k, v)), np.tile(lam.astype(np.float64), B),
+                          dy.reshape(B * H, L, D), eps=1.0, state=st0, dstate=ds)
+    g, dsi = [torch.empty(q.shape, device=dev()) for _ in range(3)], _lib.new_state(B, H, D, dev())
+    _lib.chunked_prefill_backward(*(to_dev(x) for x in (q, k, v, lam)), 1.0, state_to_dev(st0, B, H, D), to_dev(dy),
+                                  state_to_dev(ds, B, H, D), *g, dsi)
+    torch.cuda.synchronize()
+    for n, x, r in zip(("dq", "dk", "dv"), g, ref[:3]):
+        _close(to_np(x), r, n)
+    for n, x, r in zip("S0 S1 S2 K0 K1 K2".split(), state_to_np(dsi, B * H, D), ref[3]):
+        _close(x, r, "d" + n)
+
+
+@pytest.mark.parametrize("L,with_state", [(130, False), (64 * 5, True), (64 * 13 - 55, True)])
+def test_chunk_f32_selective_backward_segments(L, with_state):
+    """Few sequences: the selective backward in segments (every gradient, the decay
+    sums carried over the segments), and in one where the workspace holds no slots."""
+    B, H = 1, 3
+    args = SB._case(B, H, L, 70 + L, with_state, with_state)
+    q, k, v, ld, beta, dy, st, ds = args
+    small = (B * H * L * 8 + 255) // 256 * 256 + B * H * (L + 1) * 4
+    assert _lib.selective_backward_workspace_size(B, H, L) > small
+    ref = SB._reference(*args, 1.0)
+    for ws in (None, torch.empty(small, dtype=torch.uint8, device=dev())):
+        g = [torch.empty(q.shape, device=dev()) for _ in range(3)]
+        dld, dks = torch.empty(B, H, L, device=dev()), torch.empty(B, H, device=dev())
+        dsi = _lib.new_state(B, H, 64, dev()) if with_state else None
+        dst = lambda s: state_to_dev(s, B, H, 64) if s is not None else None
+        _lib.selective_prefill_backward(*(to_dev(x) for x in (q, k, v, ld, beta)), 1.0, dst(st), to_dev(dy), dst(ds),
+                                        *g, dsi, dld, dks, workspace=ws)
+        torch.cuda.synchronize()
+        for n, x in zip(("dq", "dk", "dv", "dlog_decay", "dk_scale"), (*g, dld, dks)):
+            _close(to_np(x), ref[n], n)
+        if with_state:
+            for x, r in zip(dsi, ref["dstate_in"]):
+                _close(to_np(x), r, "dstate")
