@@ -252,6 +252,20 @@ int prime_delta_prefill(const prime_tensor_t *q, const prime_tensor_t *k,
 size_t prime_delta_prefill_workspace_size(int B, int H, int L, unsigned flags);
 
 /*
+ * prime_delta_gates: the write rates and decays prime_delta_prefill and
+ * prime_delta_decode_step take, from the gate projections' pre-activations
+ * (chunked_delta_prime.py:110-111, 133-137): per token and head, beta = 0.5
+ * mean(sigmoid(write)), alpha = decay (1 - 0.5 mean(sigmoid(erase))), the mean
+ * over the head's D columns in fp32 of sigmoids rounded to `dtype`.
+ *   erase, write: [B, L, H*D], batch and token strides in elements, contiguous
+ *                 columns, one dtype (F32, BF16, F16); 1 <= D <= 64
+ *   beta, alpha : fp32 [B, H, L], disjoint from the inputs and each other
+ */
+int prime_delta_gates(const void *erase, int64_t erase_sb, int64_t erase_sl, const void *write, int64_t write_sb,
+                      int64_t write_sl, int dtype, float decay, int B, int H, int L, int D, float *beta, float *alpha,
+                      void *stream);
+
+/*
  * Backward of prime_delta_prefill: gradients of the chunked delta-rule
  * prefill (the autograd graph of chunked_delta_prime.py:177-283 -- features
  * :73-87, the per-chunk triangular solve, the per-chunk Lyapunov clamp) with

@@ -347,6 +347,34 @@ int prime_selective_log_decay(const void *step, int step_dtype, int64_t step_sb,
                      "selective log decay launch");
 }
 
+int prime_delta_gates(const void *erase, int64_t erase_sb, int64_t erase_sl, const void *write, int64_t write_sb,
+                      int64_t write_sl, int dtype, float decay, int B, int H, int L, int D, float *beta, float *alpha,
+                      void *stream) {
+    g_err[0] = 0;
+    if (!erase || !write || !beta || !alpha) return fail(PRIME_ERR_INVALID_ARG, "prime_delta_gates: null argument");
+    if (B <= 0 || H <= 0 || L <= 0 || erase_sb < 0 || erase_sl < 0 || write_sb < 0 || write_sl < 0)
+        return fail(PRIME_ERR_INVALID_ARG, "bad sizes B=%d H=%d L=%d or negative strides", B, H, L);
+    if (D < 1 || D > prime::kD) return fail(PRIME_ERR_UNSUPPORTED_DIM, "head dim %d unsupported (1 .. %d)", D, prime::kD);
+    if (!valid_dtype(dtype)) return fail(PRIME_ERR_UNSUPPORTED_DTYPE, "unsupported gate dtype");
+    if (B > 65535 || (H + 3) / 4 > 65535) return fail(PRIME_ERR_INVALID_ARG, "B=%d or H=%d above the grid's limit", B, H);
+    const int64_t es = elem_size(dtype);
+    if (reinterpret_cast<uintptr_t>(erase) % es || reinterpret_cast<uintptr_t>(write) % es ||
+        (reinterpret_cast<uintptr_t>(beta) & 3) || (reinterpret_cast<uintptr_t>(alpha) & 3))
+        return fail(PRIME_ERR_MISALIGNED, "erase, write, beta or alpha misaligned");
+    const size_t nout = static_cast<size_t>(B) * H * L * sizeof(float);
+    const size_t ne = static_cast<size_t>((B - 1) * erase_sb + (L - 1) * erase_sl + static_cast<int64_t>(H) * D) * es;
+    const size_t nw = static_cast<size_t>((B - 1) * write_sb + (L - 1) * write_sl + static_cast<int64_t>(H) * D) * es;
+    if (overlap(beta, nout, erase, ne) || overlap(beta, nout, write, nw) || overlap(alpha, nout, erase, ne) ||
+        overlap(alpha, nout, write, nw) || overlap(alpha, nout, beta, nout))
+        return fail(PRIME_ERR_ALIAS, "beta or alpha overlaps erase, write or each other");
+    prime::DeltaGateArgs a{};
+    a.erase = erase; a.write = write;
+    a.e_sb = erase_sb; a.e_sl = erase_sl; a.w_sb = write_sb; a.w_sl = write_sl;
+    a.dt = dtype; a.B = B; a.H = H; a.L = L; a.D = D;
+    a.decay = decay; a.beta = beta; a.alpha = alpha;
+    return check_hip(prime::launch_delta_gates(a, static_cast<hipStream_t>(stream)), "delta gates launch");
+}
+
 int prime_head_layernorm(const prime_tensor_t *x, const prime_tensor_t *out, int B, int H, int L, int D,
                          const void *weight, const void *bias, int param_dtype, float ln_eps, float scale,
                          void *stream) {

@@ -16,7 +16,6 @@ constexpr int kPW = kF + 8;     // pitch of 128-wide rows read 16 bytes per lane
 // 44-dword pitches to fit in LDS.
 constexpr int kPT = kF + 16;
 
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short i16x4;
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2;

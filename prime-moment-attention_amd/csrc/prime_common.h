@@ -14,6 +14,7 @@ constexpr int kWave = 64;   // CDNA wavefront
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4;
 
 // ---------------------------------------------------------------- conversions
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {

@@ -121,6 +121,17 @@ hipError_t launch_gelu(const void *x, void *y, int64_t n, int dt, hipStream_t st
 hipError_t launch_selective_log_decay(const void *step, int dt, int64_t sb, int64_t sl, const float *tau, float dmin,
                                       float dmax, int B, int H, int L, float *out, hipStream_t stream);
 
+// Delta-rule write rates and decays from the gate pre-activations (norm.hip):
+// erase, write [B, L, H D] rows (element strides), beta and alpha [B, H, L].
+struct DeltaGateArgs {
+    const void *erase, *write;
+    int64_t e_sb, e_sl, w_sb, w_sl;
+    int dt, B, H, L, D;
+    float decay;
+    float *beta, *alpha;
+};
+hipError_t launch_delta_gates(const DeltaGateArgs &a, hipStream_t stream);
+
 struct PrefillArgs {
     const void *q, *k, *v;
     int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;

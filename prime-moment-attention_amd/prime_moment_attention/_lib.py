@@ -34,7 +34,7 @@ EXPORTS = ("prime_abi_version", "prime_last_error", "prime_decode_step", "prime_
            "prime_selective_prefill_backward_workspace_size", "prime_hbm_stream",
            "prime_frag_rows", "prime_pack_frag", "prime_linear_frag_workspace_size", "prime_linear_frag",
            "prime_delta_prefill_backward", "prime_delta_prefill_backward_workspace_size",
-           "prime_delta_decode_step_backward")
+           "prime_delta_decode_step_backward", "prime_delta_gates")
 
 # bytes of the fixed device scratch behind prime_accumulate_noalloc
 NOALLOC_SCRATCH_BYTES = 32 << 20
@@ -181,6 +181,9 @@ def load() -> ctypes.CDLL:
     L.prime_delta_prefill_backward.argtypes = [P(PrimeTensor)] * 3 + [fp, fp] + [ctypes.c_int] * 6 + [
         ctypes.c_float] * 3 + [fp, P(PrimeTensor)] + [fp] * 8 + [ctypes.c_size_t, fp]
     L.prime_delta_prefill_backward.restype = ctypes.c_int
+    L.prime_delta_gates.argtypes = [fp, ctypes.c_int64, ctypes.c_int64] * 2 + [ctypes.c_int, ctypes.c_float] + [
+        ctypes.c_int] * 4 + [fp] * 3
+    L.prime_delta_gates.restype = ctypes.c_int
     L.prime_frag_rows.argtypes = [ctypes.c_int]
     L.prime_frag_rows.restype = ctypes.c_int
     L.prime_pack_frag.argtypes = [fp, ctypes.c_int64, ctypes.c_int64, fp, ctypes.c_int, ctypes.c_int, fp, fp]
@@ -871,6 +874,24 @@ def delta_prefill(q, k, v, beta, alpha, decay_pad: float, feat_eps: float, bound
                                     ptr(state_in), ctypes.byref(yd), ptr(state_out), ptr(workspace),
                                     workspace.numel() if workspace is not None else 0, _stream(q.device))
     _check(rc, "prime_delta_prefill")
+
+
+def delta_gates(erase: torch.Tensor, write: torch.Tensor, decay: float, H: int, D: int):
+    """prime_delta_gates: (beta, alpha) fp32 [B, H, L] from the gate
+    projections' pre-activations [B, L, H*D] (any batch and token strides)."""
+    _dev_check(erase, write)
+    B, Lt, _ = erase.shape
+    for t, n in ((erase, "erase"), (write, "write")):
+        _shape(t, (B, Lt, H * D), n)
+        if t.stride(2) != 1 or t.dtype not in _DTYPES or t.dtype != erase.dtype:
+            raise ValueError("erase and write must share a supported dtype and have contiguous columns")
+    beta, alpha = (torch.empty(B, H, Lt, device=erase.device, dtype=torch.float32) for _ in range(2))
+    rc = load().prime_delta_gates(ctypes.c_void_p(erase.data_ptr()), erase.stride(0), erase.stride(1),
+                                  ctypes.c_void_p(write.data_ptr()), write.stride(0), write.stride(1),
+                                  _DTYPES[erase.dtype], float(decay), B, H, Lt, D, ctypes.c_void_p(beta.data_ptr()),
+                                  ctypes.c_void_p(alpha.data_ptr()), _stream(erase.device))
+    _check(rc, "prime_delta_gates")
+    return beta, alpha
 
 
 def delta_backward_workspace_size(B: int, H: int, L: int, D: int = 64, chunk: int = 64) -> int:

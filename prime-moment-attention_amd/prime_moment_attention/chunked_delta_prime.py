@@ -137,6 +137,15 @@ class ChunkedGatedDeltaPrimeAttention(nn.Module):
         alpha = (self.decay * (1.0 - b * 0.5)).transpose(1, 2).contiguous()
         return beta, alpha
 
+    def _gates_inference(self, hidden_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+        """``gates`` without autograd: the projections, then one kernel
+        (prime_delta_gates) instead of its elementwise passes and means."""
+        erase, write = self.erase_proj(hidden_states), self.write_proj(hidden_states)
+        if (not erase.is_cuda or erase.dtype not in (torch.float32, torch.bfloat16, torch.float16)
+                or write.dtype != erase.dtype or erase.stride(2) != 1 or write.stride(2) != 1):
+            return self.gates(hidden_states)
+        return _lib.delta_gates(erase, write, self.decay, self.num_heads, self.head_dim)
+
     def project(self, hidden_states: torch.Tensor):
         """q (scaled), k, v as [B, H(kv), L, D] (chunked_delta_prime.py:105-126)."""
         B, L, _ = hidden_states.shape
@@ -159,7 +168,7 @@ class ChunkedGatedDeltaPrimeAttention(nn.Module):
                                                   (state is not None and state.requires_grad)):
             return self._forward_train(hidden_states, state, return_state)
         q, k, v = self.project(hidden_states)
-        beta, alpha = self.gates(hidden_states)
+        beta, alpha = self._gates_inference(hidden_states)
         if q.dtype not in (torch.bfloat16, torch.float32):
             q, k, v = q.float(), k.float(), v.float()
         y_dtype = dtype if dtype in (torch.float32, torch.bfloat16, torch.float16) else torch.float32
@@ -175,7 +184,8 @@ class ChunkedGatedDeltaPrimeAttention(nn.Module):
         else:
             q, k, v = (t if (t.stride(-1) == 1 and all((s * t.element_size()) % 16 == 0 for s in t.stride()[:-1]))
                        else t.contiguous() for t in (q, k, v))
-            y = torch.empty(B, H, L, D, device=dev, dtype=y_dtype)
+            # y written in the o_proj input layout [B, L, H, D] through strides
+            y = torch.empty(B, L, H, D, device=dev, dtype=y_dtype).transpose(1, 2)
             _lib.delta_prefill(q, k, v, beta, alpha, self.decay, self.eps, self.lyapunov_bound, s_in, y, s_out,
                                chunk=self.chunk_size)
         y = no_backward("the delta-rule PRIME (inference path)", y, q, k, v, beta, alpha, s_in)

@@ -127,6 +127,21 @@ def test_selective_log_decay_validates_before_device_work():
                                        None) == -5  # out runs into tau
 
 
+def test_delta_gates_validates_before_device_work():
+    """prime_delta_gates rejects null, out-of-range, misaligned and overlapping
+    arguments with its error codes (no launch)."""
+    L = _lib.load()
+    p = [ctypes.c_void_p((i + 1) << 24) for i in range(4)]
+    bf = _lib.PRIME_BF16
+
+    def call(e=p[0], w=p[1], dt=bf, sb=96 * 8, H=2, Lt=8, D=48, beta=p[2], alpha=p[3]):
+        return L.prime_delta_gates(e, sb, 96, w, sb, 96, dt, 0.99, 1, H, Lt, D, beta, alpha, None)
+    assert call(e=None) == -1 and call(Lt=0) == -1 and call(sb=-1) == -1
+    assert call(D=65) == -2 and call(dt=9) == -3
+    assert call(e=ctypes.c_void_p((1 << 24) + 1)) == -4 and call(alpha=ctypes.c_void_p((4 << 24) + 2)) == -4
+    assert call(beta=ctypes.c_void_p((1 << 24) + 64)) == -5 and call(alpha=p[2]) == -5
+
+
 def test_host_wrappers_refuse_cpu_tensors():
     import torch
     x = torch.zeros(1, 1, 64)

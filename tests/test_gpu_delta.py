@@ -295,3 +295,25 @@ def test_delta_module_prefill_then_step_matches_composition():
     ref1, S1 = _module_ref(mod, x[:, 100:], state=S)
     assert_close(to_np(out1), ref1, TOL_BF16, "step out")
     assert_close(to_np(st1).reshape(S1.shape), S1, TOL_BF16, "step state")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,L,D,offset", [(1, 1, 1, 64, 0), (2, 3, 65, 64, 0), (1, 5, 127, 64, 1), (2, 4, 64, 32, 0),
+                                            (1, 2, 130, 7, 0)])
+def test_delta_gates_match_module_ops(dtype, B, H, L, D, offset):
+    """prime_delta_gates against the module's torch ops (sigmoid in the dtype, fp32
+    mean): tile edges in tokens and heads, rows off 16-byte boundaries (offset), other
+    head dims, saturated gates.  bf16 / fp16: a sigmoid may round to its neighbour
+    where it lies within 1e-7 of a tie, one unit (2^-8 or 2^-11) in one of D columns."""
+    g = torch.Generator().manual_seed(B + L)
+    pre = [(torch.randn(B, L, H * D + offset, generator=g) * 3).to(dev(), dtype) for _ in range(2)]
+    pre[0][..., offset] = float("inf")
+    pre[1][:, 0] = -float("inf")
+    erase, write = (t[..., offset:] for t in pre)
+    beta, alpha = _lib.delta_gates(erase, write, 0.9995, H, D)
+    mean = lambda t: torch.sigmoid(t).reshape(B, L, H, D).float().mean(-1).transpose(1, 2)
+    rb, ra = mean(write) * 0.5, 0.9995 * (1.0 - mean(erase) * 0.5)
+    torch.cuda.synchronize()
+    tol = {torch.float32: 2e-7, torch.bfloat16: 2e-7 + 2.0 ** -9 / D, torch.float16: 2e-7 + 2.0 ** -12 / D}[dtype]
+    assert (beta - rb).abs().max().item() <= tol
+    assert (alpha - ra).abs().max().item() <= tol
