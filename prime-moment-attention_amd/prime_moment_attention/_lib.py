@@ -230,10 +230,12 @@ def _check_decay(decay: torch.Tensor, H: int) -> None:
 def _check_state(state, B: int, H: int, D: int, name: str) -> None:
     if state is None:
         return
-    shapes = [(B, H, D), (B, H, D, D), (B, H, D, D), (B, H, 1), (B, H, D), (B, H, D)]
+    shapes = ((B, H, D), (B, H, D, D), (B, H, D, D), (B, H, 1), (B, H, D), (B, H, D))
     if len(state) != 6:
         raise ValueError(f"{name} must be a 6-tuple")
     for t, sh in zip(state, shapes):
+        if t.shape == sh and t.dtype is torch.float32 and t.is_contiguous() and t.is_cuda:
+            continue
         if t.dtype != torch.float32 or not t.is_contiguous() or t.numel() != B * H * _prod(sh[2:]):
             raise ValueError(f"{name}: component of shape {tuple(t.shape)} / {t.dtype} is not a "
                              f"contiguous fp32 {sh}")
@@ -278,7 +280,10 @@ def state_desc(state: Optional[Sequence[torch.Tensor]]) -> Optional[PrimeState]:
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The device's current stream as an integer handle (without building a
+    torch.cuda.Stream: 5 us a call)."""
+    index = dev.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def bind_decode_step(q, k, v, decay: torch.Tensor, eps: float, state_in, state_out, y):
@@ -350,13 +355,16 @@ def qk_norm_on_load(q_norm, k_norm, q_scale: float, q: torch.Tensor) -> Optional
     LayerNorms with different eps (the kernels take one)."""
     if q.dtype != torch.bfloat16:
         return None
-    if q_norm is not None:
-        ps = (q_norm.weight, q_norm.bias, k_norm.weight, k_norm.bias)
-        if any(t is None or t.dtype != q.dtype or not t.is_contiguous() or t.device != q.device for t in ps):
+    if q_norm is None:
+        return qk_norm(None, None, q_scale, q.dtype)
+    ps = (q_norm.weight, q_norm.bias, k_norm.weight, k_norm.bias)
+    dtype, dev = q.dtype, q.device
+    for t in ps:
+        if t is None or t.dtype != dtype or t.device != dev or not t.is_contiguous():
             return None
-        if q_norm.eps != k_norm.eps:
-            return None
-    return qk_norm(q_norm, k_norm, q_scale, q.dtype)
+    if q_norm.eps != k_norm.eps:
+        return None
+    return PrimeQkNorm(*[t.data_ptr() for t in ps], _DTYPES[dtype], float(q_norm.eps), float(q_scale))
 
 
 def decode_step_qknorm(q, k, v, decay: torch.Tensor, eps: float, norm: PrimeQkNorm, state_in, state_out,
@@ -500,6 +508,38 @@ def linear_fused(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, epilogue: 
                                    ctypes.c_void_p(out.data_ptr()), M, N, K, x.stride(0), w.stride(0),
                                    r.stride(0) if r is not None else N, out.stride(0), _DTYPES[torch.bfloat16],
                                    int(epilogue), float(rms_eps), _stream(x.device))
+    _check(rc, "prime_linear_fused")
+    return out
+
+
+# Rows up to which a module's bf16 projection runs prime_linear_fused: up to there it beats
+# the library GEMM on the device (K = 512 .. 1024, N = 512 .. 3072: 2.8-8.2 us against
+# 3.7-9.4, but 4.6 against 4.2 at K = 1024 below 32 rows; at 1024 rows they meet) and the
+# call costs the host 6 us instead of 18.
+ROWS_LINEAR_MAX = 512
+
+
+def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``rows_linear`` takes x [..., K] and w [N, K]: few bf16 rows of the sizes
+    measured, 16-byte rows, plain dense tensors of one device, and nothing recording or
+    recasting (autograd, autocast)."""
+    K = x.shape[-1]
+    return (x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.is_cuda and w.device == x.device
+            and 0 < x.numel() <= ROWS_LINEAR_MAX * K and K % 128 == 0 and K <= 1024 and w.shape[0] % 32 == 0
+            and w.shape[0] <= 3072 and x.is_contiguous() and w.is_contiguous()
+            and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and not torch.is_autocast_enabled())
+
+
+def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T by prime_linear_fused (``rows_linear_ok``): x [..., K] -> [..., N]."""
+    N, K = w.shape
+    M = x.numel() // K
+    out = torch.empty(*x.shape[:-1], N, device=x.device, dtype=x.dtype)
+    rc = load().prime_linear_fused(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), M, N, K, K, K, N, N, PRIME_BF16,
+                                   EPILOGUE_NONE, 0.0, _stream(x.device))
     _check(rc, "prime_linear_fused")
     return out
 
@@ -1142,9 +1182,12 @@ def as_state(state, B: int, H: int, D: int, device) -> Tuple[torch.Tensor, ...]:
     """Validate a reference-layout 6-tuple; return contiguous fp32 tensors."""
     if len(state) != 6:
         raise ValueError("state must be the 6-tuple (S0, S1, S2, K0, K1, K2)")
-    shapes = [(B, H, D), (B, H, D, D), (B, H, D, D), (B, H, 1), (B, H, D), (B, H, D)]
+    shapes = ((B, H, D), (B, H, D, D), (B, H, D, D), (B, H, 1), (B, H, D), (B, H, D))
     out = []
     for t, s in zip(state, shapes):
+        if t.shape == s and t.dtype is torch.float32 and t.device == device and t.is_contiguous():
+            out.append(t)  # as it is
+            continue
         if t.numel() != _prod(s):
             raise ValueError(f"state component has shape {tuple(t.shape)}, expected {s}")
         t = t.to(device=device, dtype=torch.float32)

@@ -48,17 +48,21 @@ def _stacked_qkv(mod: nn.Module) -> Optional[torch.Tensor]:
     ws = tuple(m.weight for m in lins)
     if torch.is_grad_enabled() and any(w.requires_grad for w in ws):
         return None
-    if any(m.bias is not None for m in lins) or len({(w.dtype, w.device) for w in ws}) != 1:
+    q, k, v = ws
+    if (any(m.bias is not None for m in lins) or not q.dtype == k.dtype == v.dtype
+            or not q.device == k.device == v.device):
         return None
     # the cache holds the weight tensors themselves, so their storage
     # cannot be freed and reused by a new weight at the same address
-    key = tuple((w.data_ptr(), w._version) for w in ws)
+    key = (q.data_ptr(), k.data_ptr(), v.data_ptr(), q._version, k._version, v._version)
     cached = mod.__dict__.get("_qkv_cache")
     # (a copy made under inference_mode is rebuilt outside it: autograd could
     # not save an inference tensor for a backward through hidden_states)
-    if (cached is not None and all(a is b for a, b in zip(cached[0], ws)) and cached[1] == key
-            and (not cached[2].is_inference() or torch.is_inference_mode_enabled())):
-        return cached[2]
+    if cached is not None:
+        (cq, ck, cv), ckey, w = cached
+        if (cq is q and ck is k and cv is v and ckey == key
+                and (not w.is_inference() or torch.is_inference_mode_enabled())):
+            return w
     w = torch.cat(ws, 0)
     mod.__dict__["_qkv_cache"] = (ws, key, w)
     return w
@@ -76,10 +80,22 @@ def project_qkv(mod: nn.Module, hidden_states: torch.Tensor):
         return (mod.q_proj(hidden_states).view(B, L, H, D).transpose(1, 2),
                 mod.k_proj(hidden_states).view(B, L, Hk, D).transpose(1, 2),
                 mod.v_proj(hidden_states).view(B, L, Hk, D).transpose(1, 2))
-    qkv = torch.nn.functional.linear(hidden_states, w)
-    return (qkv[..., :H * D].view(B, L, H, D).transpose(1, 2),
-            qkv[..., H * D:(H + Hk) * D].view(B, L, Hk, D).transpose(1, 2),
-            qkv[..., (H + Hk) * D:].view(B, L, Hk, D).transpose(1, 2))
+    linear = _lib.rows_linear if _lib.rows_linear_ok(hidden_states, w) else torch.nn.functional.linear
+    qkv = linear(hidden_states, w).view(B, L, H + 2 * Hk, D).transpose(1, 2)
+    return qkv[:, :H], qkv[:, H:H + Hk], qkv[:, H + Hk:]
+
+
+def _has_hooks(m: nn.Module) -> bool:
+    g = torch.nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks or g._global_forward_pre_hooks)
+
+
+def project_out(proj: nn.Module, y: torch.Tensor) -> torch.Tensor:
+    """``proj(y)``: for few rows through the row kernel, where the module is a plain
+    nn.Linear without bias or hooks."""
+    if type(proj) is nn.Linear and proj.bias is None and not _has_hooks(proj) and _lib.rows_linear_ok(y, proj.weight):
+        return _lib.rows_linear(y, proj.weight)
+    return proj(y)
 
 
 class PrimeMomentAttention(nn.Module):
@@ -169,7 +185,7 @@ class PrimeMomentAttention(nn.Module):
             y = y.to(orig_dtype).transpose(1, 2).reshape(B, L, H * D)
             return self.o_proj(y), (next_state if return_state else None)
         y, next_state = self.mix(hidden_states, state, return_state)
-        return self.o_proj(y), (next_state if return_state else None)
+        return project_out(self.o_proj, y), (next_state if return_state else None)
 
     def mix(self, hidden_states: torch.Tensor, state: Optional[Tuple[torch.Tensor, ...]] = None,
             return_state: bool = False):

@@ -41,7 +41,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
-from .attention import project_qkv
+from .attention import project_out, project_qkv
 from .chunked_ssd import _prep, needs_grad
 
 
@@ -149,7 +149,7 @@ class PrimeSelectiveMomentAttention(nn.Module):
     def forward(self, hidden_states: torch.Tensor, state: Optional[Tuple[torch.Tensor, ...]] = None,
                 return_state: bool = False):
         y, next_state = self.mix(hidden_states, state, return_state)
-        return self.o_proj(y), next_state
+        return project_out(self.o_proj, y), next_state
 
     def mix(self, hidden_states: torch.Tensor, state: Optional[Tuple[torch.Tensor, ...]] = None,
             return_state: bool = False):

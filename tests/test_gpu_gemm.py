@@ -349,3 +349,39 @@ def test_linear_frag_rejects_bad_arguments():
         _lib.linear_frag(x, w, 32, 64, 256, x, flags=_lib.LINEAR_OUT_FRAG)
     with pytest.raises(RuntimeError, match="workspace"):
         _lib.linear_frag(x, w, 32, 64, 256, y, tokens=torch.zeros(32, device=dev(), dtype=torch.int64))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 128, 32), (33, 768, 2304), (400, 768, 768), (512, 1024, 3072)])
+def test_rows_linear_matches_fp32_and_its_rule(M, K, N):
+    """The modules' few-row projection: one rounding of the fp32 product (2^-9, and the
+    sums' order), and the calls it leaves to torch."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(2, M // 2, K, generator=g).to(dev(), torch.bfloat16) if M % 2 == 0 else \
+        torch.randn(M, 1, K, generator=g).to(dev(), torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) / K ** 0.5).to(dev(), torch.bfloat16)
+    assert _lib.rows_linear_ok(x, w)
+    y = _lib.rows_linear(x, w)
+    ref = x.float() @ w.float().t()
+    assert y.shape == ref.shape and ((y.float() - ref).abs() <= ref.abs() * 2 ** -8 + 1e-3).all()
+    big = torch.zeros(513, K, device=dev(), dtype=torch.bfloat16)
+    assert not _lib.rows_linear_ok(big, w) and not _lib.rows_linear_ok(x.float(), w)
+    assert not _lib.rows_linear_ok(x[..., :64], w[:, :64].contiguous())
+    assert not _lib.rows_linear_ok(x, w.clone().requires_grad_())
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not _lib.rows_linear_ok(x, w)
+
+
+def test_module_output_projection_keeps_hooks_and_replacements():
+    """A hooked or replaced o_proj runs as the module it is."""
+    from prime_moment_attention import PrimeMomentAttention
+    m = PrimeMomentAttention(128, 2, 64).to(dev(), torch.bfloat16)
+    x = torch.randn(1, 8, 128, device=dev(), dtype=torch.bfloat16)
+    with torch.no_grad():
+        y, _ = m(x)
+        seen = []
+        h = m.o_proj.register_forward_hook(lambda mod, i, o: seen.append(o))
+        y2, _ = m(x)
+        h.remove()
+        assert len(seen) == 1 and torch.allclose(y.float(), y2.float(), atol=2 ** -7)
+        m.o_proj = torch.nn.Sequential(m.o_proj, torch.nn.ReLU())
+        assert (m(x)[0] >= 0).all()
