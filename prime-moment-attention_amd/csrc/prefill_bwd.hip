@@ -15,7 +15,14 @@
 //   dM_in = l R_0   (the adjoint of the incoming state),
 // and dq = dphi_q[q] + 2 q * dphi_q[q*q], dk = dphi_k[k] + k * dphi_k[k*k/2].
 //
-// Two kernels, one workgroup (4 waves) per sequence, 64-token chunks:
+// Two kernels, one workgroup of eight waves per sequence, 64-token chunks: four
+// readout waves (16 tokens each) form a chunk's gradients while four update waves
+// advance the carried state and prepare the next chunk's tiles; between two
+// barriers the update waves write both to LDS (80 KB and 128 registers, so two
+// workgroups share a CU).  Both passes are bound by the readout waves' chain of
+// dependent products and its LDS traffic, not by HBM: 384 sequences of 2048 tokens
+// take 430 us for 1.1 GB (572 with four waves that did everything in turn and
+// waited for each prefetched row where it was loaded); 768 of 256, 97 (139).
 //
 //  * dq pass (chunks in order).  The forward chunk loop again -- the value
 //    columns of M carried in MFMA accumulators, a bf16 copy of them in LDS for
@@ -51,24 +58,23 @@ constexpr int kSR = kD + 1;    // rows of a transposed state copy: 64 value colu
 
 __device__ __forceinline__ void st16(uint16_t *p, u32x4 x) { *reinterpret_cast<u32x4 *>(p) = x; }
 
-// 8 consecutive elements of a row of dtype dt, as packed bf16 (round to nearest even)
-__device__ __forceinline__ u32x4 load_packed(const void *base, int64_t off, int dt) {
-    if (dt == PRIME_BF16) return *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(base) + off);
+// 8 consecutive elements of a row of dtype dt as loaded (16 bytes, or two times
+// 16 for fp32), as packed bf16 (round to nearest even)
+__device__ __forceinline__ u32x4 pack_raw(const u32x4 (&x)[2], int dt) {
+    if (dt == PRIME_BF16) return x[0];
     float f[8];
     if (dt == PRIME_F32) {
-        const f32x4 a = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + off);
-        const f32x4 b = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(base) + off + 4);
+        const f32x4 lo = __builtin_bit_cast(f32x4, x[0]), hi = __builtin_bit_cast(f32x4, x[1]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            f[i] = a[i];
-            f[4 + i] = b[i];
+            f[i] = lo[i];
+            f[4 + i] = hi[i];
         }
     } else {
-        const u32x4 r = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(base) + off);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            f[2 * i] = h16_bits_to_f32(static_cast<uint16_t>(r[i] & 0xFFFFu));
-            f[2 * i + 1] = h16_bits_to_f32(static_cast<uint16_t>(r[i] >> 16));
+            f[2 * i] = h16_bits_to_f32(static_cast<uint16_t>(x[0][i] & 0xFFFFu));
+            f[2 * i + 1] = h16_bits_to_f32(static_cast<uint16_t>(x[0][i] >> 16));
         }
     }
     return pack8(f);
@@ -122,74 +128,151 @@ __device__ __forceinline__ bf16x8 scale_op(bf16x8 x, const float (&wt)[8]) {
     return as_bf16x8(pack8(f));
 }
 
-// v[r][fb] to base[o[r] + 16 fb + c16] for the rows with ok[r], in dtype dt
-// (one wave-uniform dtype branch around all 16 stores)
-__device__ __forceinline__ void store_rows4(void *base, int dt, const int64_t (&o)[4], const bool (&ok)[4], int c16,
-                                            const float (&v)[4][4]) {
+// v[fb][r] to base[o + 16 fb + r] (o includes the lane's 4g), in dtype dt: one
+// 16- or 8-byte store per block where the rows allow it (vec)
+__device__ __forceinline__ void store_row16(void *base, int dt, bool vec, int64_t o, const f32x4 (&v)[4]) {
     if (dt == PRIME_F32) {
-        float *p = static_cast<float *>(base) + c16;
+        float *p = static_cast<float *>(base) + o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (ok[r])
+        for (int fb = 0; fb < 4; ++fb) {
+            if (vec) {
+                *reinterpret_cast<f32x4 *>(p + 16 * fb) = v[fb];
+            } else {
 #pragma unroll
-                for (int fb = 0; fb < 4; ++fb) p[o[r] + 16 * fb] = v[r][fb];
+                for (int r = 0; r < 4; ++r) p[16 * fb + r] = v[fb][r];
+            }
+        }
     } else {
-        uint16_t *p = static_cast<uint16_t *>(base) + c16;
-        const bool bf = dt == PRIME_BF16;
+        uint16_t *p = static_cast<uint16_t *>(base) + o;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (ok[r])
+        for (int fb = 0; fb < 4; ++fb) {
+            uint2 x;
+            if (dt == PRIME_BF16) {
+                x = uint2{pack2(v[fb][0], v[fb][1]), pack2(v[fb][2], v[fb][3])};
+            } else {
+                uint32_t hb[4];
 #pragma unroll
-                for (int fb = 0; fb < 4; ++fb)
-                    p[o[r] + 16 * fb] = bf ? f32_to_bf16_bits(v[r][fb]) : f32_to_h16_bits(v[r][fb]);
+                for (int r = 0; r < 4; ++r) hb[r] = f32_to_h16_bits(v[fb][r]);
+                x = uint2{hb[0] | hb[1] << 16, hb[2] | hb[3] << 16};
+            }
+            if (vec) {
+                *reinterpret_cast<uint2 *>(p + 16 * fb) = x;
+            } else {
+                p[16 * fb] = static_cast<uint16_t>(x.x);
+                p[16 * fb + 1] = static_cast<uint16_t>(x.x >> 16);
+                p[16 * fb + 2] = static_cast<uint16_t>(x.y);
+                p[16 * fb + 3] = static_cast<uint16_t>(x.y >> 16);
+            }
+        }
     }
 }
 
-// One chunk's inputs for one thread: rows ra and ra + 32, columns col..col+7.
+// four consecutive packed bf16 at p (8-byte aligned)
+__device__ __forceinline__ f32x4 unpack4(const uint16_t *p) {
+    const uint2 x = *reinterpret_cast<const uint2 *>(p);
+    return f32x4{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xFFFF0000u), __uint_as_float(x.y << 16),
+                 __uint_as_float(x.y & 0xFFFF0000u)};
+}
+
+// an operand row with the tr_op K permutation, as it lies in LDS
+__device__ __forceinline__ bf16x8 perm_row(const uint16_t *row, int ks, int g) {
+    const uint2 a = *reinterpret_cast<const uint2 *>(row + 32 * ks + 4 * g);
+    const uint2 b = *reinterpret_cast<const uint2 *>(row + 32 * ks + 16 + 4 * g);
+    return as_bf16x8(u32x4{a.x, a.y, b.x, b.y});
+}
+
+// Keeps a value's computation before this point (an update wave prepares the next
+// tiles before the barrier that the readout waves are still on their way to).
+__device__ __forceinline__ void settle(u32x4 &x) { asm volatile("" : "+v"(x)); }
+
+// Orders a wave's LDS writes before its own later LDS reads by other lanes.
+__device__ __forceinline__ void lds_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// An index the compiler cannot trace: addresses formed from it are formed where
+// they are used instead of being kept in registers over the whole chunk loop.
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// One chunk's inputs for one update thread: rows ra and ra + 32, columns
+// col..col+7, as they lie in memory (q, k, v are bf16 here; dy of any dtype).
+// Nothing may touch the results before they are needed, or the wave waits out
+// the latency where the load is issued.  q, k and v are loaded a chunk ahead; dy
+// and its two per-token numbers only once the state update is done (the readout
+// waves take longer), so that the loads in flight and the state fit 128 registers.
 struct Rows {
-    u32x4 q[2], k[2], v[2], dy[2];  // packed bf16
+    u32x4 q[2], k[2], v[2], dy[2][2];
     float inv[2], gden[2];
 };
 
-__device__ __forceinline__ void load_rows(Rows &R, const BwdArgs &a, int b, int h, int c, int ra, int col,
-                                          bool want_q, bool want_kv, bool want_g) {
+template <bool KV>
+__device__ __forceinline__ void load_qkv(Rows &R, const BwdArgs &a, int b, int h, int c, int ra, int col) {
+    const int64_t t0 = static_cast<int64_t>(c) * kC;
+    const int last = min(kC, a.L - c * kC) - 1;
+    const uint16_t *q = static_cast<const uint16_t *>(a.q) + b * a.q_sb + h * a.q_sh + t0 * a.q_sl;
+    const uint16_t *k = static_cast<const uint16_t *>(a.k) + b * a.k_sb + h * a.k_sh + t0 * a.k_sl;
+    const uint16_t *v = static_cast<const uint16_t *>(a.v) + b * a.v_sb + h * a.v_sh + t0 * a.v_sl;
+    ra = opaque(ra);  // scalar bases plus a lane offset formed here
+    col = opaque(col);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-        const int64_t t = min(c * kC + ra + 32 * s, a.L - 1);  // clamped; rows past L are zeroed when stored
-        if (want_q) R.q[s] = load_packed(a.q, b * a.q_sb + h * a.q_sh + t * a.q_sl + col, a.dt_in);
-        if (want_kv) {
-            R.k[s] = load_packed(a.k, b * a.k_sb + h * a.k_sh + t * a.k_sl + col, a.dt_in);
-            R.v[s] = load_packed(a.v, b * a.v_sb + h * a.v_sh + t * a.v_sl + col, a.dt_in);
-        }
-        R.dy[s] = load_packed(a.dy, b * a.dy_sb + h * a.dy_sh + t * a.dy_sl + col, a.dt_dy);
-        if (want_g) {
-            const size_t o = static_cast<size_t>(b * a.H + h) * a.L + t;
-            R.inv[s] = a.inv_den[o];
-            R.gden[s] = a.g_den[o];
+        const int64_t t = min(ra + 32 * s, last);  // clamped; rows past L are zeroed when prepared
+        R.q[s] = *reinterpret_cast<const u32x4 *>(q + t * a.q_sl + col);
+        if constexpr (KV) {
+            R.k[s] = *reinterpret_cast<const u32x4 *>(k + t * a.k_sl + col);
+            R.v[s] = *reinterpret_cast<const u32x4 *>(v + t * a.v_sl + col);
         }
     }
 }
 
+template <bool DEN>
+__device__ __forceinline__ void load_dy(Rows &R, const BwdArgs &a, int b, int h, int c, int ra, int col) {
+    const int64_t t0 = static_cast<int64_t>(c) * kC;
+    const int last = min(kC, a.L - c * kC) - 1;
+    const int es = a.dt_dy == PRIME_F32 ? 4 : 2, step = a.dt_dy == PRIME_F32 ? 16 : 0;
+    const char *dy = static_cast<const char *>(a.dy) + es * (b * a.dy_sb + h * a.dy_sh + t0 * a.dy_sl);
+    const size_t o = static_cast<size_t>(b * a.H + h) * a.L + t0;
+    ra = opaque(ra);
+    col = opaque(col);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int64_t t = min(ra + 32 * s, last);
+        const char *p = dy + es * (t * a.dy_sl + col);
+        R.dy[s][0] = *reinterpret_cast<const u32x4 *>(p);
+        R.dy[s][1] = *reinterpret_cast<const u32x4 *>(p + step);
+        if constexpr (DEN) {
+            R.inv[s] = a.inv_den[o + t];
+            R.gden[s] = a.g_den[o + t];
+        }
+    }
+}
 
 }  // namespace
 
 // ---------------------------------------------------------------- dq pass
 // DIN: the dense double clamp with an incoming state (BwdArgs::dense_in)
 template <bool DIN>
-__global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(512, DIN ? 2 : 4) void prefill_bwd_dq_kernel(const BwdArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t sQf[kC][kPT];   // [q | q*q]
     __shared__ __attribute__((aligned(16))) uint16_t sKf[kC][kPT];   // [k | k*k/2]
-    __shared__ __attribute__((aligned(16))) uint16_t sV[kC][kPV];    // [v | 0..]
-    __shared__ __attribute__((aligned(16))) uint16_t sG[kC][kPV];    // dy, overwritten by the value part of G (dy / d)
+    __shared__ __attribute__((aligned(16))) uint16_t sV[kC][kPV];    // v
+    __shared__ __attribute__((aligned(16))) uint16_t sG[kC][kPV];    // dy
     __shared__ __attribute__((aligned(16))) uint16_t sSt[kD][kPT];   // bf16 value columns of M^T entering the chunk
     // fp32: the K column of M (the denominator's moments) entering the chunk, S0, K0
-    __shared__ float sKv[kF], sS0[kD], sK0[1], sGd[kC], sPg[kC], sPw[kC + 2], sPs[kC + 2];
-    __shared__ float sRedK[kF], sRedS[kD];  // the chunk's K and S0 increments
+    __shared__ __attribute__((aligned(16))) float sKv[kF], sS0[kD];
+    __shared__ float sK0[1], sPw[kC + 2], sPs[kC + 2];
+    __shared__ float sRedK[kF];  // the chunk's K increment (written and read by the same update wave)
     // dense double clamp with an incoming state: the incoming [K1; K2/2] and K0
     // (the carried K above is then the call's own), and per token of the chunk
-    // l^(t+1) times the outer-clamp denominator adjoint (sPc) and times the part
-    // of it the inner clamp withholds from the call's tokens (sDh)
-    __shared__ float sKin[kF], sK0in[1], sPc[kC], sDh[kC];
+    // l^(t+1) times the part of the outer-clamp denominator adjoint that the
+    // inner clamp withholds from the call's tokens (sDh)
+    __shared__ __attribute__((aligned(16))) float sKin[kF];
+    __shared__ float sK0in[1], sDh[kC];
     // the state-update weights l^(n-1-j) of a full chunk (0) and of the
     // sequence's last chunk (1, n = its valid tokens), and the same weights split
     // into three bf16 parts (hi, mid, lo: about fp32 precision in sum), row 3
@@ -198,7 +281,9 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
     __shared__ __attribute__((aligned(16))) uint16_t sWp[2][4][kC];
 
     const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const bool is_u = wave >= 4;                // update role
+    const int w = wave & 3, ut = tid & 255;     // wave and thread index within the role
     const int g = lane >> 4, c16 = lane & 15;
     const int tr_r = c16 >> 2, tr_c = 4 * (c16 & 3);
     const int unit = blockIdx.x;
@@ -230,67 +315,6 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
         sPs[tid] = static_cast<float>(ps);
     }
     constexpr bool din = DIN;  // (then G == 1: the S*p are state_in)
-    if (tid < kD) sS0[tid] = S0p ? S0p[tid] : 0.f;
-    if (tid == 0) {
-        sK0[0] = K0p && !din ? K0p[0] : 0.f;
-        sK0in[0] = K0p && din ? K0p[0] : 0.f;
-    }
-    // the denominator's moments [K1; K2/2] in fp32, one feature per thread (tid < 128)
-    float kv = 0.f;
-    if (tid < kF && K1p) kv = tid < kD ? K1p[tid] : 0.5f * K2p[tid - kD];
-    if (din) {
-        if (tid < kF) sKin[tid] = kv;
-        kv = 0.f;
-    }
-    float corr = 0.f;  // (din) this thread's feature (tid < 128) or K0 (tid == 128) of the correction
-    // constant columns of the 80-wide tiles
-    for (int idx = tid; idx < kC * 16; idx += 256) {
-        const int row = idx >> 4, cc = kD + (idx & 15);
-        sV[row][cc] = 0u;
-        sG[row][cc] = 0u;
-    }
-
-
-
-    // value columns of M (features 32w..32w+31 of this wave, value blocks 0..3) from state_in
-    f32x4 st[2][4];
-#pragma unroll
-    for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
-                const float x = S1p ? (f < kD ? S1p : S2p)[fr * kD + n] : 0.f;
-                st[fi][nb][r] = f < kD ? x : 0.5f * x;
-            }
-    auto publish = [&]() {
-#pragma unroll
-        for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                *reinterpret_cast<uint2 *>(&sSt[16 * nb + c16][16 * (2 * w + fi) + 4 * g]) =
-                    uint2{pack2(st[fi][nb][0], st[fi][nb][1]), pack2(st[fi][nb][2], st[fi][nb][3])};
-        if (tid < kF) sKv[tid] = kv;
-    };
-
-    const int ra = tid >> 3, col = 8 * (tid & 7);
-    Rows R;
-    auto store_rows = [&](int c) {
-        const int nv = min(kC, a.L - c * kC);
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int row = ra + 32 * s;
-            const uint32_t m = row < nv ? 0xFFFFFFFFu : 0u;
-            const u32x4 q = and4(R.q[s], m), k = and4(R.k[s], m);
-            st16(&sQf[row][col], q);
-            st16(&sQf[row][kD + col], sq8(q, 1.f));
-            st16(&sKf[row][col], k);
-            st16(&sKf[row][kD + col], sq8(k, 0.5f));
-            st16(&sV[row][col], and4(R.v[s], m));
-            st16(&sG[row][col], and4(R.dy[s], m));
-        }
-    };
 
     __syncthreads();  // power tables
     if (tid < 2 * kC) {  // the two weight tables (read after the chunk loop's first barrier)
@@ -306,9 +330,199 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
         sWp[which][2][t] = f32_to_bf16_bits(r1 - bf16_bits_to_f32(mid));
         sWp[which][3][t] = 0u;
     }
-    // readout constants of this lane: row iw of the transposed blocks, rows
-    // 16w + 4g + r of the [num | den] accumulators (powers from the table:
-    // sPw[n] is l^n rounded from fp64)
+    if (is_u) {
+        // ================ update role: the carried state and the tiles
+        // value columns of M (features 32w..32w+31 of this wave, value blocks 0..3) from state_in
+        f32x4 st[2][4];
+        // the denominator's moments [K1; K2/2] in fp32, feature 32w + lane (lane < 32);
+        // S0 of value column 16w + c16 (lane group 0); K0
+        float kv = 0.f, s0 = 0.f, k0 = 0.f;
+#pragma unroll
+        for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) st[fi][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (S1p) {
+            const float *Sp = w < 2 ? S1p : S2p, *Kp = w < 2 ? K1p : K2p;  // waves 0, 1 hold features 0..63
+            const float sc = w < 2 ? 1.0f : 0.5f;
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int fr = (16 * (2 * w + fi) + 4 * g + r) & (kD - 1);
+                        st[fi][nb][r] = Sp[fr * kD + 16 * nb + c16];
+                    }
+            kv = sc * Kp[(32 * w + (lane & 31)) & (kD - 1)];
+            s0 = S0p[16 * w + c16];
+            k0 = K0p[0];
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) st[fi][nb] *= sc;
+        }
+        if (din) {
+            if (lane < 32) sKin[32 * w + lane] = kv;
+            if (ut == 0) sK0in[0] = k0;
+            kv = k0 = 0.f;
+        }
+        float corr = 0.f;  // (din) this thread's feature (ut < 128) or K0 (ut == 128) of the correction
+        const int ra = ut >> 3, col = 8 * (ut & 7);
+        Rows R;
+        u32x4 q2[2], k2[2], gr[2];  // squares, and dy as bf16
+        auto prepare = [&](int c) {
+            const int nv = min(kC, a.L - c * kC);
+            load_dy<false>(R, a, b, h, c, ra, col);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if (nv < kC) {
+                    const uint32_t m = ra + 32 * s < nv ? 0xFFFFFFFFu : 0u;
+                    R.q[s] = and4(R.q[s], m);
+                    R.k[s] = and4(R.k[s], m);
+                    R.v[s] = and4(R.v[s], m);
+                }
+                q2[s] = sq8(R.q[s], 1.f);
+                k2[s] = sq8(R.k[s], 0.5f);
+                settle(q2[s]);
+                settle(k2[s]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                gr[s] = pack_raw(R.dy[s], a.dt_dy);
+                if (nv < kC) gr[s] = and4(gr[s], ra + 32 * s < nv ? 0xFFFFFFFFu : 0u);
+                settle(gr[s]);
+            }
+        };
+        auto publish = [&]() {  // the prepared tiles and the state entering their chunk
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int row = ra + 32 * s;
+                st16(&sQf[row][col], R.q[s]);
+                st16(&sQf[row][kD + col], q2[s]);
+                st16(&sKf[row][col], R.k[s]);
+                st16(&sKf[row][kD + col], k2[s]);
+                st16(&sV[row][col], R.v[s]);
+                st16(&sG[row][col], gr[s]);
+            }
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb)
+                    *reinterpret_cast<uint2 *>(&sSt[16 * nb + c16][16 * (2 * w + fi) + 4 * g]) =
+                        uint2{pack2(st[fi][nb][0], st[fi][nb][1]), pack2(st[fi][nb][2], st[fi][nb][3])};
+            if (lane < 32) sKv[32 * w + lane] = kv;
+            if (g == 0) sS0[16 * w + c16] = s0;
+            if (ut == 0) sK0[0] = k0;
+        };
+        load_qkv<true>(R, a, b, h, c_begin, ra, col);
+        prepare(c_begin);
+        publish();
+        if (c_begin + 1 < c_end) load_qkv<true>(R, a, b, h, c_begin + 1, ra, col);
+        for (int c = c_begin; c < c_end; ++c) {
+            const int nvalid = min(kC, a.L - c * kC);
+            const int wsel = nvalid == kC ? 0 : 1;  // weights of a full chunk or of the last one
+            __syncthreads();  // tiles of chunk c and M_c in LDS
+            if (c + 1 < c_end) {
+                // ---- M <- l^n M + (w phi_k)^T v with w_j = l^(n-1-j) on the A operand's
+                // token slots; S0 and K = [K1; K2/2] (fp32) as partial sums over all threads
+                const float ln = sPw[nvalid];
+#pragma unroll
+                for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) st[fi][nb][r] *= ln;
+                // K and S0 increments on MFMA, against the three parts of w (fp32-accurate
+                // sums: K decides the clamp): dk[fi] rows = features, columns 0..2 = parts;
+                // ds0 rows 0..2 = parts, columns = value block w
+                f32x4 dk[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+                f32x4 ds0 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    float wt[8];
+                    {
+                        const f32x4 w0 = *reinterpret_cast<const f32x4 *>(&sWt[wsel][32 * ks + 4 * g]);
+                        const f32x4 w1 = *reinterpret_cast<const f32x4 *>(&sWt[wsel][32 * ks + 16 + 4 * g]);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            wt[t] = w0[t];
+                            wt[4 + t] = w1[t];
+                        }
+                    }
+                    // lane (g, c16): part min(c16, 3) of w at its eight token slots, the
+                    // same slots as the transposed operands (token 32ks + 16(t/4) + 4g + t%4)
+                    const int pr = min(c16, 3);
+                    const uint2 p0 = *reinterpret_cast<const uint2 *>(&sWp[wsel][pr][32 * ks + 4 * g]);
+                    const uint2 p1 = *reinterpret_cast<const uint2 *>(&sWp[wsel][pr][32 * ks + 16 + 4 * g]);
+                    const bf16x8 wpart = as_bf16x8(u32x4{p0.x, p0.y, p1.x, p1.y});
+                    bf16x8 ak[2];
+#pragma unroll
+                    for (int fi = 0; fi < 2; ++fi) {
+                        const uint16_t *pk = &sKf[32 * ks + 4 * g + tr_r][16 * (2 * w + fi) + tr_c];
+                        const bf16x8 raw = tr_op<false>(pk, pk + 16 * kPT, 0).h;
+                        dk[fi] = mfma(raw, wpart, dk[fi]);
+                        ak[fi] = scale_op(raw, wt);
+                    }
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb) {
+                        const uint16_t *p0v = &sV[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
+                        const bf16x8 vb = tr_op<false>(p0v, p0v + 16 * kPV, 0).h;
+#pragma unroll
+                        for (int fi = 0; fi < 2; ++fi) st[fi][nb] = mfma(ak[fi], vb, st[fi][nb]);
+                        if (nb == w) ds0 = mfma(wpart, vb, ds0);  // wave-uniform
+                    }
+                }
+                {
+                    // K increment of features 16(2w + fi) + 4g + r: the quad (columns 0..3) sum
+#pragma unroll
+                    for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float x = dk[fi][r];
+                            x += xor_lane<1>(x);
+                            x += xor_lane<2>(x);
+                            if (c16 == 0) sRedK[16 * (2 * w + fi) + 4 * g + r] = x;
+                        }
+                    // S0 of value column 16w + c16: rows 0..2 of the increment (lane group g = 0)
+                    s0 = ln * s0 + ((ds0[0] + ds0[1]) + ds0[2]);
+                    k0 = ln * k0 + sPs[nvalid];
+                    lds_wave_sync();
+                    if (lane < 32) kv = ln * kv + sRedK[32 * w + lane];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                prepare(c + 1);
+            }
+            __syncthreads();  // every read of chunk c's tiles and of M_c is done
+            if (din) {  // correction: sum over the chunk of sDh_t phi_q(t) (chunk c's tiles are still in LDS)
+                if (ut < kF) {
+                    float sacc = 0.f;
+                    for (int i = 0; i < nvalid; ++i) sacc += sDh[i] * bf16_bits_to_f32(sQf[i][ut]);
+                    corr += sacc;
+                } else if (ut == kF) {
+                    float sacc = 0.f;
+                    for (int i = 0; i < nvalid; ++i) sacc += sDh[i];
+                    corr += sacc;
+                }
+                __syncthreads();  // before the tiles change
+            }
+            if (c + 1 < c_end) {
+                publish();
+                __builtin_amdgcn_sched_barrier(0);
+                if (c + 2 < c_end) load_qkv<true>(R, a, b, h, c + 2, ra, col);
+            }
+        }
+        if (din && ut <= kF) a.kcorr[static_cast<size_t>(seq) * kBwdCorr + ut] = corr;
+        return;
+    }
+
+    // ================ readout role: dq of rows 16w..16w+15 of every chunk
+    // Every product is formed transposed (tokens on the columns), so a lane holds
+    // one token, iw, and four consecutive columns of each 16-wide block: G becomes
+    // an operand in registers, per-token factors are lane scalars, and rows are
+    // stored 8 or 16 bytes at a time.  (powers from the table: sPw[n] is l^n
+    // rounded from fp64)
     const int iw = 16 * w + c16;
     float mask[4][4];
 #pragma unroll
@@ -319,20 +533,11 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
             mask[jb][r] = (jb <= w && d >= 0) ? sPw[max(d, 0)] : 0.f;
         }
     const float pinc = sPw[iw + 1];
-    float pinr[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) pinr[r] = sPw[16 * w + 4 * g + r + 1];
-    load_rows(R, a, b, h, c_begin, ra, col, true, true, false);
-    store_rows(c_begin);
-    publish();
-    if (c_begin + 1 < c_end) load_rows(R, a, b, h, c_begin + 1, ra, col, true, true, false);
-
     for (int c = c_begin; c < c_end; ++c) {
         const int nvalid = min(kC, a.L - c * kC);
         // (din) l^(64 c): the incoming state's decay to the chunk's start
         const float lc = din ? static_cast<float>(pow(static_cast<double>(lam), 64.0 * c)) : 0.f;
         __syncthreads();  // tiles of chunk c and M_c in LDS
-        const int wsel = nvalid == kC ? 0 : 1;  // weights of a full chunk or of the last one
         // ---- scores S^T[j][iw] (blocks jb <= w), masked: A = l^(i-j) (1 + phi_q . phi_k)
         f32x4 sT[4];
 #pragma unroll
@@ -346,7 +551,7 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) sT[jb][r] = mask[jb][r] * (1.0f + sT[jb][r]);
         }
-        // ---- numerator rows 16w + 4g + r: A V + pin (phi_q M + S0)
+        // ---- numerator of row iw, columns 16nb + 4g + r: A V + pin (phi_q M + S0)
         f32x4 acc[4], accC[4];
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) acc[nb] = accC[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -357,7 +562,7 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb) {
                 const uint16_t *p0 = &sV[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
-                acc[nb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPV, 0).h, acc[nb]);
+                acc[nb] = mfma(tr_op<false>(p0, p0 + 16 * kPV, 0).h, A, acc[nb]);
             }
         }
 #pragma unroll
@@ -365,13 +570,13 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
             const bf16x8 Aq = as_bf16x8(lds128(&sQf[iw][32 * ks + 8 * g]));
 #pragma unroll
             for (int nb = 0; nb < 4; ++nb)
-                accC[nb] = mfma(Aq, as_bf16x8(lds128(&sSt[16 * nb + c16][32 * ks + 8 * g])), accC[nb]);
+                accC[nb] = mfma(as_bf16x8(lds128(&sSt[16 * nb + c16][32 * ks + 8 * g])), Aq, accC[nb]);
         }
 #pragma unroll
         for (int nb = 0; nb < 4; ++nb) {
-            const float m0 = sS0[16 * nb + c16];
+            const f32x4 m0 = *reinterpret_cast<const f32x4 *>(&sS0[16 * nb + 4 * g]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[nb][r] += pinr[r] * (accC[nb][r] + m0);
+            for (int r = 0; r < 4; ++r) acc[nb][r] += pinc * (accC[nb][r] + m0[r]);
         }
         // ---- denominator of row iw in fp32 (whether the clamp is active decides
         // the gradient): row sum of the masked scores + pin (phi_q . K + K0)
@@ -393,74 +598,43 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
         }
         dsum = sum_lane32(sum_lane16(dsum));
         dcar = sum_lane32(sum_lane16(dcar));
-        const float den_iw = dsum + pinc * (dcar + sK0[0]);
-        // (din) the incoming state's denominator term l^(t+1) (K0 + phi_q . K), outside the inner clamp
-        const float cr_iw = din ? lc * pinc * (sum_lane32(sum_lane16(dcin)) + sK0in[0]) : 0.f;
-        // ---- G of rows i = 16w + 4g + r; dy of those rows at column 16nb + c16
-        // from transposed reads (dyt[nb] element r: row 16w + 4g + r)
-        uint2 dyt[4];
+        const float den = dsum + pinc * (dcar + sK0[0]);
+        // single clamp max(den, eps), or (din) the double clamp max(max(den, eps) + cr, eps) with the
+        // incoming state's denominator term cr = l^(t+1) (K0 + phi_q . K) outside the inner clamp
+        const float d1 =
+            din ? fmaxf(den, a.eps) + lc * pinc * (sum_lane32(sum_lane16(dcin)) + sK0in[0]) : den;
+        const float inv = 1.0f / fmaxf(d1, a.eps);
+        // ---- G of row iw, columns 16nb + 4g + r; gop: its bf16 values as an operand in the tr_op K order
+        const bool valid = iw < nvalid;
+        float part = 0.f;
+        f32x4 gn[4];
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) dyt[nb] = lds_tr(&sG[16 * w + 4 * g + tr_r][16 * nb + tr_c]);
+        for (int nb = 0; nb < 4; ++nb) {
+            const f32x4 dyv = unpack4(&sG[iw][16 * nb + 4 * g]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = 16 * w + 4 * g + r;
-            const bool valid = i < nvalid;
-            const float den = __shfl(den_iw, 4 * g + r, kWave);  // row i's denominator sits in lane c16 = 4g + r
-            // single clamp max(den, eps), or the double clamp max(max(den, eps) + cr, eps)
-            const float d1 = din ? fmaxf(den, a.eps) + __shfl(cr_iw, 4 * g + r, kWave) : den;
-            const float d = fmaxf(d1, a.eps);
-            const float inv = 1.0f / d;
-            float part = 0.f, gn[4];
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const uint32_t dw = r < 2 ? dyt[nb].x : dyt[nb].y;  // overwritten below by this lane
-                const float dyv = __uint_as_float((r & 1) ? dw & 0xFFFF0000u : dw << 16);
-                part += dyv * (acc[nb][r] * inv);
-                gn[nb] = valid ? dyv * inv : 0.f;
-            }
-            part += xor_lane<1>(part);
-            part += xor_lane<2>(part);
-            part += xor_lane<4>(part);
-            part += xor_lane<8>(part);
-            // the outer clamp's adjoint, and the call's share of it (inner clamp)
-            const float gout = (valid && d1 >= a.eps) ? -part * inv : 0.f;
-            const float gden = den >= a.eps ? gout : 0.f;
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) sG[i][16 * nb + c16] = f32_to_bf16_bits(gn[nb]);
-            if (c16 == 0) {
-                sGd[i] = gden;
-                sPg[i] = pinr[r] * gden;
-                if (din) {
-                    sPc[i] = lc * pinr[r] * gout;
-                    sDh[i] = lc * pinr[r] * (gout - gden);
-                }
-                if (valid) {
-                    const size_t o = static_cast<size_t>(seq) * a.L + c * kC + i;
-                    a.inv_den[o] = inv;
-                    a.g_den[o] = gden;
-                }
+            for (int r = 0; r < 4; ++r) {
+                part += dyv[r] * (acc[nb][r] * inv);
+                gn[nb][r] = valid ? dyv[r] * inv : 0.f;
             }
         }
-        // G of the chunk in LDS: each wave reads back only its own rows of sG, sGd
-        // and sPg below, so a wave-local ordering suffices
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // ---- P^T[j][iw] = mask * (v_j . g_iw + gden_iw)
+        part = sum_lane32(sum_lane16(part));
+        // the outer clamp's adjoint, and the call's share of it (inner clamp)
+        const float gout = (valid && d1 >= a.eps) ? -part * inv : 0.f;
+        const float gden = den >= a.eps ? gout : 0.f;
+        if (din && g == 0) sDh[iw] = lc * pinc * (gout - gden);
+        const bf16x8 gop[2] = {acc_op(gn[0], gn[1]), acc_op(gn[2], gn[3])};
+        // ---- P^T[j][iw] = mask * (v_j . g_iw + gden)
         f32x4 pT[4];
-        const float gdi = sGd[iw];
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb) {
             pT[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
             if (jb > w) continue;
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                pT[jb] = mfma(as_bf16x8(lds128(&sV[16 * jb + c16][32 * ks + 8 * g])),
-                              as_bf16x8(lds128(&sG[iw][32 * ks + 8 * g])), pT[jb]);
+            for (int ks = 0; ks < 2; ++ks) pT[jb] = mfma(perm_row(&sV[16 * jb + c16][0], ks, g), gop[ks], pT[jb]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pT[jb][r] = mask[jb][r] * (pT[jb][r] + gdi);
+            for (int r = 0; r < 4; ++r) pT[jb][r] = mask[jb][r] * (pT[jb][r] + gden);
         }
-        // ---- dphi_q rows 16w + 4g + r, features 16fb + c16: P phi_k + pin G M^T
+        // ---- dphi_q of row iw, features 16fb + 4g + r: P phi_k + pin G M^T
         f32x4 dphi[8];
 #pragma unroll
         for (int fb = 0; fb < 8; ++fb) dphi[fb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -471,162 +645,70 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dq_kernel(const BwdArgs a)
 #pragma unroll
             for (int fb = 0; fb < 8; ++fb) {
                 const uint16_t *p0 = &sKf[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
-                dphi[fb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPT, 0).h, dphi[fb]);
+                dphi[fb] = mfma(tr_op<false>(p0, p0 + 16 * kPT, 0).h, A, dphi[fb]);
             }
         }
+        const float pin8[8] = {pinc, pinc, pinc, pinc, pinc, pinc, pinc, pinc};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const bf16x8 A = perm_row_op(&sG[iw][0], ks, g, pinc);
+            const bf16x8 A = scale_op(gop[ks], pin8);
 #pragma unroll
             for (int fb = 0; fb < 8; ++fb) {
                 const uint16_t *p0 = &sSt[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
-                dphi[fb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPT, 0).h, dphi[fb]);
+                dphi[fb] = mfma(tr_op<false>(p0, p0 + 16 * kPT, 0).h, A, dphi[fb]);
             }
         }
 #pragma unroll
-        for (int fb = 0; fb < 8; ++fb) {
-            const float kf = sKv[16 * fb + c16];  // K column of M
+        for (int fb = 0; fb < 8; ++fb) {  // the denominator: K column of M, and (din) the incoming K under the outer clamp
+            const f32x4 kf = *reinterpret_cast<const f32x4 *>(&sKv[16 * fb + 4 * g]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) dphi[fb][r] += sPg[16 * w + 4 * g + r] * kf;
-        }
-        if (din) {  // the incoming K's denominator term, under the outer clamp only
+            for (int r = 0; r < 4; ++r) dphi[fb][r] += (pinc * gden) * kf[r];
+            if (din) {
+                const f32x4 ki = *reinterpret_cast<const f32x4 *>(&sKin[16 * fb + 4 * g]);
 #pragma unroll
-            for (int fb = 0; fb < 8; ++fb) {
-                const float kf = sKin[16 * fb + c16];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) dphi[fb][r] += sPc[16 * w + 4 * g + r] * kf;
+                for (int r = 0; r < 4; ++r) dphi[fb][r] += (lc * pinc * gout) * ki[r];
             }
         }
         // ---- dq = dphi[q] + 2 q dphi[q*q]
-        {
-            int64_t o[4];
-            bool ok[4];
-            float dv[4][4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = 16 * w + 4 * g + r;
-                ok[r] = i < nvalid;
-                o[r] = b * a.g_sb + h * a.g_sh + static_cast<int64_t>(c * kC + i) * a.g_sl;
-            }
+        if (valid) {
+            f32x4 dv[4];
 #pragma unroll
             for (int fb = 0; fb < 4; ++fb) {
-                // q of rows 16w + 4g + r at column 16fb + c16: one transposed read
-                const uint2 qt = lds_tr(&sQf[16 * w + 4 * g + tr_r][16 * fb + tr_c]);
+                const f32x4 qv = unpack4(&sQf[iw][16 * fb + 4 * g]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t qw = r < 2 ? qt.x : qt.y;
-                    const float qv = __uint_as_float((r & 1) ? qw & 0xFFFF0000u : qw << 16);
-                    dv[r][fb] = dphi[fb][r] + 2.0f * qv * dphi[fb + 4][r];
-                }
+                for (int r = 0; r < 4; ++r) dv[fb][r] = dphi[fb][r] + 2.0f * qv[r] * dphi[fb + 4][r];
             }
-            store_rows4(a.dq, a.dt_g, o, ok, c16, dv);
+            const int64_t i = c * kC + opaque(iw);
+            store_row16(a.dq, a.dt_g, a.g_vec, b * a.g_sb + h * a.g_sh + i * a.g_sl + 4 * g, dv);
+            // 1/d and the denominator adjoint: even lane groups the one, odd the other
+            (g & 1 ? a.g_den : a.inv_den)[static_cast<size_t>(seq) * a.L + i] = g & 1 ? gden : inv;
         }
-        // ---- M <- l^n M + (w phi_k)^T v with w_j = l^(n-1-j) on the A operand's
-        // token slots; S0 and K = [K1; K2/2] (fp32) as partial sums over all threads
-        const float ln = sPw[nvalid];
-#pragma unroll
-        for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) st[fi][nb][r] *= ln;
-        // K and S0 increments on MFMA, against the three parts of w (fp32-accurate
-        // sums: K decides the clamp): dk[fi] rows = features, columns 0..2 = parts;
-        // ds0 rows 0..2 = parts, columns = value block w
-        f32x4 dk[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-        f32x4 ds0 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            float wt[8];
-            {
-                const f32x4 w0 = *reinterpret_cast<const f32x4 *>(&sWt[wsel][32 * ks + 4 * g]);
-                const f32x4 w1 = *reinterpret_cast<const f32x4 *>(&sWt[wsel][32 * ks + 16 + 4 * g]);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    wt[t] = w0[t];
-                    wt[4 + t] = w1[t];
-                }
-            }
-            // lane (g, c16): part min(c16, 3) of w at its eight token slots, the
-            // same slots as the transposed operands (token 32ks + 16(t/4) + 4g + t%4)
-            const int pr = min(c16, 3);
-            const uint2 p0 = *reinterpret_cast<const uint2 *>(&sWp[wsel][pr][32 * ks + 4 * g]);
-            const uint2 p1 = *reinterpret_cast<const uint2 *>(&sWp[wsel][pr][32 * ks + 16 + 4 * g]);
-            const bf16x8 wpart = as_bf16x8(u32x4{p0.x, p0.y, p1.x, p1.y});
-            bf16x8 ak[2];
-#pragma unroll
-            for (int fi = 0; fi < 2; ++fi) {
-                const uint16_t *pk = &sKf[32 * ks + 4 * g + tr_r][16 * (2 * w + fi) + tr_c];
-                const bf16x8 raw = tr_op<false>(pk, pk + 16 * kPT, 0).h;
-                dk[fi] = mfma(raw, wpart, dk[fi]);
-                ak[fi] = scale_op(raw, wt);
-            }
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const uint16_t *p0v = &sV[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
-                const bf16x8 vb = tr_op<false>(p0v, p0v + 16 * kPV, 0).h;
-#pragma unroll
-                for (int fi = 0; fi < 2; ++fi) st[fi][nb] = mfma(ak[fi], vb, st[fi][nb]);
-                if (nb == w) ds0 = mfma(wpart, vb, ds0);  // wave-uniform
-            }
-        }
-        {
-            // K increment of features 16(2w + fi) + 4g + r: the quad (columns 0..3) sum
-#pragma unroll
-            for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float x = dk[fi][r];
-                    x += xor_lane<1>(x);
-                    x += xor_lane<2>(x);
-                    if (c16 == 0) sRedK[16 * (2 * w + fi) + 4 * g + r] = x;
-                }
-            // S0 increment of value column 16w + c16: rows 0..2 (lane group g = 0)
-            if (g == 0) sRedS[16 * w + c16] = (ds0[0] + ds0[1]) + ds0[2];
-        }
-        __syncthreads();  // every read of chunk c's tiles and of M_c is done; partial sums in LDS
-        if (din) {  // correction: sum over the chunk of sDh_t phi_q(t) (chunk c's tiles are still in LDS)
-            if (tid < kF) {
-                float sacc = 0.f;
-                for (int i = 0; i < nvalid; ++i) sacc += sDh[i] * bf16_bits_to_f32(sQf[i][tid]);
-                corr += sacc;
-            } else if (tid == kF) {
-                float sacc = 0.f;
-                for (int i = 0; i < nvalid; ++i) sacc += sDh[i];
-                corr += sacc;
-            }
-        }
-        if (c + 1 < c_end) {
-            if (tid < kF) kv = ln * kv + sRedK[tid];
-            if (tid < kD) sS0[tid] = ln * sS0[tid] + sRedS[tid];
-            if (tid == kF) sK0[0] = ln * sK0[0] + sPs[nvalid];
-            publish();
-            store_rows(c + 1);
-            if (c + 2 < c_end) load_rows(R, a, b, h, c + 2, ra, col, true, true, false);
-        }
+        __syncthreads();  // every read of chunk c's tiles and of M_c is done
+        if (din) __syncthreads();  // (the correction's reads too)
     }
-    if (din && tid <= kF) a.kcorr[static_cast<size_t>(seq) * kBwdCorr + tid] = corr;
 }
 
 // ---------------------------------------------------------------- dk, dv pass
 // DUAL: the dual-state pass of a segment only -- from zero, no dk / dv, the
 // segment's contribution sum_t l^(t-s0+1) phi_q(t) G_t^T written to its slot.
 template <bool DUAL>
-__global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(DUAL ? 256 : 512, DUAL ? 2 : 4) void prefill_bwd_dkv_kernel(const BwdArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t sQf[kC][kPT];   // [q | q*q]
     __shared__ __attribute__((aligned(16))) uint16_t sKf[kC][kPT];   // [k | k*k/2]
     __shared__ __attribute__((aligned(16))) uint16_t sV[kC][kPV];    // [v | 0..]
     __shared__ __attribute__((aligned(16))) uint16_t sG[kC][kPV];    // [dy / d | gden | 0..]
     __shared__ __attribute__((aligned(16))) uint16_t sW[kSR][kPT];   // bf16 W^T at the chunk end
-    __shared__ float sW1[kSR], sGd[kC], sPw[kC + 2];
+    __shared__ __attribute__((aligned(16))) float sW1[kSR], sGd[kC];
+    __shared__ float sPw[kC + 2];
     __shared__ __attribute__((aligned(16))) float sOm[kC];  // om_t = l^(t+1) (= sPw[t + 1]), 16-byte aligned
-    __shared__ float sRed[kD], sRedG[1];  // the chunk's W1 increment (value columns, gden column)
     // om_t = l^(t+1) split into three bf16 parts (hi, mid, lo), row 3 zero: the
     // A operand of the W1 increment on MFMA
     __shared__ __attribute__((aligned(16))) uint16_t sOmp[4][kC];
 
     const int tid = threadIdx.x;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const bool is_u = DUAL || wave >= 4;     // update role
+    const int w = wave & 3, ut = tid & 255;  // wave and thread index within the role
     const int g = lane >> 4, c16 = lane & 15;
     const int tr_r = c16 >> 2, tr_c = 4 * (c16 & 3);
     const int unit = blockIdx.x;
@@ -651,309 +733,328 @@ __global__ __launch_bounds__(256, 2) void prefill_bwd_dkv_kernel(const BwdArgs a
         sOmp[2][tid] = f32_to_bf16_bits(r1 - bf16_bits_to_f32(mid));
         sOmp[3][tid] = 0u;
     }
-    for (int idx = tid; idx < kC * 16; idx += 256) {
+    for (int idx = tid; idx < kC * 16; idx += DUAL ? 256 : 512) {
         const int row = idx >> 4, cc = kD + (idx & 15);
         sV[row][cc] = 0u;
         sG[row][cc] = 0u;
     }
 
-    // this lane's key row jw of the transposed blocks; rows 16w + 4g + r of the outputs
-    const int jw = 16 * w + c16;
-
-    // dual state W (features 32w..32w+31, value blocks 0..4) from the final state's adjoint
-    f32x4 st[2][5];
-#pragma unroll
-    for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-        for (int nb = 0; nb < 5; ++nb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
-                float x = 0.f;
-                if (DUAL) {
-                } else if (slot) {  // W at the segment end, in this kernel's convention
-                    if (n < kD) x = slot[(f < kD ? kWsS1 : kWsS2) + fr * kD + n];
-                    else if (n == kD) x = slot[(f < kD ? kWsK1 : kWsK2) + fr];
-                } else if (a.ds1o) {
-                    if (n < kD) x = (f < kD ? a.ds1o : a.ds2o)[so1 + fr * kD + n];
-                    else if (n == kD) x = (f < kD ? a.dk1o : a.dk2o)[so0 + fr];
-                    if (f >= kD) x *= 2.0f;  // rows 64.. of M hold S2/2 and K2/2
-                }
-                st[fi][nb][r] = x;
-            }
-    float w1 = 0.f;  // constant row of W, column tid (tid <= 64)
-    if (!DUAL && tid <= kD) {
-        if (slot) w1 = slot[tid < kD ? kWsS0 + tid : kWsK0];
-        else if (a.ds1o) w1 = tid < kD ? a.ds0o[so0 + tid] : a.dk0o[seq];
-    }
-    auto publish = [&]() {
-#pragma unroll
-        for (int fi = 0; fi < 2; ++fi)
-#pragma unroll
-            for (int nb = 0; nb < 5; ++nb) {
-                const int n = 16 * nb + c16;
-                if (n > kD) continue;
-                *reinterpret_cast<uint2 *>(&sW[n][16 * (2 * w + fi) + 4 * g]) =
-                    uint2{pack2(st[fi][nb][0], st[fi][nb][1]), pack2(st[fi][nb][2], st[fi][nb][3])};
-            }
-        if (tid <= kD) sW1[tid] = w1;
-    };
-
-    const int ra = tid >> 3, col = 8 * (tid & 7);
-    Rows R;
-    auto store_rows = [&](int c) {
-        const int nv = min(kC, a.L - c * kC);
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int row = ra + 32 * s;
-            const bool ok = row < nv;
-            const uint32_t m = ok ? 0xFFFFFFFFu : 0u;
-            const float inv = ok ? R.inv[s] : 0.f, gd = ok ? R.gden[s] : 0.f;
-            float gn[8];
-            unpack8(R.dy[s], gn);
-            const u32x4 q = and4(R.q[s], m);
-            st16(&sQf[row][col], q);
-            st16(&sQf[row][kD + col], sq8(q, 1.f));
-            if constexpr (!DUAL) {
-                const u32x4 k = and4(R.k[s], m);
-                st16(&sKf[row][col], k);
-                st16(&sKf[row][kD + col], sq8(k, 0.5f));
-                st16(&sV[row][col], and4(R.v[s], m));
-            }
-            st16(&sG[row][col], pack8s(gn, inv));
-            if (col == 0) {
-                sGd[row] = gd;
-                sG[row][kD] = f32_to_bf16_bits(gd);
-            }
-        }
-    };
-
     __syncthreads();  // power table
-    float mask[4][4];  // l^(i-j) [i >= j] for i = 16ib + 4g + r, j = jw (sPw[n]: l^n rounded from fp64)
-#pragma unroll
-    for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int d = 16 * ib + 4 * g + r - jw;
-            mask[ib][r] = (ib >= w && d >= 0) ? sPw[max(d, 0)] : 0.f;
-        }
-    load_rows(R, a, b, h, c_end - 1, ra, col, true, !DUAL, true);
-    store_rows(c_end - 1);
-    publish();
-    if (c_end - 2 >= c_begin) load_rows(R, a, b, h, c_end - 2, ra, col, true, !DUAL, true);
 
-    for (int c = c_end - 1; c >= c_begin; --c) {
-        const int nvalid = min(kC, a.L - c * kC);
-        __syncthreads();  // tiles of chunk c and W at its end in LDS
-        if constexpr (!DUAL) {
-        // ---- A[i][jw] = mask (1 + phi_q(i) . phi_k(jw)) and P[i][jw] = mask (g_i . v_jw + gden_i), i blocks ib >= w
-        f32x4 sc[4], pp[4];
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib) {
-            sc[ib] = pp[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (ib < w) continue;
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-                sc[ib] = mfma(as_bf16x8(lds128(&sQf[16 * ib + c16][32 * ks + 8 * g])),
-                              as_bf16x8(lds128(&sKf[jw][32 * ks + 8 * g])), sc[ib]);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                pp[ib] = mfma(as_bf16x8(lds128(&sG[16 * ib + c16][32 * ks + 8 * g])),
-                              as_bf16x8(lds128(&sV[jw][32 * ks + 8 * g])), pp[ib]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                sc[ib][r] = mask[ib][r] * (1.0f + sc[ib][r]);
-                pp[ib][r] = mask[ib][r] * (pp[ib][r] + sGd[16 * ib + 4 * g + r]);
-            }
+    if (is_u) {
+        // ================ update role: the dual state and the tiles
+        // dual state W (features 32w..32w+31, value blocks 0..4) from the final
+        // state's adjoint or the segment's slot (W at its end, in this kernel's
+        // convention): one uniform choice of source, then every load in flight at once
+        const float *W1p = nullptr, *W2p = nullptr, *W0p = nullptr, *Wk1p = nullptr, *Wk2p = nullptr, *Wk0p = nullptr;
+        float two = 1.0f;  // rows 64.. of M hold S2/2 and K2/2
+        if (!DUAL && slot) {
+            W1p = slot + kWsS1; W2p = slot + kWsS2; W0p = slot + kWsS0;
+            Wk1p = slot + kWsK1; Wk2p = slot + kWsK2; Wk0p = slot + kWsK0;
+        } else if (!DUAL && a.ds1o) {
+            W1p = a.ds1o + so1; W2p = a.ds2o + so1; W0p = a.ds0o + so0;
+            Wk1p = a.dk1o + so0; Wk2p = a.dk2o + so0; Wk0p = a.dk0o + seq;
+            two = 2.0f;
         }
-        // tail weights l^(e-1-j): for the A-operand row jw and the output rows 16w + 4g + r
-        const float tjc = jw < nvalid ? sPw[nvalid - 1 - jw] : 0.f;
-        float tjr[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = 16 * w + 4 * g + r;
-            tjr[r] = j < nvalid ? sPw[nvalid - 1 - j] : 0.f;
-        }
-        // ---- dv rows 16w + 4g + r: A^T G + tail (phi_k W + W1)
-        f32x4 dvv[4];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) dvv[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            if (2 * ks + 1 < w) continue;
-            const bf16x8 A = acc_op(sc[2 * ks], sc[2 * ks + 1]);
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb) {
-                const uint16_t *p0 = &sG[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
-                dvv[nb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPV, 0).h, dvv[nb]);
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            float kf[8];
-            unpack8(lds128(&sKf[jw][32 * ks + 8 * g]), kf);
-            const bf16x8 A = as_bf16x8(pack8s(kf, tjc));
-#pragma unroll
-            for (int nb = 0; nb < 4; ++nb)
-                dvv[nb] = mfma(A, as_bf16x8(lds128(&sW[16 * nb + c16][32 * ks + 8 * g])), dvv[nb]);
-        }
-        int64_t orow[4];
-        bool okr[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = 16 * w + 4 * g + r;
-            okr[r] = j < nvalid;
-            orow[r] = b * a.g_sb + h * a.g_sh + static_cast<int64_t>(c * kC + j) * a.g_sl;
-        }
-        {
-            float dv[4][4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int nb = 0; nb < 4; ++nb) dv[r][nb] = dvv[nb][r] + tjr[r] * sW1[16 * nb + c16];
-            store_rows4(a.dv, a.dt_g, orow, okr, c16, dv);
-        }
-        // ---- dphi_k rows 16w + 4g + r: P^T phi_q + tail (W V')
-        f32x4 dphi[8];
-#pragma unroll
-        for (int fb = 0; fb < 8; ++fb) dphi[fb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            if (2 * ks + 1 < w) continue;
-            const bf16x8 A = acc_op(pp[2 * ks], pp[2 * ks + 1]);
-#pragma unroll
-            for (int fb = 0; fb < 8; ++fb) {
-                const uint16_t *p0 = &sQf[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
-                dphi[fb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPT, 0).h, dphi[fb]);
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const bf16x8 A = perm_row_op(&sV[jw][0], ks, g, tjc);
-#pragma unroll
-            for (int fb = 0; fb < 8; ++fb) {
-                const uint16_t *p0 = &sW[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
-                dphi[fb] = mfma(A, tr_op<false>(p0, p0 + 16 * kPT, 0).h, dphi[fb]);
-            }
-        }
-#pragma unroll
-        for (int fb = 0; fb < 8; ++fb) {
-            const float wk = bf16_bits_to_f32(sW[kD][16 * fb + c16]);  // K column of W
-#pragma unroll
-            for (int r = 0; r < 4; ++r) dphi[fb][r] += tjr[r] * wk;
-        }
-        // ---- dk = dphi[k] + k dphi[k*k/2]
-        {
-            float dv[4][4];
-#pragma unroll
-            for (int fb = 0; fb < 4; ++fb) {
-                // k of rows 16w + 4g + r at column 16fb + c16: one transposed read
-                const uint2 kt = lds_tr(&sKf[16 * w + 4 * g + tr_r][16 * fb + tr_c]);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t kw = r < 2 ? kt.x : kt.y;
-                    dv[r][fb] = dphi[fb][r] + __uint_as_float((r & 1) ? kw & 0xFFFF0000u : kw << 16) * dphi[fb + 4][r];
-                }
-            }
-            store_rows4(a.dk, a.dt_g, orow, okr, c16, dv);
-        }
-        }  // !DUAL
-        // ---- W <- l^n W + (om phi_q)^T G with om_t = l^(t-c0+1) on the A operand's
-        // token slots; W1 likewise from partial sums over all threads
-        const float ln = sPw[nvalid];
+        f32x4 st[2][5];
 #pragma unroll
         for (int fi = 0; fi < 2; ++fi)
 #pragma unroll
-            for (int nb = 0; nb < 5; ++nb)
+            for (int nb = 0; nb < 5; ++nb) st[fi][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // constant row of W: column 16w + c16 (lane group 0), and the gden column
+        float w1 = 0.f, w1g = 0.f;
+        if (W1p) {
+            const float *Wp = w < 2 ? W1p : W2p, *Wk = w < 2 ? Wk1p : Wk2p;  // waves 0, 1 hold features 0..63
+            const float sc = w < 2 ? 1.0f : two;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) st[fi][nb][r] *= ln;
-        f32x4 dw1 = f32x4{0.f, 0.f, 0.f, 0.f};  // W1 increment of value block w: rows 0..2 = om parts
+            for (int fi = 0; fi < 2; ++fi)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            float om[8];
+                for (int nb = 0; nb < 5; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int fr = (16 * (2 * w + fi) + 4 * g + r) & (kD - 1);
+                        st[fi][nb][r] = nb < 4 ? Wp[fr * kD + 16 * nb + c16] : Wk[fr];
+                    }
+            w1 = W0p[16 * w + c16];
+            w1g = Wk0p[0];
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 5; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) st[fi][nb][r] = nb < 4 || c16 == 0 ? sc * st[fi][nb][r] : 0.f;
+        }
+        const int ra = ut >> 3, col = 8 * (ut & 7);
+        Rows R;
+        u32x4 gr[2];  // dy / d as bf16
+        float gdr[2];
+        auto prepare = [&](int c) {
+            const int nv = min(kC, a.L - c * kC);
+            load_dy<true>(R, a, b, h, c, ra, col);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const bool ok = ra + 32 * s < nv;
+                gdr[s] = ok ? R.gden[s] : 0.f;
+                float gn[8];
+                unpack8(pack_raw(R.dy[s], a.dt_dy), gn);
+                gr[s] = pack8s(gn, ok ? R.inv[s] : 0.f);
+                settle(gr[s]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                if (nv < kC) {
+                    const uint32_t m = ra + 32 * s < nv ? 0xFFFFFFFFu : 0u;
+                    R.q[s] = and4(R.q[s], m);
+                    if constexpr (!DUAL) {
+                        R.k[s] = and4(R.k[s], m);
+                        R.v[s] = and4(R.v[s], m);
+                    }
+                }
+            }
+        };
+        auto publish = [&]() {  // the prepared tiles and W at their chunk's end
+            const int t = opaque(ut), ra = t >> 3, col = 8 * (t & 7);
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int row = ra + 32 * s;
+                st16(&sQf[row][col], R.q[s]);
+                st16(&sQf[row][kD + col], sq8(R.q[s], 1.f));
+                if constexpr (!DUAL) {
+                    st16(&sKf[row][col], R.k[s]);
+                    st16(&sKf[row][kD + col], sq8(R.k[s], 0.5f));
+                    st16(&sV[row][col], R.v[s]);
+                }
+                st16(&sG[row][col], gr[s]);
+                if (col == 0) {
+                    sGd[row] = gdr[s];
+                    sG[row][kD] = f32_to_bf16_bits(gdr[s]);
+                }
+            }
+            if constexpr (!DUAL) {
+#pragma unroll
+                for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                    for (int nb = 0; nb < 5; ++nb) {
+                        const int n = 16 * nb + c16;
+                        if (n > kD) continue;
+                        *reinterpret_cast<uint2 *>(&sW[n][16 * (2 * w + fi) + 4 * g]) =
+                            uint2{pack2(st[fi][nb][0], st[fi][nb][1]), pack2(st[fi][nb][2], st[fi][nb][3])};
+                    }
+                if (g == 0) sW1[16 * w + c16] = w1;
+            }
+        };
+        load_qkv<!DUAL>(R, a, b, h, c_end - 1, ra, col);
+        prepare(c_end - 1);
+        publish();
+        if (c_end - 2 >= c_begin) load_qkv<!DUAL>(R, a, b, h, c_end - 2, ra, col);
+        for (int c = c_end - 1; c >= c_begin; --c) {
+            const int nvalid = min(kC, a.L - c * kC);
+            __syncthreads();  // tiles of chunk c and W at its end in LDS
+            // ---- W <- l^n W + (om phi_q)^T G with om_t = l^(t-c0+1) on the A operand's
+            // token slots; W1 likewise from partial sums over all threads
+            const float ln = sPw[nvalid];
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 5; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) st[fi][nb][r] *= ln;
+            f32x4 dw1 = f32x4{0.f, 0.f, 0.f, 0.f};  // W1 increment of value block w: rows 0..2 = om parts
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                float om[8];
+                {
+                    const f32x4 o0 = *reinterpret_cast<const f32x4 *>(&sOm[32 * ks + 4 * g]);
+                    const f32x4 o1 = *reinterpret_cast<const f32x4 *>(&sOm[32 * ks + 16 + 4 * g]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        om[t] = o0[t];
+                        om[4 + t] = o1[t];
+                    }
+                }
+                // lane (g, c16): part min(c16, 3) of om at its eight token slots
+                const int pr = min(c16, 3);
+                const uint2 o0 = *reinterpret_cast<const uint2 *>(&sOmp[pr][32 * ks + 4 * g]);
+                const uint2 o1 = *reinterpret_cast<const uint2 *>(&sOmp[pr][32 * ks + 16 + 4 * g]);
+                const bf16x8 ompart = as_bf16x8(u32x4{o0.x, o0.y, o1.x, o1.y});
+                bf16x8 aq[2];
+#pragma unroll
+                for (int fi = 0; fi < 2; ++fi) {
+                    const uint16_t *p0 = &sQf[32 * ks + 4 * g + tr_r][16 * (2 * w + fi) + tr_c];
+                    aq[fi] = scale_op(tr_op<false>(p0, p0 + 16 * kPT, 0).h, om);
+                }
+#pragma unroll
+                for (int nb = 0; nb < 5; ++nb) {
+                    const uint16_t *p0 = &sG[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
+                    const bf16x8 gb = tr_op<false>(p0, p0 + 16 * kPV, 0).h;
+#pragma unroll
+                    for (int fi = 0; fi < 2; ++fi) st[fi][nb] = mfma(aq[fi], gb, st[fi][nb]);
+                    if (nb == w) dw1 = mfma(ompart, gb, dw1);  // wave-uniform
+                }
+            }
             {
-                const f32x4 o0 = *reinterpret_cast<const f32x4 *>(&sOm[32 * ks + 4 * g]);
-                const f32x4 o1 = *reinterpret_cast<const f32x4 *>(&sOm[32 * ks + 16 + 4 * g]);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    om[t] = o0[t];
-                    om[4 + t] = o1[t];
-                }
+                // W1[n] = sum_t om_t G_t[n]: value column 16w + c16 from the three om parts
+                // (rows 0..2, lane group g = 0); the gden column (fp32) in every wave alike
+                w1 = ln * w1 + ((dw1[0] + dw1[1]) + dw1[2]);
+                w1g = ln * w1g + wave_sum(sPw[lane + 1] * sGd[lane]);
             }
-            // lane (g, c16): part min(c16, 3) of om at its eight token slots
-            const int pr = min(c16, 3);
-            const uint2 o0 = *reinterpret_cast<const uint2 *>(&sOmp[pr][32 * ks + 4 * g]);
-            const uint2 o1 = *reinterpret_cast<const uint2 *>(&sOmp[pr][32 * ks + 16 + 4 * g]);
-            const bf16x8 ompart = as_bf16x8(u32x4{o0.x, o0.y, o1.x, o1.y});
-            bf16x8 aq[2];
-#pragma unroll
-            for (int fi = 0; fi < 2; ++fi) {
-                const uint16_t *p0 = &sQf[32 * ks + 4 * g + tr_r][16 * (2 * w + fi) + tr_c];
-                aq[fi] = scale_op(tr_op<false>(p0, p0 + 16 * kPT, 0).h, om);
-            }
-#pragma unroll
-            for (int nb = 0; nb < 5; ++nb) {
-                const uint16_t *p0 = &sG[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
-                const bf16x8 gb = tr_op<false>(p0, p0 + 16 * kPV, 0).h;
-#pragma unroll
-                for (int fi = 0; fi < 2; ++fi) st[fi][nb] = mfma(aq[fi], gb, st[fi][nb]);
-                if (nb == w) dw1 = mfma(ompart, gb, dw1);  // wave-uniform
+            __builtin_amdgcn_sched_barrier(0);
+            if (c > c_begin) prepare(c - 1);
+            __syncthreads();  // every read of chunk c's tiles and of W is done
+            if (c > c_begin) {
+                publish();
+                __builtin_amdgcn_sched_barrier(0);
+                if (c - 2 >= c_begin) load_qkv<!DUAL>(R, a, b, h, c - 2, ra, col);
             }
         }
-        {
-            // W1[n] = sum_t om_t G_t[n]: value column 16w + c16 from the three om parts
-            // (rows 0..2, lane group g = 0); the gden column (fp32) on wave 0
-            if (g == 0) sRed[16 * w + c16] = (dw1[0] + dw1[1]) + dw1[2];
-            if (w == 0) {
-                const float gs = wave_sum(sPw[lane + 1] * sGd[lane]);
-                if (lane == 0) sRedG[0] = gs;
-            }
-        }
-        __syncthreads();  // every read of chunk c's tiles and of W is done; partial sums in LDS
-        if (tid < kD) {
-            w1 = ln * w1 + sRed[tid];
-        } else if (tid == kD) {
-            w1 = ln * w1 + sRedG[0];
-        }
-        if (c > c_begin) {
-            publish();
-            store_rows(c - 1);
-            if (c - 2 >= c_begin) load_rows(R, a, b, h, c - 2, ra, col, true, !DUAL, true);
-        }
-    }
-    if constexpr (DUAL) {
-        // the segment's contribution, in this kernel's convention
+        if constexpr (DUAL) {
+            // the segment's contribution, in this kernel's convention
 #pragma unroll
-        for (int fi = 0; fi < 2; ++fi)
+            for (int fi = 0; fi < 2; ++fi)
 #pragma unroll
-            for (int nb = 0; nb < 5; ++nb)
+                for (int nb = 0; nb < 5; ++nb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
-                    if (n < kD) slot[(f < kD ? kWsS1 : kWsS2) + fr * kD + n] = st[fi][nb][r];
-                    else if (n == kD) slot[(f < kD ? kWsK1 : kWsK2) + fr] = st[fi][nb][r];
-                }
-        if (tid <= kD) slot[tid < kD ? kWsS0 + tid : kWsK0] = w1;
+                    for (int r = 0; r < 4; ++r) {
+                        const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
+                        if (n < kD) slot[(f < kD ? kWsS1 : kWsS2) + fr * kD + n] = st[fi][nb][r];
+                        else if (n == kD) slot[(f < kD ? kWsK1 : kWsK2) + fr] = st[fi][nb][r];
+                    }
+            if (g == 0) slot[kWsS0 + 16 * w + c16] = w1;
+            if (ut == 0) slot[kWsK0] = w1g;
+            return;
+        }
+        // ---- the incoming state's adjoint: W after chunk 0 (S2, K2 rows halved back);
+        // with segments the dual scan writes it
+        if (a.ds1i && a.G == 1) {
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < 5; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
+                        float x = st[fi][nb][r];
+                        if (n == kD && a.dense_in) x += a.kcorr[static_cast<size_t>(seq) * kBwdCorr + f];
+                        if (f >= kD) x *= 0.5f;
+                        if (n < kD) (f < kD ? a.ds1i : a.ds2i)[so1 + fr * kD + n] = x;
+                        else if (n == kD) (f < kD ? a.dk1i : a.dk2i)[so0 + fr] = x;
+                    }
+            if (g == 0) a.ds0i[so0 + 16 * w + c16] = w1;
+            if (ut == 0) a.dk0i[seq] = w1g + (a.dense_in ? a.kcorr[static_cast<size_t>(seq) * kBwdCorr + kF] : 0.f);
+        }
         return;
     }
-    // ---- the incoming state's adjoint: W after chunk 0 (S2, K2 rows halved back);
-    // with segments the dual scan writes it
-    if (a.ds1i && a.G == 1) {
+
+    // ================ readout role: dk and dv of rows 16w..16w+15 of every chunk
+    if constexpr (!DUAL) {
+        const int jw = 16 * w + c16;  // this lane's key row of the transposed blocks
+        float mask[4][4];  // l^(i-j) [i >= j] for i = 16ib + 4g + r, j = jw (sPw[n]: l^n rounded from fp64)
 #pragma unroll
-        for (int fi = 0; fi < 2; ++fi)
+        for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
-            for (int nb = 0; nb < 5; ++nb)
+            for (int r = 0; r < 4; ++r) {
+                const int d = 16 * ib + 4 * g + r - jw;
+                mask[ib][r] = (ib >= w && d >= 0) ? sPw[max(d, 0)] : 0.f;
+            }
+        for (int c = c_end - 1; c >= c_begin; --c) {
+            const int nvalid = min(kC, a.L - c * kC);
+            __syncthreads();  // tiles of chunk c and W at its end in LDS
+            // ---- A[i][jw] = mask (1 + phi_q(i) . phi_k(jw)) and P[i][jw] = mask (g_i . v_jw + gden_i), i blocks ib >= w
+            f32x4 sc[4], pp[4];
+#pragma unroll
+            for (int ib = 0; ib < 4; ++ib) {
+                sc[ib] = pp[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (ib < w) continue;
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks)
+                    sc[ib] = mfma(as_bf16x8(lds128(&sQf[16 * ib + c16][32 * ks + 8 * g])),
+                                  as_bf16x8(lds128(&sKf[jw][32 * ks + 8 * g])), sc[ib]);
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+                    pp[ib] = mfma(as_bf16x8(lds128(&sG[16 * ib + c16][32 * ks + 8 * g])),
+                                  as_bf16x8(lds128(&sV[jw][32 * ks + 8 * g])), pp[ib]);
+                const f32x4 gd = *reinterpret_cast<const f32x4 *>(&sGd[16 * ib + 4 * g]);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int f = 16 * (2 * w + fi) + 4 * g + r, fr = f & (kD - 1), n = 16 * nb + c16;
-                    float x = st[fi][nb][r];
-                    if (n == kD && a.dense_in) x += a.kcorr[static_cast<size_t>(seq) * kBwdCorr + f];
-                    if (f >= kD) x *= 0.5f;
-                    if (n < kD) (f < kD ? a.ds1i : a.ds2i)[so1 + fr * kD + n] = x;
-                    else if (n == kD) (f < kD ? a.dk1i : a.dk2i)[so0 + fr] = x;
+                    sc[ib][r] = mask[ib][r] * (1.0f + sc[ib][r]);
+                    pp[ib][r] = mask[ib][r] * (pp[ib][r] + gd[r]);
                 }
-        if (tid < kD) a.ds0i[so0 + tid] = w1;
-        else if (tid == kD) a.dk0i[seq] = w1 + (a.dense_in ? a.kcorr[static_cast<size_t>(seq) * kBwdCorr + kF] : 0.f);
+            }
+            // tail weight l^(e-1-j) of row jw
+            const float tjc = jw < nvalid ? sPw[nvalid - 1 - jw] : 0.f;
+            const int64_t orow = b * a.g_sb + h * a.g_sh + static_cast<int64_t>(c * kC + opaque(jw)) * a.g_sl + 4 * g;
+            // ---- dv of row jw, columns 16nb + 4g + r: A^T G + tail (phi_k W + W1)
+            {
+                f32x4 dvv[4];
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) dvv[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    if (2 * ks + 1 < w) continue;
+                    const bf16x8 A = acc_op(sc[2 * ks], sc[2 * ks + 1]);
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb) {
+                        const uint16_t *p0 = &sG[32 * ks + 4 * g + tr_r][16 * nb + tr_c];
+                        dvv[nb] = mfma(tr_op<false>(p0, p0 + 16 * kPV, 0).h, A, dvv[nb]);
+                    }
+                }
+#pragma unroll
+                for (int ks = 0; ks < 4; ++ks) {
+                    float kf[8];
+                    unpack8(lds128(&sKf[jw][32 * ks + 8 * g]), kf);
+                    const bf16x8 A = as_bf16x8(pack8s(kf, tjc));
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb)
+                        dvv[nb] = mfma(as_bf16x8(lds128(&sW[16 * nb + c16][32 * ks + 8 * g])), A, dvv[nb]);
+                }
+#pragma unroll
+                for (int nb = 0; nb < 4; ++nb) {
+                    const f32x4 w1v = *reinterpret_cast<const f32x4 *>(&sW1[16 * nb + 4 * g]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) dvv[nb][r] += tjc * w1v[r];
+                }
+                if (jw < nvalid) store_row16(a.dv, a.dt_g, a.g_vec, orow, dvv);
+            }
+            // ---- dphi_k of row jw, features 16fb + 4g + r: P^T phi_q + tail (W V')
+            f32x4 dphi[8];
+#pragma unroll
+            for (int fb = 0; fb < 8; ++fb) dphi[fb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                if (2 * ks + 1 < w) continue;
+                const bf16x8 A = acc_op(pp[2 * ks], pp[2 * ks + 1]);
+#pragma unroll
+                for (int fb = 0; fb < 8; ++fb) {
+                    const uint16_t *p0 = &sQf[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
+                    dphi[fb] = mfma(tr_op<false>(p0, p0 + 16 * kPT, 0).h, A, dphi[fb]);
+                }
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const bf16x8 A = perm_row_op(&sV[jw][0], ks, g, tjc);
+#pragma unroll
+                for (int fb = 0; fb < 8; ++fb) {
+                    const uint16_t *p0 = &sW[32 * ks + 4 * g + tr_r][16 * fb + tr_c];
+                    dphi[fb] = mfma(tr_op<false>(p0, p0 + 16 * kPT, 0).h, A, dphi[fb]);
+                }
+            }
+            // ---- dk = dphi[k] + k dphi[k*k/2], the K column of W added to both
+            if (jw < nvalid) {
+                f32x4 dv[4];
+#pragma unroll
+                for (int fb = 0; fb < 4; ++fb) {
+                    const f32x4 kv = unpack4(&sKf[jw][16 * fb + 4 * g]);
+                    const f32x4 wa = unpack4(&sW[kD][16 * fb + 4 * g]), wb = unpack4(&sW[kD][kD + 16 * fb + 4 * g]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        dv[fb][r] = (dphi[fb][r] + tjc * wa[r]) + kv[r] * (dphi[fb + 4][r] + tjc * wb[r]);
+                }
+                store_row16(a.dk, a.dt_g, a.g_vec, orow, dv);
+            }
+            __syncthreads();  // every read of chunk c's tiles and of W is done
+        }
     }
 }
 
@@ -1039,8 +1140,13 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
     *G = (NC + c - 1) / c;  // no empty segments
 }
 
-hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream) {
-    if (a.dt_in == PRIME_F32) return launch_prefill_backward_f32(a, stream);
+hipError_t launch_prefill_backward(const BwdArgs &args, hipStream_t stream) {
+    if (args.dt_in == PRIME_F32) return launch_prefill_backward_f32(args, stream);
+    BwdArgs a = args;
+    // gradient rows take one store of four elements if every row starts on such a boundary
+    const uintptr_t gsz = (a.dt_g == PRIME_F32 ? 4 : 2) * 4;
+    a.g_vec = !((reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
+                 reinterpret_cast<uintptr_t>(a.dv)) % gsz || a.g_sb % 4 || a.g_sh % 4 || a.g_sl % 4);
     const int S = a.B * a.H;
     hipError_t e;
     if (a.G > 1) {
@@ -1059,9 +1165,9 @@ hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream) {
     const int units = S * a.G;
     const TimerEvents t1 = timer_events(PRIME_KERNEL_BWD_DQ);
     if (a.dense_in)
-        hipExtLaunchKernelGGL(prefill_bwd_dq_kernel<true>, dim3(units), dim3(256), 0, stream, t1.start, t1.stop, 0, a);
+        hipExtLaunchKernelGGL(prefill_bwd_dq_kernel<true>, dim3(units), dim3(512), 0, stream, t1.start, t1.stop, 0, a);
     else
-        hipExtLaunchKernelGGL(prefill_bwd_dq_kernel<false>, dim3(units), dim3(256), 0, stream, t1.start, t1.stop, 0,
+        hipExtLaunchKernelGGL(prefill_bwd_dq_kernel<false>, dim3(units), dim3(512), 0, stream, t1.start, t1.stop, 0,
                               a);
     if ((e = hipGetLastError()) != hipSuccess) return timer_drop(t1), e;
     if (a.G > 1) {
@@ -1073,7 +1179,7 @@ hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream) {
         if ((e = launch_bwd_dual_scan(a, stream)) != hipSuccess) return e;
     }
     const TimerEvents t2 = timer_events(PRIME_KERNEL_BWD_DKV);
-    hipExtLaunchKernelGGL(prefill_bwd_dkv_kernel<false>, dim3(units), dim3(256), 0, stream, t2.start, t2.stop, 0,
+    hipExtLaunchKernelGGL(prefill_bwd_dkv_kernel<false>, dim3(units), dim3(512), 0, stream, t2.start, t2.stop, 0,
                           a);
     if ((e = hipGetLastError()) != hipSuccess) timer_drop(t2);
     return e;

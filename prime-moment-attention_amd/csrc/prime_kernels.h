@@ -205,6 +205,7 @@ struct BwdArgs {
     void *dq, *dk, *dv;
     int dt_g;
     int64_t g_sb, g_sh, g_sl;                               // strides of dq, dk, dv
+    bool g_vec;  // (bf16 passes) gradient rows on boundaries of four elements; set by the launch
     float *ds0i, *ds1i, *ds2i, *dk0i, *dk1i, *dk2i;         // adjoint of the incoming state (null => none)
     float *inv_den, *g_den;                                 // [B*H, L] fp32, written by the dq pass
     // the dense branch's double clamp with an incoming state (G == 1): the dq

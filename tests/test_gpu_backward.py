@@ -375,3 +375,31 @@ def test_backward_segmented_equals_one_segment(with_state, dtype):
     ref = O.recurrent_vjp(q.reshape(BH, L, D), k.reshape(BH, L, D), v.reshape(BH, L, D),
                           np.tile(lam.astype(np.float64), B), dy.reshape(BH, L, D), state=st0, dstate=ds)
     _check(ref, outs[0][0], outs[0][1], TOL_BF16 if bf else TOL_F32)
+
+
+@pytest.mark.parametrize("L", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("dense_state", [False, True])
+def test_backward_row_alignment_and_dy_dtype(L, dense_state):
+    """Gradient rows that start off the four-element boundary (element stores)
+    against aligned ones (one store per four), and a wide dy against bf16 dy of the
+    same values: the same arithmetic, so the same bits, for every gradient dtype."""
+    B, H = 2, 3
+    q, k, v = (to_dev(x, torch.bfloat16) for x in O.make_inputs((B, H, L, D), seed=500 + L, bf16=True))
+    lam = to_dev(np.array([0.99, 0.995, 0.9995], np.float32))
+    dy = to_dev(O.bf16_round(np.random.default_rng(501).standard_normal((B, H, L, D)).astype(np.float32)))
+    st0 = state_to_dev(random_state(B * H, D, 502), B, H, D) if dense_state else None
+
+    def run(gdtype, dydtype, pitch):
+        g = [torch.empty(B, H, L, pitch, device=dev(), dtype=gdtype)[..., pitch - D:] for _ in range(3)]
+        dsi = _lib.new_state(B, H, D, dev()) if dense_state else None
+        _lib.chunked_prefill_backward(q, k, v, lam, 1.0, st0, dy.to(dydtype), None, *g, dsi,
+                                      flags=1 if dense_state else 0)
+        torch.cuda.synchronize()
+        return [x.contiguous() for x in g] + list(dsi or ())
+
+    for gdtype in (torch.bfloat16, torch.float16, torch.float32):
+        ref = run(gdtype, torch.bfloat16, D)
+        for dydtype, pitch in ((torch.bfloat16, D + 1), (torch.float32, D + 3), (torch.float32, D)):
+            print(f"[backward rows] L={L} {gdtype} dy {dydtype} pitch {pitch}", flush=True)
+            for x, y in zip(ref, run(gdtype, dydtype, pitch)):
+                assert torch.isfinite(x.float()).all() and torch.equal(x, y)
