@@ -379,35 +379,57 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(const PrefillArgs a) {
     const size_t so0 = static_cast<size_t>(seq) * kD;
     f32x4 st[2][NBX];  // feature blocks 2u+fi (rows 4g+r), value blocks nb (column c16)
     if (is_u) {
+        // one uniform choice of source, then every load in flight at once (a choice
+        // per element makes each load wait for the last)
+        const float *S1p = nullptr, *S2p = nullptr, *S0p = nullptr, *K1p = nullptr, *K2p = nullptr, *K0p = nullptr;
+        if (from_ws) {
+            S1p = wslot + kWsS1; S2p = wslot + kWsS2; S0p = wslot + kWsS0;
+            K1p = wslot + kWsK1; K2p = wslot + kWsK2; K0p = wslot + kWsK0;
+        } else if (has_in) {
+            S1p = a.s1i + so1; S2p = a.s2i + so1; S0p = a.s0i + so0;
+            K1p = a.k1i + so0; K2p = a.k2i + so0; K0p = a.k0i + seq;
+        }
 #pragma unroll
         for (int fi = 0; fi < 2; ++fi)
 #pragma unroll
-            for (int nb = 0; nb < NBX; ++nb)
+            for (int nb = 0; nb < NBX; ++nb) st[fi][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float x0 = 0.f;  // S0[utid], or the incoming K feature / K0 by thread, below
+        if (S1p) {
+            const bool first = u < 2;  // waves 0, 1 hold features 0..63: S1, K1
+            const float *Sp = first ? S1p : S2p, *Kp = first ? K1p : K2p;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int f = 16 * (2 * u + fi) + 4 * g + r, fr = f & (kD - 1);
-                    const int n = 16 * nb + c16;
-                    float x = 0.f;
-                    if (n < kD) {
-                        if (from_ws) x = wslot[(f < kD ? kWsS1 : kWsS2) + fr * kD + n];
-                        else if (has_in) x = (f < kD ? a.s1i : a.s2i)[so1 + fr * kD + n];
-                    } else if (n == kD && !dense) {  // dense: K of the call only, incoming in sKi
-                        if (from_ws) x = wslot[(f < kD ? kWsK1 : kWsK2) + fr];
-                        else if (has_in) x = (f < kD ? a.k1i : a.k2i)[so0 + fr];
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < NBX; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int fr = (16 * (2 * u + fi) + 4 * g + r) & (kD - 1);
+                        st[fi][nb][r] = nb < NB ? Sp[fr * kD + 16 * nb + c16] : Kp[fr];
                     }
-                    st[fi][nb][r] = f < kD ? x : 0.5f * x;
-                }
+            const int f = (utid - kD) & (kF - 1);
+            const float *p0 = utid < kD ? S0p + utid : utid == kD + kF ? K0p : (f < kD ? K1p : K2p) + (f & (kD - 1));
+            x0 = *p0;
+#pragma unroll
+            for (int fi = 0; fi < 2; ++fi)
+#pragma unroll
+                for (int nb = 0; nb < NBX; ++nb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        // column 64 is K (dense: K of the call only, the incoming one in sKi)
+                        const bool have = nb < NB || (c16 == 0 && !dense);
+                        const float x = st[fi][nb][r];
+                        st[fi][nb][r] = !have ? 0.f : first ? x : 0.5f * x;
+                    }
+        }
         if (utid < kD) {
-            sS0[utid] = from_ws ? wslot[kWsS0 + utid] : (has_in ? a.s0i[so0 + utid] : 0.f);
+            sS0[utid] = x0;
         } else if (utid < kD + kF) {
-            const int f = utid - kD, fr = f & (kD - 1);
-            float x = 0.f;
-            if (dense && has_in) x = (f < kD ? a.k1i : a.k2i)[so0 + fr];
+            const int f = utid - kD;
+            const float x = dense && has_in ? x0 : 0.f;
             sKi[f] = f < kD ? x : 0.5f * x;
         } else if (utid == kD + kF) {
-            const float x = from_ws ? wslot[kWsK0] : (has_in ? a.k0i[seq] : 0.f);
-            sK0[0] = dense ? 0.f : x;
-            sK0[1] = dense ? x : 0.f;
+            sK0[0] = dense ? 0.f : x0;
+            sK0[1] = dense ? x0 : 0.f;
         }
         // constant columns 64..79 of v (1, 0, ...) and 65..79 of w v (column 64,
         // w, is written with every chunk's tile, racing nothing here)
