@@ -676,7 +676,10 @@ static int prefill_impl(const prime_tensor_t *q, const prime_tensor_t *k, const 
     if (workspace && !aligned16(workspace))
         return fail(PRIME_ERR_MISALIGNED, "workspace must be 16-byte aligned");
     const int S = B * H;
-    prime::plan_segments(S, L, a.dense_clamp != 0, workspace ? workspace_bytes : 0, &a.G, &a.cps);
+    const bool f32 = q->dtype == PRIME_F32;
+    const prime::PlanKind kind = a.log_decay ? (f32 ? prime::kPlanSelF32 : prime::kPlanSelBf16)
+                                             : (f32 ? prime::kPlanF32 : prime::kPlanBf16);
+    prime::plan_segments(S, L, a.dense_clamp != 0, workspace ? workspace_bytes : 0, kind, &a.G, &a.cps);
     a.ws = a.G > 1 ? static_cast<float *>(workspace) : nullptr;
     if (a.G == 1 && workspace && q->dtype == PRIME_BF16 && !a.dense_clamp) {
         // more sequences than CUs: the paired split, when the workspace holds it
@@ -766,7 +769,7 @@ int accumulate_launch(const prime_tensor_t *k, const prime_tensor_t *v, int B, i
     a.s0o = state_out->s0; a.s1o = state_out->s1; a.s2o = state_out->s2;
     a.k0o = state_out->k0; a.k1o = state_out->k1; a.k2o = state_out->k2;
     // G = 1 (one slot per sequence, cps = all chunks) when the workspace holds no more
-    prime::plan_segments(S, L, false, workspace_bytes, &a.G, &a.cps);
+    prime::plan_accumulate(S, L, workspace_bytes, &a.G, &a.cps);
     a.ws = static_cast<float *>(workspace);
     a.accumulate = 1;
     // in place is safe: the scan reads state_in and the slots before it writes
@@ -1459,19 +1462,23 @@ int prime_delta_decode_step(const prime_tensor_t *q, const prime_tensor_t *k, co
 size_t prime_accumulate_workspace_size(int B, int H, int L) {
     if (B <= 0 || H <= 0 || L <= 0) return 0;
     int G, cps;
-    prime::plan_segments(B * H, L, false, static_cast<size_t>(-1), &G, &cps);
+    prime::plan_accumulate(B * H, L, static_cast<size_t>(-1), &G, &cps);
     return static_cast<size_t>(B) * H * (G > 1 ? G : 1) * prime::kWsStride * sizeof(float);
 }
 
 size_t prime_chunked_prefill_workspace_size(int B, int H, int L, unsigned flags) {
     if (B <= 0 || H <= 0 || L <= 0) return 0;
-    int G, cps;
-    prime::plan_segments(B * H, L, (flags & PRIME_FLAG_DENSE_CLAMP) != 0, static_cast<size_t>(-1), &G, &cps);
-    if (G > 1) return static_cast<size_t>(B) * H * G * prime::kWsStride * sizeof(float);
     if (flags & PRIME_FLAG_DENSE_CLAMP) return 0;
+    // the most that any form of the call (bf16 or fp32, selective or not) has a use for
+    size_t need = 0;
+    for (int kind = prime::kPlanBf16; kind <= prime::kPlanSelF32; ++kind) {
+        int G, cps;
+        prime::plan_segments(B * H, L, false, static_cast<size_t>(-1), static_cast<prime::PlanKind>(kind), &G, &cps);
+        if (G > 1) need = std::max(need, static_cast<size_t>(B) * H * G * prime::kWsStride * sizeof(float));
+    }
     int K, pcs;
     prime::plan_pairs(B * H, L, &K, &pcs);
-    return K > 0 ? prime::pair_ws_bytes(K) : 0;
+    return std::max(need, K > 0 ? prime::pair_ws_bytes(K) : size_t{0});
 }
 
 }  // extern "C"

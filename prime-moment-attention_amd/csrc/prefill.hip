@@ -190,15 +190,6 @@ __device__ __forceinline__ void store_tiles_fn(const TileRegs<F32IN> &R, int rt,
                                     sVw, plVw, kPV);
 }
 
-// Segment plan.  Without a workspace (or for the dense branch, whose clamp
-// needs the incoming state apart from the tokens of this call) every sequence
-// is one segment.  Otherwise choose the number of segments G minimising a
-// simple cost in chunk-steps: the fused kernel runs one workgroup per CU, in
-// ceil(S*G / CUs) rounds of cps chunks each; the state-only pass (about half
-// the cost per chunk, several workgroups per CU) and the scan add the rest,
-// and every workspace slot costs ~4 x 33.8 KB of HBM traffic (~0.03 chunk-steps).
-constexpr int kMinCps = 4;
-
 int device_cus() {
     static int cached[64] = {0};
     int dev = 0;
@@ -211,10 +202,68 @@ int device_cus() {
     return cached[dev];
 }
 
-void plan_segments(int S, int L, bool dense_clamp, size_t ws_bytes, int *G, int *cps) {
+// Segment plan.  Without a workspace (or for the dense branch, whose clamp
+// needs the incoming state apart from the tokens of this call) every sequence
+// is one segment.  Otherwise the number of segments with the least cost in
+// microseconds: the fused kernel runs one workgroup per CU, in ceil(S*G / CUs)
+// rounds of `unit` (launch, power tables, state) plus `fused` per chunk; with
+// G > 1 come the state-only pass (`state` per chunk, `share` workgroups per CU
+// before they slow each other), the scan and launches (`fixed`) and each slot's
+// traffic (`slot`).  The five figures of each kernel are fitted to 13 shapes from
+// 12 x 128 to 96 x 8192 tokens with every G (times within 10 % of the model at the
+// chosen G): the plan is within 0.5 % of the best G on fp32 and bf16, 13 % at worst
+// (selective bf16, 12 x 1000).  12 x 512 fp32: 8 segments 25.9 us, 2 segments 44.3;
+// 12 x 512 bf16: one 20.1, 2 segments 27.3; 96 x 2048 bf16: one 59.8, 2 68.5;
+// 96 x 8192 bf16: 8 160.5, 7 169.8; 48 x 777 selective fp32: 5 56.8, 3 78.8.
+namespace {
+
+struct PlanCost {
+    double fused, state, unit, fixed, slot, share;
+};
+constexpr PlanCost kPlanCost[4] = {
+    {1.6, 1.1, 6.0, 10.0, 0.03, 3.0},   // kPlanBf16
+    {5.2, 1.9, 6.6, 10.0, 0.03, 1.0},   // kPlanF32
+    {2.1, 1.2, 6.6, 10.0, 0.025, 2.0},  // kPlanSelBf16
+    {9.5, 3.0, 5.0, 8.0, 0.03, 1.5},    // kPlanSelF32
+};
+
+}  // namespace
+
+void plan_segments(int S, int L, bool dense_clamp, size_t ws_bytes, PlanKind kind, int *G, int *cps) {
     const int NC = (L + kC - 1) / kC;
     int best_g = 1, best_c = NC;
-    if (!dense_clamp && NC >= 2 * kMinCps) {
+    if (!dense_clamp && NC > 1) {
+        const PlanCost &p = kPlanCost[kind];
+        const int cu = device_cus();
+        const double cus = cu;
+        double best = static_cast<double>((S + cu - 1) / cu) * (p.unit + p.fused * NC);
+        for (int g0 = 2; g0 <= min(NC, 64); ++g0) {
+            const int c = (NC + g0 - 1) / g0;
+            const int g = (NC + c - 1) / c;  // no empty segments
+            if (static_cast<size_t>(S) * g * kWsStride * sizeof(float) > ws_bytes) continue;
+            const int64_t units = static_cast<int64_t>(S) * g;
+            const double rounds = static_cast<double>((units + cu - 1) / cu);
+            const double states = std::max(1.0, static_cast<double>(units - S) / (p.share * cus));
+            const double cost =
+                rounds * (p.unit + p.fused * c) + p.fixed + states * p.state * c + p.slot * static_cast<double>(units);
+            if (cost < best - 1e-9) {
+                best = cost;
+                best_g = g;
+                best_c = c;
+            }
+        }
+    }
+    *G = best_g;
+    *cps = best_c;
+}
+
+// The accumulate call's plan (state-only pass and scan, no readout), in
+// chunk-steps: at least four chunks per segment and 0.03 steps per slot.
+void plan_accumulate(int S, int L, size_t ws_bytes, int *G, int *cps) {
+    constexpr int kMinCps = 4;
+    const int NC = (L + kC - 1) / kC;
+    int best_g = 1, best_c = NC;
+    if (NC >= 2 * kMinCps) {
         const int cu = device_cus();
         const int gmax = NC / kMinCps < 64 ? NC / kMinCps : 64;
         double best = 1e300;

@@ -245,7 +245,10 @@ hipError_t launch_segment_scan(const PrefillArgs &a, hipStream_t stream);
 // selective form with fp32 inputs (chunk_f32.hip)
 hipError_t launch_selective_f32(const PrefillArgs &a, hipStream_t stream);
 // segments per sequence for the launch plan, given the workspace the caller has
-void plan_segments(int S, int L, bool dense_clamp, size_t ws_bytes, int *G, int *cps);
+// and the kernel that will run (its costs differ)
+enum PlanKind { kPlanBf16, kPlanF32, kPlanSelBf16, kPlanSelF32 };
+void plan_segments(int S, int L, bool dense_clamp, size_t ws_bytes, PlanKind kind, int *G, int *cps);
+void plan_accumulate(int S, int L, size_t ws_bytes, int *G, int *cps);
 // paired split for the bf16 fused kernel when S exceeds the CU count (K = 0:
 // none pays); its workspace: K slots, then K 8-byte flags
 void plan_pairs(int S, int L, int *K, int *pcs);

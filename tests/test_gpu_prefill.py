@@ -178,3 +178,32 @@ def test_prefill_segmented_equals_one_segment(with_state):
                        state_to_np(st0, BH, D))
     assert_close(outs[0][0], yo.reshape(B, H, L, D), TOL_BF16, "y vs oracle")
     assert_state_close(outs[0][1], so, TOL_BF16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("selective", [False, True])
+@pytest.mark.parametrize("L", [64, 65, 129, 513, 1000])
+def test_prefill_short_segments_equal_one_segment(L, selective, dtype):
+    """The plan splits down to one chunk per segment (a ragged last one too): with
+    the workspace it asks for against one segment per sequence, grouped k/v and an
+    incoming state.  The two differ by the rounding of a state that is summed per
+    segment: the tolerances of the segmented tests of longer sequences."""
+    B, H, Hkv = 1, 6, 2
+    q, _, _ = O.make_inputs((B, H, L, D), seed=70, bf16=True)
+    _, k, v = O.make_inputs((B, Hkv, L, D), seed=71, bf16=True)
+    q, k, v = (to_dev(x, dtype) for x in (q, k, v))
+    st0 = state_to_dev(random_state(B * H, D, 72), B, H, D)
+    lam = to_dev(np.linspace(0.99, 0.9999, H).astype(np.float32))
+    ld = -0.02 * torch.rand(B, H, L, device=dev())
+    outs = []
+    for ws in (None, torch.empty(0, dtype=torch.uint8, device=dev())):
+        y, st = torch.empty(B, H, L, D, device=dev()), _lib.new_state(B, H, D, dev())
+        if selective:
+            _lib.selective_prefill(q, k, v, ld, torch.full((H,), 0.7, device=dev()), 1.0, st0, y, st, workspace=ws)
+        else:
+            _lib.chunked_prefill(q, k, v, lam, 1.0, 64, st0, y, st, 0, workspace=ws)
+        torch.cuda.synchronize()
+        outs.append((to_np(y), state_to_np(st, B * H, D)))
+    tol = 2e-3 if dtype == torch.bfloat16 else 1e-4
+    assert_close(outs[0][0], outs[1][0], tol, "y")
+    assert_state_close(outs[0][1], outs[1][1], tol)
