@@ -318,7 +318,7 @@ __device__ __forceinline__ void put_tile(int w, int g, int c16, f32x4 p, float (
 
 // the powers of the head's decay, l^0 .. l^64 (rounded once)
 __device__ __forceinline__ void put_powers(const ChunkF32Args &a, int h, int tid, float *sPw) {
-    if (tid <= kC) sPw[tid] = tid == 0 ? 1.0f : static_cast<float>(pow(static_cast<double>(a.decay[h]), tid));
+    if (tid <= kC) sPw[tid] = static_cast<float>(pow_sum(a.decay[h], tid).p);
 }
 
 // A state in the layout of the kernels: unit (db, dv) of M's two halves in a
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     const int i = tid >> 4, part = tid & 15, d0 = K::NE * part;
     float seg_ld = 0.f;
     double l64 = 1.0, lcd = 1.0;  // (DIN) l^64, l^(64 c)
-    if constexpr (DIN) l64 = pow(static_cast<double>(a.decay[h]), 64.0);
+    if constexpr (DIN) l64 = int_pow(a.decay[h], kC);
     Rows<DP> R;
     load_rows<DP, VEC, SEL, false, STATE_ONLY>(a, b, h, seq, c_begin, tid, R);
     if constexpr (!SEL) __syncthreads();  // sPw
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     }
     if (a.s1o && seg == a.G - 1) {
         if constexpr (DIN) {
-            const float lL = static_cast<float>(pow(static_cast<double>(a.decay[h]), static_cast<double>(a.L)));
+            const float lL = static_cast<float>(int_pow(a.decay[h], a.L));
             C.kf += lL * kfin;
             C.k0 += lL * k0in;
         }
@@ -673,7 +673,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
         if ((tid & 7) == 0 && (tid >> 3) < K::FP) sKin[tid >> 3] = C.kf;
         k0in = C.k0;
         C.kf = C.k0 = 0.f;
-        l64 = pow(static_cast<double>(a.decay[h]), 64.0);
+        l64 = int_pow(a.decay[h], kC);
     }
     if constexpr (!SEL) put_powers(a, h, tid, sPw);
 

@@ -415,11 +415,9 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(const PrefillArgs a) {
     float *wslot = a.ws ? a.ws + (static_cast<size_t>(seq) * a.G + seg) * kWsStride : nullptr;
 
     if (tid < kC + 2) {
-        const double ld = static_cast<double>(lam);
-        sPw[tid] = static_cast<float>(pow(ld, static_cast<double>(tid)));
-        double ps = 0.0, pm = 1.0;  // prefix sum of powers in fp64 (1 - l is tiny near l = 1)
-        for (int m = 0; m < tid; ++m, pm *= ld) ps += pm;
-        sPs[tid] = static_cast<float>(ps);
+        const PowSum t = pow_sum(lam, tid);
+        sPw[tid] = static_cast<float>(t.p);
+        sPs[tid] = static_cast<float>(t.s);
     }
     __syncthreads();  // the power tables are read by the first store_tiles below
 
@@ -655,7 +653,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(const PrefillArgs a) {
                     }
                     ki += __shfl_xor(ki, 16, kWave);
                     ki += __shfl_xor(ki, 32, kWave);
-                    const float den_init = pin * (sK0[1] + ki * static_cast<float>(pow(static_cast<double>(lam), 64.0 * c)));
+                    const float den_init = pin * (sK0[1] + ki * static_cast<float>(int_pow(lam, int64_t{kC} * c)));
                     den = fmaxf(fmaxf(den_call, a.eps) + den_init, a.eps);
                 } else {
                     den = fmaxf(den_call, a.eps);
@@ -770,7 +768,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(const PrefillArgs a) {
         off1 = so1; off0 = so0; offk0 = seq;
     }
     // dense clamp: the incoming K state decays separately (l^L over the call)
-    const float linit = dense ? static_cast<float>(pow(static_cast<double>(lam), static_cast<double>(a.L))) : 0.f;
+    const float linit = dense ? static_cast<float>(int_pow(lam, a.L)) : 0.f;
 #pragma unroll
     for (int fi = 0; fi < 2; ++fi)
 #pragma unroll
@@ -801,7 +799,7 @@ __global__ __launch_bounds__(256) void segment_scan_kernel(const PrefillArgs a) 
     const int seq = static_cast<int>(gid / kWsElems), e = static_cast<int>(gid % kWsElems);
     const int h = seq % a.H;
     const bool sel = a.log_decay != nullptr;
-    const float lT = sel ? 0.f : static_cast<float>(pow(static_cast<double>(a.decay[h]), static_cast<double>(a.cps) * kC));
+    const float lT = sel ? 0.f : static_cast<float>(int_pow(a.decay[h], int64_t{kC} * a.cps));
     float carry = 0.f;
     if (a.s1i != nullptr) {
         const size_t so1 = static_cast<size_t>(seq) * kD * kD, so0 = static_cast<size_t>(seq) * kD;
@@ -817,8 +815,7 @@ __global__ __launch_bounds__(256) void segment_scan_kernel(const PrefillArgs a) 
     // otherwise: exclusive prefixes for the chunk loop, in place
     const int ns = a.accumulate ? a.G : a.G - 1;
     const float lLast = (a.accumulate && !sel)
-        ? static_cast<float>(pow(static_cast<double>(a.decay[h]),
-                                 static_cast<double>(a.L - (a.G - 1) * a.cps * kC)))
+        ? static_cast<float>(int_pow(a.decay[h], a.L - (a.G - 1) * a.cps * kC))
         : 0.f;
     // eight slots' loads in flight at a time, then their dependent updates
     for (int s0 = 0; s0 < ns; s0 += 8) {

@@ -273,16 +273,13 @@ __global__ __launch_bounds__(64 * ((STATE_ONLY ? 0 : (RH ? 8 : 4)) + (UW8 ? 8 : 
     }
 
     if (tid < kC + 2) {
-        const double ld = static_cast<double>(lam);
-        sPw[tid] = static_cast<float>(pow(ld, static_cast<double>(tid)));
-        double ps = 0.0, pm = 1.0;  // prefix sum of powers in fp64 (1 - l is tiny near l = 1)
-        for (int m = 0; m < tid; ++m, pm *= ld) ps += pm;
-        sPs[tid] = static_cast<float>(ps);
+        const PowSum t = pow_sum(lam, tid);
+        sPw[tid] = static_cast<float>(t.p);
+        sPs[tid] = static_cast<float>(t.s);
     }
     if constexpr (RH) {
         if (tid < 2 * kC)
-            sPm[tid] = tid >= kC - 1 ? static_cast<float>(pow(static_cast<double>(lam), static_cast<double>(tid - (kC - 1))))
-                                     : 0.f;
+            sPm[tid] = tid >= kC - 1 ? static_cast<float>(pow_sum(lam, tid - (kC - 1)).p) : 0.f;
     }
     if constexpr (QKN) {
         if (tid < 4 * kD) {
@@ -480,7 +477,7 @@ __global__ __launch_bounds__(64 * ((STATE_ONLY ? 0 : (RH ? 8 : 4)) + (UW8 ? 8 : 
             pin = sPw[iw + 1];  // the power tables: sPw[n] is l^n rounded from fp64
         }
         // dense: l^(64 c) of the chunk, advanced by one chunk decay per step
-        float dcr = dense ? static_cast<float>(pow(static_cast<double>(lam), 64.0 * c_begin)) : 0.f;
+        float dcr = dense ? static_cast<float>(int_pow(lam, int64_t{kC} * c_begin)) : 0.f;
         for (int c = c_begin; c < c_end; ++c) {
             const int p = STATE_ONLY ? 0 : c & 1;
             const int nvalid = min(kC, a.L - c * kC);
@@ -705,7 +702,7 @@ __global__ __launch_bounds__(64 * ((STATE_ONLY ? 0 : (RH ? 8 : 4)) + (UW8 ? 8 : 
         off1 = so1; off0 = so0; offk0 = seq;
     }
     // dense clamp: the incoming K state decays separately (l^L over the call)
-    const float linit = dense ? static_cast<float>(pow(static_cast<double>(lam), static_cast<double>(a.L))) : 0.f;
+    const float linit = dense ? static_cast<float>(int_pow(lam, a.L)) : 0.f;
 #pragma unroll
     for (int fi = 0; fi < FI; ++fi)
 #pragma unroll

@@ -308,11 +308,9 @@ __global__ __launch_bounds__(512, DIN ? 2 : 4) void prefill_bwd_dq_kernel(const 
     }
 
     if (tid < kC + 2) {
-        const double ld = static_cast<double>(lam);
-        sPw[tid] = static_cast<float>(pow(ld, static_cast<double>(tid)));
-        double ps = 0.0, pm = 1.0;
-        for (int m = 0; m < tid; ++m, pm *= ld) ps += pm;
-        sPs[tid] = static_cast<float>(ps);
+        const PowSum t = pow_sum(lam, tid);
+        sPw[tid] = static_cast<float>(t.p);
+        sPs[tid] = static_cast<float>(t.s);
     }
     constexpr bool din = DIN;  // (then G == 1: the S*p are state_in)
 
@@ -536,7 +534,7 @@ __global__ __launch_bounds__(512, DIN ? 2 : 4) void prefill_bwd_dq_kernel(const 
     for (int c = c_begin; c < c_end; ++c) {
         const int nvalid = min(kC, a.L - c * kC);
         // (din) l^(64 c): the incoming state's decay to the chunk's start
-        const float lc = din ? static_cast<float>(pow(static_cast<double>(lam), 64.0 * c)) : 0.f;
+        const float lc = din ? static_cast<float>(int_pow(lam, int64_t{kC} * c)) : 0.f;
         __syncthreads();  // tiles of chunk c and M_c in LDS
         // ---- scores S^T[j][iw] (blocks jb <= w), masked: A = l^(i-j) (1 + phi_q . phi_k)
         f32x4 sT[4];
@@ -721,9 +719,9 @@ __global__ __launch_bounds__(DUAL ? 256 : 512, DUAL ? 2 : 4) void prefill_bwd_dk
     const size_t so1 = static_cast<size_t>(seq) * kD * kD, so0 = static_cast<size_t>(seq) * kD;
     float *slot = a.G > 1 ? a.ws + static_cast<size_t>(unit) * kWsStride : nullptr;
 
-    if (tid < kC + 2) sPw[tid] = static_cast<float>(pow(static_cast<double>(lam), static_cast<double>(tid)));
+    if (tid < kC + 2) sPw[tid] = static_cast<float>(pow_sum(lam, tid).p);
     if (tid < kC) {
-        const float om = static_cast<float>(pow(static_cast<double>(lam), static_cast<double>(tid + 1)));
+        const float om = static_cast<float>(pow_sum(lam, tid + 1).p);
         sOm[tid] = om;
         const uint16_t hi = f32_to_bf16_bits(om);
         const float r1 = om - bf16_bits_to_f32(hi);
@@ -1071,8 +1069,8 @@ __global__ __launch_bounds__(256) void bwd_dual_scan_kernel(const BwdArgs a) {
     // (selective: segment s's own log2 decay, beside its slot's state)
     const bool sel = a.logd != nullptr;
     const double ld = sel ? 1.0 : static_cast<double>(a.decay[h]);
-    const float lT = sel ? 0.f : static_cast<float>(pow(ld, static_cast<double>(a.cps) * kC));
-    const float lLast = sel ? 0.f : static_cast<float>(pow(ld, static_cast<double>(a.L - (a.G - 1) * a.cps * kC)));
+    const float lT = sel ? 0.f : static_cast<float>(int_pow(ld, int64_t{kC} * a.cps));
+    const float lLast = sel ? 0.f : static_cast<float>(int_pow(ld, a.L - (a.G - 1) * a.cps * kC));
     const float f2 = sel ? 1.0f : 2.0f;  // the kernels' factor on the second-order adjoints
     const size_t so1 = static_cast<size_t>(seq) * kD * kD, so0 = static_cast<size_t>(seq) * kD;
     // the element's place in the reference state, and the factor of this kernel's convention

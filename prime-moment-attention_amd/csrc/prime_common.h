@@ -80,6 +80,37 @@ __device__ __forceinline__ float xor_lane(float x) {
     }
 }
 
+// l^n by squaring, in fp64 (relative error about n 2^-53: far below the fp32
+// rounding that follows).  pow() costs a few hundred dependent fp64 instructions,
+// a good part of a short launch's prologue.
+__device__ __forceinline__ double int_pow(double l, int64_t n) {
+    double r = 1.0;
+    for (; n > 0; n >>= 1, l *= l)
+        if (n & 1) r *= l;
+    return r;
+}
+
+// l^n (p) and sum_{m<n} l^m (s), n < 128, in seven steps of doubling: n -> 2n is
+// s -> s + p s, p -> p^2.  Every term is positive, so near l = 1 nothing cancels
+// (a closed form would).  With pow() and a loop over m, 8 x 12 x 8192 bf16 took
+// 188.9 us, now 181.8; forward and backward of 8 x 12 x 1000 fp32 406, now 389.
+struct PowSum {
+    double p, s;
+};
+__device__ __forceinline__ PowSum pow_sum(double l, int n) {
+    PowSum r{1.0, 0.0};
+#pragma unroll
+    for (int bit = 6; bit >= 0; --bit) {
+        r.s = fma(r.s, r.p, r.s);
+        r.p *= r.p;
+        if (n >> bit & 1) {
+            r.s += r.p;
+            r.p *= l;
+        }
+    }
+    return r;
+}
+
 // x + x of lane (lane ^ 16), or (lane ^ 32), on the VALU: a v_permlane16_swap /
 // v_permlane32_swap of x with itself leaves, in every lane, its own x in one
 // result and its partner's in the other, so their sum is the pair's sum.
