@@ -1109,8 +1109,32 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
     const int NC = (L + kC - 1) / kC;
     int g = 1;
     const int cu = device_cus();
-    if (S > 0 && S < per_cu * cu) g = min(min(per_cu * cu / S, NC / 8), 64);
-    if (per_cu == 1 && S > 0) {
+    if (per_cu == 2 && S > 0) {
+        // bf16 passes, two workgroups per CU, in microseconds: a round of up to one
+        // workgroup per CU costs 8 and 7.8 a chunk (both passes), of up to two 8 and 11;
+        // segments add 16 for the scans and launches, 3 a chunk for the state-only and
+        // dual passes (three units per CU before they slow each other) and 0.04 a slot.
+        // Fitted to 15 shapes from 12 x 128 to 96 x 8192 with every count; the choice is
+        // within 1 % of the best in each.  12 x 512: 8 segments 38 us, one 71; 12 x 1000:
+        // 16 49, 2 107; 48 x 777: 7 70, one 111; 200 x 1024: one 138, 2 166.
+        auto cost = [&](int u, int c) {
+            const int64_t units = static_cast<int64_t>(S) * u, full = units / (2 * cu), rem = units % (2 * cu);
+            double t = static_cast<double>(full) * (8.0 + 11.0 * c);
+            if (rem) t += 8.0 + (rem <= cu ? 7.8 : 11.0) * c;
+            if (u > 1)
+                t += 16.0 + 3.0 * c * max(1.0, static_cast<double>(units) / (3.0 * cu)) +
+                     0.04 * static_cast<double>(units);
+            return t;
+        };
+        double best = cost(1, NC);
+        for (int t = 2; t <= min(NC, 64); ++t) {
+            const int c = (NC + t - 1) / t, u = (NC + c - 1) / c;
+            if (cost(u, c) < best - 1e-9) {
+                best = cost(u, c);
+                g = u;
+            }
+        }
+    } else if (S > 0) {
         // fp32 passes, one workgroup per CU: in periods of a chunk of the dq or dk/dv
         // pass (16-18 us each), a round of units over the CUs costs 2 a chunk, with
         // segments 2.6 (the state-only and dual passes) and about 1.2 for the two scans

@@ -229,9 +229,8 @@ constexpr int kBwdCorr = 132;  // floats per sequence in BwdArgs::kcorr (128 fea
 hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream);
 // fp32 inputs: the fp32 dq and dk/dv passes (chunk_f32.hip)
 hipError_t launch_prefill_backward_f32(const BwdArgs &a, hipStream_t stream);
-// segments per sequence for the backward: enough (sequence, segment) units to
-// fill per_cu workgroups per CU (2 for the bf16 passes, of at least 8 chunks a
-// segment; 1 for the fp32 ones, by their passes' costs)
+// segments per sequence for the backward, by the passes' measured costs: per_cu 2
+// for the bf16 passes, 1 for the fp32 ones (workgroups per CU)
 void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu = 2);
 // the reverse scan over segments of the backward's dual states (prefill_bwd.hip)
 hipError_t launch_bwd_dual_scan(const BwdArgs &a, hipStream_t stream);

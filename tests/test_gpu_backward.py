@@ -403,3 +403,28 @@ def test_backward_row_alignment_and_dy_dtype(L, dense_state):
             print(f"[backward rows] L={L} {gdtype} dy {dydtype} pitch {pitch}", flush=True)
             for x, y in zip(ref, run(gdtype, dydtype, pitch)):
                 assert torch.isfinite(x.float()).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("L", [129, 256, 513, 1000])
+def test_backward_short_segments_equal_one_segment(L):
+    """The bf16 plan splits down to one chunk per segment (a ragged last one too):
+    against one segment per sequence (minimum workspace), with an incoming state and
+    a final-state adjoint; the tolerance of the segmented test of longer sequences."""
+    B, H = 1, 6
+    q, k, v = (to_dev(x, torch.bfloat16) for x in O.make_inputs((B, H, L, D), seed=520, bf16=True))
+    dy = to_dev(np.random.default_rng(521).standard_normal((B, H, L, D)).astype(np.float32), torch.bfloat16)
+    lam = to_dev(np.linspace(0.99, 0.9999, H).astype(np.float32))
+    st0 = state_to_dev(random_state(B * H, D, 522), B, H, D)
+    ds = state_to_dev(random_state(B * H, D, 523), B, H, D)
+    small = (B * H * L * 8 + 255) // 256 * 256
+    outs = []
+    for nbytes in (_lib.backward_workspace_size(B, H, L), small):
+        g = [torch.empty(B, H, L, D, device=dev()) for _ in range(3)]
+        dsi = _lib.new_state(B, H, D, dev())
+        _lib.chunked_prefill_backward(q, k, v, lam, 1.0, st0, dy, ds, *g, dsi,
+                                      workspace=torch.empty(nbytes, dtype=torch.uint8, device=dev()))
+        torch.cuda.synchronize()
+        outs.append(([to_np(x) for x in g], state_to_np(dsi, B * H, D)))
+    for x, y, n in zip(outs[0][0], outs[1][0], ("dq", "dk", "dv")):
+        assert_close(x, y, 5e-3, n)
+    assert_state_close(outs[0][1], outs[1][1], 5e-3, "dstate_in")
