@@ -48,6 +48,8 @@
 // A operand for row i with that same K permutation.  Every MFMA runs under
 // wave-uniform control flow.
 
+#include <algorithm>
+
 #include "prefill_common.h"
 
 namespace prime {
@@ -1113,7 +1115,7 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
         // bf16 passes, two workgroups per CU, in microseconds: a round of up to one
         // workgroup per CU costs 8 and 7.8 a chunk (both passes), of up to two 8 and 11;
         // segments add 16 for the scans and launches, 3 a chunk for the state-only and
-        // dual passes (three units per CU before they slow each other) and 0.04 a slot.
+        // dual passes (two units per CU before they slow each other) and 0.04 a slot.
         // Fitted to 15 shapes from 12 x 128 to 96 x 8192 with every count; the choice is
         // within 1 % of the best in each.  12 x 512: 8 segments 38 us, one 71; 12 x 1000:
         // 16 49, 2 107; 48 x 777: 7 70, one 111; 200 x 1024: one 138, 2 166.
@@ -1122,7 +1124,7 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
             double t = static_cast<double>(full) * (8.0 + 11.0 * c);
             if (rem) t += 8.0 + (rem <= cu ? 7.8 : 11.0) * c;
             if (u > 1)
-                t += 16.0 + 3.0 * c * max(1.0, static_cast<double>(units) / (3.0 * cu)) +
+                t += 16.0 + 3.0 * c * std::max(1.0, static_cast<double>(units) / (2.0 * cu)) +
                      0.04 * static_cast<double>(units);
             return t;
         };
