@@ -522,9 +522,10 @@ ROWS_LINEAR_MAX = 512
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``rows_linear`` takes x [..., K] and w [N, K]: few bf16 rows of the sizes
     measured, 16-byte rows, plain dense tensors of one device, and nothing recording or
-    recasting (autograd, autocast)."""
+    recasting (autograd, autocast).  An x of another width is left to torch, which
+    refuses it."""
     K = x.shape[-1]
-    return (x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.is_cuda and w.device == x.device
+    return (w.shape[1] == K and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.is_cuda and w.device == x.device
             and 0 < x.numel() <= ROWS_LINEAR_MAX * K and K % 128 == 0 and K <= 1024 and w.shape[0] % 32 == 0
             and w.shape[0] <= 3072 and x.is_contiguous() and w.is_contiguous()
             and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)

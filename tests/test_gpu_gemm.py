@@ -385,3 +385,21 @@ def test_module_output_projection_keeps_hooks_and_replacements():
         assert len(seen) == 1 and torch.allclose(y.float(), y2.float(), atol=2 ** -7)
         m.o_proj = torch.nn.Sequential(m.o_proj, torch.nn.ReLU())
         assert (m(x)[0] >= 0).all()
+
+
+@pytest.mark.parametrize("width", [256, 512, 1024])
+def test_module_refuses_inputs_of_another_width(width):
+    """An input whose last dimension is not the weights' is not taken by the few-row
+    kernel (its row count would be the elements over the weights' width) and raises as
+    nn.Linear does, in the projections and in o_proj."""
+    from prime_moment_attention import PrimeMomentAttention
+    from prime_moment_attention.attention import project_out
+    m = PrimeMomentAttention(128, 2, 64).to(dev(), torch.bfloat16).requires_grad_(False)
+    x = torch.randn(1, 8, width, device=dev(), dtype=torch.bfloat16)
+    narrow = torch.randn(1, 8, 128, device=dev(), dtype=torch.bfloat16)
+    wide = torch.zeros(128, width, device=dev(), dtype=torch.bfloat16)
+    assert not _lib.rows_linear_ok(x, m.o_proj.weight) and not _lib.rows_linear_ok(narrow, wide)
+    with pytest.raises(RuntimeError):
+        m(x)
+    with pytest.raises(RuntimeError):
+        project_out(m.o_proj, x)
