@@ -85,15 +85,24 @@ def project_qkv(mod: nn.Module, hidden_states: torch.Tensor):
     return qkv[:, :H], qkv[:, H:H + Hk], qkv[:, H + Hk:]
 
 
-def _has_hooks(m: nn.Module) -> bool:
+_LINEAR_FORWARD = nn.Linear.forward
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """Whether m(x) is x @ weight.T and nothing else: an nn.Linear without bias or hooks
+    whose ``forward`` nobody has replaced, on the instance (offloading, adapter and
+    quantisation wrappers do) or on the class."""
     g = torch.nn.modules.module
-    return bool(m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks or g._global_forward_pre_hooks)
+    return (type(m) is nn.Linear and m.bias is None and "forward" not in m.__dict__
+            and nn.Linear.forward is _LINEAR_FORWARD
+            and not (m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks
+                     or g._global_forward_pre_hooks))
 
 
 def project_out(proj: nn.Module, y: torch.Tensor) -> torch.Tensor:
     """``proj(y)``: for few rows through the row kernel, where the module is a plain
-    nn.Linear without bias or hooks."""
-    if type(proj) is nn.Linear and proj.bias is None and not _has_hooks(proj) and _lib.rows_linear_ok(y, proj.weight):
+    nn.Linear and torch has nothing to record or transform."""
+    if _plain_linear(proj) and _lib.rows_linear_ok(y, proj.weight):
         return _lib.rows_linear(y, proj.weight)
     return proj(y)
 

@@ -403,3 +403,20 @@ def test_module_refuses_inputs_of_another_width(width):
         m(x)
     with pytest.raises(RuntimeError):
         project_out(m.o_proj, x)
+
+
+def test_output_projection_keeps_a_replaced_forward(monkeypatch):
+    """A ``forward`` set on the instance or the class runs at few rows as at many."""
+    from prime_moment_attention import PrimeMomentAttention
+    m = PrimeMomentAttention(128, 2, 64).to(dev(), torch.bfloat16).requires_grad_(False)
+    w = m.o_proj.weight
+    for rows in (8, 600):
+        x = torch.randn(1, rows, 128, device=dev(), dtype=torch.bfloat16)
+        plain, _ = m(x)
+        m.o_proj.forward = lambda y: torch.nn.functional.linear(y, w) * 0 + 3
+        assert (m(x)[0] == 3).all(), rows
+        del m.o_proj.forward
+        with monkeypatch.context() as mp:
+            mp.setattr(torch.nn.Linear, "forward", lambda self, y: torch.nn.functional.linear(y, w) * 0 + 4)
+            assert (m(x)[0] == 4).all(), rows
+        assert torch.equal(m(x)[0], plain)
