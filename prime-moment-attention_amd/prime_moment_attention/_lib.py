@@ -11,6 +11,7 @@ import os
 from typing import Optional, Sequence, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libprime_mi355x.so")
@@ -519,19 +520,29 @@ def linear_fused(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, epilogue: 
 ROWS_LINEAR_MAX = 512
 
 
+def plain_eager(*ts: torch.Tensor) -> bool:
+    """Whether torch would only compute an operation over ts: no autograd recording, no
+    forward-mode level or functorch transform (their tensors look plain), no dispatch or
+    function mode, tracer or autocast that has to see the call.  (1.3 us)"""
+    C = torch._C
+    return (not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+            and forward_ad._current_level < 0 and C._functorch.peek_interpreter_stack() is None
+            and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
+            and C._get_tracing_state() is None and not torch.compiler.is_compiling()
+            and not torch.is_autocast_enabled())
+
+
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``rows_linear`` takes x [..., K] and w [N, K]: few bf16 rows of the sizes
-    measured, 16-byte rows, plain dense tensors of one device, and nothing recording or
-    recasting (autograd, autocast).  An x of another width is left to torch, which
-    refuses it."""
+    measured, 16-byte rows, plain dense tensors of one device, and nothing recording,
+    transforming or recasting the call (``plain_eager``).  An x of another width is left to
+    torch, which refuses it."""
     K = x.shape[-1]
     return (w.shape[1] == K and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.is_cuda and w.device == x.device
             and 0 < x.numel() <= ROWS_LINEAR_MAX * K and K % 128 == 0 and K <= 1024 and w.shape[0] % 32 == 0
             and w.shape[0] <= 3072 and x.is_contiguous() and w.is_contiguous()
             and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
-            and not torch.is_autocast_enabled())
+            and plain_eager(x, w) and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

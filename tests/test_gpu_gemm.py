@@ -420,3 +420,44 @@ def test_output_projection_keeps_a_replaced_forward(monkeypatch):
             mp.setattr(torch.nn.Linear, "forward", lambda self, y: torch.nn.functional.linear(y, w) * 0 + 4)
             assert (m(x)[0] == 4).all(), rows
         assert torch.equal(m(x)[0], plain)
+
+
+def test_output_projection_under_transforms():
+    """Forward-mode tangents, torch.func transforms and dispatch modes reach the output
+    projection at few rows as they reach nn.Linear."""
+    from torch.autograd import forward_ad as fwd
+    from torch.utils.flop_counter import FlopCounterMode
+    from prime_moment_attention.attention import project_out
+    proj = torch.nn.Linear(128, 64, bias=False).to(dev(), torch.bfloat16).requires_grad_(False)
+    y = torch.randn(1, 8, 128, device=dev(), dtype=torch.bfloat16)
+    t = torch.randn(64, 128, device=dev(), dtype=torch.bfloat16)
+    want = torch.nn.functional.linear(y, t)
+    w0 = proj.weight.detach().clone()
+    assert _lib.rows_linear_ok(y, w0)
+    with fwd.dual_level():
+        assert not _lib.rows_linear_ok(y, fwd.make_dual(w0, t))
+        del proj._parameters["weight"]
+        proj.weight = fwd.make_dual(w0, t)
+        tangent = fwd.unpack_dual(project_out(proj, y)).tangent
+        assert tangent is not None and torch.equal(tangent, want)
+    del proj.weight
+    proj.weight = torch.nn.Parameter(w0, requires_grad=False)
+    call = lambda w: torch.func.functional_call(_Out(proj), {"p.weight": w}, (y,))
+    _, tangent = torch.func.jvp(call, (w0,), (t,))
+    assert torch.equal(tangent, want)
+    taken = []  # (the rule alone: vmap's batched product has a transposed bf16 operand)
+    torch.func.vmap(lambda w: (taken.append(_lib.rows_linear_ok(y, w)), w * 1)[1])(torch.stack([w0, t]))
+    assert taken == [False]
+    with FlopCounterMode(display=False) as fc:
+        project_out(proj, y)
+    assert fc.get_total_flops() == 2 * 8 * 128 * 64
+
+
+class _Out(torch.nn.Module):
+    def __init__(self, p):
+        super().__init__()
+        self.p = p
+
+    def forward(self, y):
+        from prime_moment_attention.attention import project_out
+        return project_out(self.p, y)
