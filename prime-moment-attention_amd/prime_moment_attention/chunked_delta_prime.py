@@ -128,23 +128,20 @@ class ChunkedGatedDeltaPrimeAttention(nn.Module):
         nn.init.constant_(self.write_proj.bias, -1.0)
 
     def gates(self, hidden_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-        """(beta, alpha) fp32 [B, H, L] (chunked_delta_prime.py:110-111, 133-137)."""
+        """(beta, alpha) fp32 [B, H, L] (chunked_delta_prime.py:110-111, 133-137): torch ops
+        where autograd records or transforms them, else one kernel (prime_delta_gates)."""
         B, L, _ = hidden_states.shape
         H, D = self.num_heads, self.head_dim
-        b = torch.sigmoid(self.erase_proj(hidden_states)).view(B, L, H, D).float().mean(-1)
-        w = torch.sigmoid(self.write_proj(hidden_states)).view(B, L, H, D).float().mean(-1)
+        erase, write = self.erase_proj(hidden_states), self.write_proj(hidden_states)
+        if (type(erase) is type(write) is torch.Tensor and erase.is_cuda and _lib.plain_eager(erase, write)
+                and erase.dtype in (torch.float32, torch.bfloat16, torch.float16) and write.dtype == erase.dtype
+                and erase.stride(2) == 1 and write.stride(2) == 1):
+            return _lib.delta_gates(erase, write, self.decay, H, D)
+        b = torch.sigmoid(erase).view(B, L, H, D).float().mean(-1)
+        w = torch.sigmoid(write).view(B, L, H, D).float().mean(-1)
         beta = (w * 0.5).transpose(1, 2).contiguous()
         alpha = (self.decay * (1.0 - b * 0.5)).transpose(1, 2).contiguous()
         return beta, alpha
-
-    def _gates_inference(self, hidden_states: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-        """``gates`` without autograd: the projections, then one kernel
-        (prime_delta_gates) instead of its elementwise passes and means."""
-        erase, write = self.erase_proj(hidden_states), self.write_proj(hidden_states)
-        if (not erase.is_cuda or erase.dtype not in (torch.float32, torch.bfloat16, torch.float16)
-                or write.dtype != erase.dtype or erase.stride(2) != 1 or write.stride(2) != 1):
-            return self.gates(hidden_states)
-        return _lib.delta_gates(erase, write, self.decay, self.num_heads, self.head_dim)
 
     def project(self, hidden_states: torch.Tensor):
         """q (scaled), k, v as [B, H(kv), L, D] (chunked_delta_prime.py:105-126)."""
@@ -168,7 +165,7 @@ class ChunkedGatedDeltaPrimeAttention(nn.Module):
                                                   (state is not None and state.requires_grad)):
             return self._forward_train(hidden_states, state, return_state)
         q, k, v = self.project(hidden_states)
-        beta, alpha = self._gates_inference(hidden_states)
+        beta, alpha = self.gates(hidden_states)
         if q.dtype not in (torch.bfloat16, torch.float32):
             q, k, v = q.float(), k.float(), v.float()
         y_dtype = dtype if dtype in (torch.float32, torch.bfloat16, torch.float16) else torch.float32

@@ -317,3 +317,38 @@ def test_delta_gates_match_module_ops(dtype, B, H, L, D, offset):
     tol = {torch.float32: 2e-7, torch.bfloat16: 2e-7 + 2.0 ** -9 / D, torch.float16: 2e-7 + 2.0 ** -12 / D}[dtype]
     assert (beta - rb).abs().max().item() <= tol
     assert (alpha - ra).abs().max().item() <= tol
+
+
+def test_module_gates_override_runs_in_inference():
+    """An overridden ``gates`` (subclass or instance) gives the rates of inference as of
+    training, prefill and step; called directly it is differentiable in forward mode."""
+    from torch.autograd import forward_ad as fwd
+    from prime_moment_attention import ChunkedGatedDeltaPrimeAttention as M
+
+    class Sub(M):
+        def gates(self, x):
+            beta, alpha = super().gates(x)
+            return beta * 0.25, alpha * 0.5
+
+    torch.manual_seed(1)
+    base = M(128, 2, 64, decay=0.99).to(dev())
+    sub = Sub(128, 2, 64, decay=0.99).to(dev())
+    sub.load_state_dict(base.state_dict())
+    inst = M(128, 2, 64, decay=0.99).to(dev())
+    inst.load_state_dict(base.state_dict())
+    inst.gates = lambda x: Sub.gates(sub, x)
+    for L in (1, 70):
+        x = torch.randn(2, L, 128, device=dev())
+        with torch.no_grad():
+            y, ys, yi = base(x)[0], sub(x)[0], inst(x)[0]
+        trained = sub(x)[0].detach()  # autograd records through the parameters
+        assert torch.equal(ys, yi)
+        # fp32 on both sides, the gates by a kernel or by torch ops
+        assert_close(to_np(ys), to_np(trained), 1e-4, "inference against training")
+        assert (ys - y).abs().max() > 1e-2 * y.abs().max()
+    base.requires_grad_(False)
+    x, t = torch.randn(2, 2, 9, 128, device=dev())
+    with fwd.dual_level():
+        beta, alpha = base.gates(fwd.make_dual(x, t))
+        tb, ta = fwd.unpack_dual(beta).tangent, fwd.unpack_dual(alpha).tangent
+    assert tb is not None and ta is not None and tb.abs().max() > 0 and ta.abs().max() > 0
