@@ -356,7 +356,7 @@ int prime_delta_gates(const void *erase, int64_t erase_sb, int64_t erase_sl, con
         return fail(PRIME_ERR_INVALID_ARG, "bad sizes B=%d H=%d L=%d or negative strides", B, H, L);
     if (D < 1 || D > prime::kD) return fail(PRIME_ERR_UNSUPPORTED_DIM, "head dim %d unsupported (1 .. %d)", D, prime::kD);
     if (!valid_dtype(dtype)) return fail(PRIME_ERR_UNSUPPORTED_DTYPE, "unsupported gate dtype");
-    if (B > 65535 || (H + 3) / 4 > 65535) return fail(PRIME_ERR_INVALID_ARG, "B=%d or H=%d above the grid's limit", B, H);
+    if ((H + 3) / 4 > 65535) return fail(PRIME_ERR_INVALID_ARG, "H=%d above the grid's limit", H);
     const int64_t es = elem_size(dtype);
     if (reinterpret_cast<uintptr_t>(erase) % es || reinterpret_cast<uintptr_t>(write) % es ||
         (reinterpret_cast<uintptr_t>(beta) & 3) || (reinterpret_cast<uintptr_t>(alpha) & 3))

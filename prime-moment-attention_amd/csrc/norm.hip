@@ -6,6 +6,8 @@
 // fp32).  All loads of a row are issued before the first store, so a row costs
 // one memory round trip for x/delta/weight and one for the stores.
 
+#include <algorithm>
+
 #include "prime_kernels.h"
 
 namespace prime {
@@ -343,15 +345,12 @@ constexpr int kGateTok = 64, kGateHeads = 4;
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict__ erase, const void *__restrict__ write,
                                                           int64_t e_sb, int64_t e_sl, int64_t w_sb, int64_t w_sl,
-                                                          float decay, int H, int L, int D, float *__restrict__ beta,
-                                                          float *__restrict__ alpha) {
+                                                          float decay, int B, int H, int L, int D,
+                                                          float *__restrict__ beta, float *__restrict__ alpha) {
     __shared__ float sSum[2][kGateHeads][kGateTok + 1];
     constexpr int ES = DT == PRIME_F32 ? 4 : 2;
     const int tid = threadIdx.x, part = tid & 7;
     const int t0 = blockIdx.x * kGateTok, h0 = blockIdx.y * kGateHeads;
-    const int64_t b = blockIdx.z;
-    const char *eb = static_cast<const char *>(erase) + (b * e_sb + static_cast<int64_t>(t0) * e_sl) * ES;
-    const char *wb = static_cast<const char *>(write) + (b * w_sb + static_cast<int64_t>(t0) * w_sl) * ES;
     const int nt = min(kGateTok, L - t0), nh = min(kGateHeads, H - h0);
     auto sig = [](float x) {
         if constexpr (DT == PRIME_F32) return 1.0f / (1.0f + expf(-x));
@@ -376,50 +375,56 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict
         }
         return a;
     };
-    // row rr = 4 token + head: 8 rounds of 32 rows
+    for (int64_t b = blockIdx.z; b < B; b += gridDim.z) {
+        const char *eb = static_cast<const char *>(erase) + (b * e_sb + static_cast<int64_t>(t0) * e_sl) * ES;
+        const char *wb = static_cast<const char *>(write) + (b * w_sb + static_cast<int64_t>(t0) * w_sl) * ES;
+        // row rr = 4 token + head: 8 rounds of 32 rows
 #pragma unroll 4
-    for (int it = 0; it < kGateTok * kGateHeads / 32; ++it) {
-        const int rr = it * 32 + (tid >> 3), tk = rr / kGateHeads, hh = rr % kGateHeads;
-        const int64_t t = min(tk, nt - 1), h = h0 + min(hh, nh - 1);
-        const char *pe = eb + (t * e_sl + h * D) * ES, *pw = wb + (t * w_sl + h * D) * ES;
-        float se = 0.f, sw = 0.f;
-        if constexpr (VEC) {
-            u32x4 re[DT == PRIME_F32 ? 2 : 1], rw[DT == PRIME_F32 ? 2 : 1];
+        for (int it = 0; it < kGateTok * kGateHeads / 32; ++it) {
+            const int rr = it * 32 + (tid >> 3), tk = rr / kGateHeads, hh = rr % kGateHeads;
+            const int64_t t = min(tk, nt - 1), h = h0 + min(hh, nh - 1);
+            const char *pe = eb + (t * e_sl + h * D) * ES, *pw = wb + (t * w_sl + h * D) * ES;
+            float se = 0.f, sw = 0.f;
+            if constexpr (VEC) {
+                u32x4 re[DT == PRIME_F32 ? 2 : 1], rw[DT == PRIME_F32 ? 2 : 1];
 #pragma unroll
-            for (int i = 0; i < (DT == PRIME_F32 ? 2 : 1); ++i) {
-                re[i] = reinterpret_cast<const u32x4 *>(pe + 8 * part * ES)[i];
-                rw[i] = reinterpret_cast<const u32x4 *>(pw + 8 * part * ES)[i];
+                for (int i = 0; i < (DT == PRIME_F32 ? 2 : 1); ++i) {
+                    re[i] = reinterpret_cast<const u32x4 *>(pe + 8 * part * ES)[i];
+                    rw[i] = reinterpret_cast<const u32x4 *>(pw + 8 * part * ES)[i];
+                }
+                se = row_sum8(re);
+                sw = row_sum8(rw);
+            } else {
+                for (int d = part; d < D; d += 8) {
+                    se += sig(load_elem(pe, d, DT));
+                    sw += sig(load_elem(pw, d, DT));
+                }
             }
-            se = row_sum8(re);
-            sw = row_sum8(rw);
-        } else {
-            for (int d = part; d < D; d += 8) {
-                se += sig(load_elem(pe, d, DT));
-                sw += sig(load_elem(pw, d, DT));
+            se += xor_lane<1>(se);
+            sw += xor_lane<1>(sw);
+            se += xor_lane<2>(se);
+            sw += xor_lane<2>(sw);
+            se += xor_lane<4>(se);
+            sw += xor_lane<4>(sw);
+            if (part == 0) {
+                sSum[0][hh][tk] = se / static_cast<float>(D);
+                sSum[1][hh][tk] = sw / static_cast<float>(D);
             }
         }
-        se += xor_lane<1>(se);
-        sw += xor_lane<1>(sw);
-        se += xor_lane<2>(se);
-        sw += xor_lane<2>(sw);
-        se += xor_lane<4>(se);
-        sw += xor_lane<4>(sw);
-        if (part == 0) {
-            sSum[0][hh][tk] = se / static_cast<float>(D);
-            sSum[1][hh][tk] = sw / static_cast<float>(D);
+        __syncthreads();
+        const int tk = tid & 63, hh = tid >> 6;
+        if (tk < nt && hh < nh) {
+            const int64_t o = (b * H + h0 + hh) * L + t0 + tk;
+            beta[o] = sSum[1][hh][tk] * 0.5f;
+            alpha[o] = decay * (1.0f - sSum[0][hh][tk] * 0.5f);
         }
-    }
-    __syncthreads();
-    const int tk = tid & 63, hh = tid >> 6;
-    if (tk < nt && hh < nh) {
-        const int64_t o = (b * H + h0 + hh) * L + t0 + tk;
-        beta[o] = sSum[1][hh][tk] * 0.5f;
-        alpha[o] = decay * (1.0f - sSum[0][hh][tk] * 0.5f);
+        __syncthreads();
     }
 }
 
 hipError_t launch_delta_gates(const DeltaGateArgs &a, hipStream_t stream) {
-    const dim3 g((a.L + kGateTok - 1) / kGateTok, (a.H + kGateHeads - 1) / kGateHeads, a.B), blk(256);
+    // (a grid's z ends at 65,535: workgroups take further sequences in turn)
+    const dim3 g((a.L + kGateTok - 1) / kGateTok, (a.H + kGateHeads - 1) / kGateHeads, std::min(a.B, 65535)), blk(256);
     auto al = [](const void *p, int64_t sb, int64_t sl, int64_t es) {
         return reinterpret_cast<uintptr_t>(p) % 16 == 0 && sb * es % 16 == 0 && sl * es % 16 == 0;
     };
@@ -427,7 +432,7 @@ hipError_t launch_delta_gates(const DeltaGateArgs &a, hipStream_t stream) {
     const bool vec = a.D == 64 && al(a.erase, a.e_sb, a.e_sl, es) && al(a.write, a.w_sb, a.w_sl, es);
 #define PRIME_GATES(DT, V)                                                                                          \
     hipLaunchKernelGGL((delta_gates_kernel<DT, V>), g, blk, 0, stream, a.erase, a.write, a.e_sb, a.e_sl, a.w_sb,    \
-                       a.w_sl, a.decay, a.H, a.L, a.D, a.beta, a.alpha)
+                       a.w_sl, a.decay, a.B, a.H, a.L, a.D, a.beta, a.alpha)
     if (a.dt == PRIME_BF16) { if (vec) PRIME_GATES(PRIME_BF16, true); else PRIME_GATES(PRIME_BF16, false); }
     else if (a.dt == PRIME_F16) { if (vec) PRIME_GATES(PRIME_F16, true); else PRIME_GATES(PRIME_F16, false); }
     else { if (vec) PRIME_GATES(PRIME_F32, true); else PRIME_GATES(PRIME_F32, false); }

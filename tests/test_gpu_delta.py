@@ -352,3 +352,20 @@ def test_module_gates_override_runs_in_inference():
         beta, alpha = base.gates(fwd.make_dual(x, t))
         tb, ta = fwd.unpack_dual(beta).tangent, fwd.unpack_dual(alpha).tangent
     assert tb is not None and ta is not None and tb.abs().max() > 0 and ta.abs().max() > 0
+
+
+def test_delta_gates_and_step_beyond_the_grid_z_limit():
+    """A decode batch above 65,535 sequences: the gates of the last sequences equal those
+    of a small call on them, and the module's step takes the batch."""
+    from prime_moment_attention import ChunkedGatedDeltaPrimeAttention
+    B = 65535 + 70
+    g = torch.Generator().manual_seed(3)
+    pre = [torch.randn(B, 1, 16, generator=g).to(dev()) for _ in range(2)]
+    beta, alpha = _lib.delta_gates(pre[0], pre[1], 0.99, 2, 8)
+    for n in (slice(0, 70), slice(65535, B)):
+        b2, a2 = _lib.delta_gates(pre[0][n], pre[1][n], 0.99, 2, 8)
+        assert torch.equal(beta[n], b2) and torch.equal(alpha[n], a2)
+    mod = ChunkedGatedDeltaPrimeAttention(16, 1, 8, decay=0.99).to(dev()).requires_grad_(False)
+    x = torch.randn(B, 1, 16, generator=g).to(dev())
+    y, last = mod(x)[0], mod(x[-70:])[0]
+    assert torch.allclose(y[-70:], last, rtol=1e-4, atol=1e-6)  # (the projections' GEMMs differ in shape)
