@@ -369,3 +369,18 @@ def test_delta_gates_and_step_beyond_the_grid_z_limit():
     x = torch.randn(B, 1, 16, generator=g).to(dev())
     y, last = mod(x)[0], mod(x[-70:])[0]
     assert torch.allclose(y[-70:], last, rtol=1e-4, atol=1e-6)  # (the projections' GEMMs differ in shape)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_delta_gates_sigmoid_is_torchs_for_every_value(dtype):
+    """Every bf16 / fp16 pattern as a head of one column (the mean is then the sigmoid):
+    the gates are torch's bit for bit, NaN where it is NaN, and 0 where torch's is a
+    subnormal fp32 number (the hardware reciprocal flushes it)."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype).to(dev())
+    beta, alpha = _lib.delta_gates(x.view(1, 512, 128), x.view(1, 512, 128), 0.9995, 128, 1)
+    s = torch.sigmoid(x).float()
+    s = torch.where(s.abs() < 2.0 ** -126, torch.zeros_like(s), s)
+    rb = (s * 0.5).view(1, 512, 128).transpose(1, 2)
+    ra = (0.9995 * (1.0 - s * 0.5)).view(1, 512, 128).transpose(1, 2)
+    for got, want in ((beta, rb), (alpha, ra)):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
