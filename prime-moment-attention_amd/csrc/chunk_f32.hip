@@ -218,8 +218,23 @@ __device__ __forceinline__ void put_rows(const ChunkF32Args &a, const Rows<DP> &
     put_elems<DP>(sV, i, d0, x);
 }
 
+// e^(a + b) for a in whole steps of kLogStep and |b| small: the rounding of the sum is put
+// back as a factor
+__device__ __forceinline__ float exp_sum(float a, float b) {
+    const float d = a + b, e = expf(d), r = b - (d - a);
+    return fabsf(r) < 1.f ? fmaf(e, r, e) : e;  // (not for infinities and NaN)
+}
+
 // The chunk's decays: sEc[i] = e_i, sW[j] = w_j (0 past L), and e_63, sum w in
 // sSc[0], sSc[1]; selective: sCum, the cumulative log decays.  Wave 0.
+//
+// The selective decays are differences of prefix sums, and one strong decay makes every
+// later sum large: in one fp32 number the mild decays after it keep the absolute error of
+// that large sum (1.6e-5 of y with half the tokens at e^-25, against 1e-7 token by token).
+// So each log decay is split at kLogStep = 2^-9: the sums of the steps are exact (at most 64 x
+// 200 < 2^14, 23 bits), those of the rest stay below 2^-3.  sCum holds both, [0, 64) and
+// [64, 128).
+constexpr float kLogStep = 1.0f / 512;
 template <bool SEL>
 __device__ __forceinline__ void put_decays(int nv, int lane, float ld, const float *sPw, float *sCum, float *sEc,
                                            float *sW, float *sSc) {
@@ -227,12 +242,15 @@ __device__ __forceinline__ void put_decays(int nv, int lane, float ld, const flo
     if constexpr (SEL) {
         // (e^-200 is 0 in fp32; -inf would make the differences NaN)
         const float x = lane < nv ? (ld < -200.f ? -200.f : ld) : 0.f;
-        const float cum = wave_prefix_sum(x);
+        const float xs = rintf(x * (1.0f / kLogStep)) * kLogStep;
+        const float cum = wave_prefix_sum(xs), low = wave_prefix_sum(x - xs);
         const float cend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cum), 63));
+        const float lend = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(low), 63));
         sCum[lane] = cum;
-        e = expf(cum);
-        w = lane < nv ? expf(cend - cum) : 0.f;
-        e63 = expf(cend);
+        sCum[kC + lane] = low;
+        e = exp_sum(cum, low);
+        w = lane < nv ? exp_sum(cend - cum, lend - low) : 0.f;
+        e63 = exp_sum(cend, lend);
     } else {
         e = sPw[min(lane + 1, nv)];
         w = lane < nv ? sPw[nv - 1 - lane] : 0.f;
@@ -249,7 +267,7 @@ __device__ __forceinline__ void put_decays(int nv, int lane, float ld, const flo
 
 template <bool SEL>
 __device__ __forceinline__ float decay_ij(int i, int j, const float *sPw, const float *sCum) {
-    if constexpr (SEL) return expf(sCum[i] - sCum[j]);
+    if constexpr (SEL) return exp_sum(sCum[i] - sCum[j], sCum[kC + i] - sCum[kC + j]);
     else return sPw[i - j];
 }
 
@@ -514,7 +532,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     __shared__ __attribute__((aligned(16))) float sV[kC][K::PC];
     __shared__ __attribute__((aligned(16))) float sA[STATE_ONLY ? 1 : kC][kPA];
     __shared__ __attribute__((aligned(16))) float sM[STATE_ONLY ? 1 : K::FP][K::PB];
-    __shared__ float sKf[K::FP], sKin[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sDen[kC], sSc[2];
+    __shared__ float sKf[K::FP], sKin[K::FP], sS0[DP], sPw[kC + 1], sCum[2 * kC], sEc[kC], sW[kC], sDen[kC], sSc[2];
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -647,7 +665,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
     __shared__ __attribute__((aligned(16))) float sG[kC][K::PR];  // dy, then g
     __shared__ __attribute__((aligned(16))) float sA[kC][kPA];    // a, then da
     __shared__ __attribute__((aligned(16))) float sM[K::FP][K::PB];
-    __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sH[kC], sSc[2];
+    __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[2 * kC], sEc[kC], sW[kC], sH[kC], sSc[2];
     __shared__ float sPart[K::ND][kC];
     // dense double clamp: the incoming Kf, l^(64c) times the outer clamp's adjoint, and
     // l^(t+1) times the part of it the inner clamp withholds from the call's tokens
@@ -876,7 +894,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
     __shared__ __attribute__((aligned(16))) float sG[kC][K::PC];
     __shared__ __attribute__((aligned(16))) float sA[kC][kPAt];     // a, then da
     __shared__ __attribute__((aligned(16))) float sM[K::FP][K::PB];  // dM
-    __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[kC], sEc[kC], sW[kC], sH[kC], sEh[kC], sSc[2];
+    __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[2 * kC], sEc[kC], sW[kC], sH[kC], sEh[kC], sSc[2];
     __shared__ float sPp[K::ND][kC], sPc[kC];  // SEL: the feature blocks' parts, the constant feature's
     __shared__ float sFin[kNW];
 

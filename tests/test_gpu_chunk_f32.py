@@ -11,6 +11,7 @@ from oracle import oracle as O
 from prime_moment_attention import _lib
 
 import test_gpu_selective_backward as SB
+from selective_ref import selective_forward
 from gpu_util import dev, random_state, state_to_dev, state_to_np, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -158,3 +159,37 @@ def test_chunk_f32_selective_backward_segments(L, with_state):
         if with_state:
             for x, r in zip(dsi, ref["dstate_in"]):
                 _close(to_np(x), r, "dstate")
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("share", [0.1, 0.5])
+def test_chunk_f32_selective_strong_decays(D, share):
+    """Tokens that decay by e^-25 (the module's Delta <= 50 at tau = 2) among mild ones:
+    the mild decays keep fp32 precision though the chunk's log decays add up to
+    hundreds.  2-norm error against float64; 1e-6 is some tens of fp32 roundings (with a
+    single fp32 prefix sum y is 2e-6 to 6e-6 off here, the state 1e-5).  The log decays'
+    adjoint is a suffix sum whose terms cancel (1e-6 to 4e-6 here): 1e-5."""
+    B, H, L = 2, 2, 130
+    q, k, v, _, rng = _case(B, H, L, D, 300 + D)
+    ld = -rng.uniform(0.001, 0.2, (B, H, L))
+    ld[rng.random((B, H, L)) < share] = -25.0
+    ld, beta = ld.astype(np.float32), rng.uniform(0.6, 2.0, H).astype(np.float32)
+    dy = rng.standard_normal(q.shape).astype(np.float32)
+    t = [torch.from_numpy(x.astype(np.float64)).requires_grad_() for x in
+         (q, k, v, ld, np.broadcast_to(beta, (B, H)).copy())]
+    ref, st_ref = selective_forward(*t, 1.0)
+    (ref * torch.from_numpy(dy.astype(np.float64))).sum().backward()
+    d = [to_dev(x) for x in (q, k, v, ld, beta)]
+    y, st = torch.empty(q.shape, device=dev()), _lib.new_state(B, H, D, dev())
+    _lib.selective_prefill(*d, 1.0, None, y, st)
+    g = [torch.empty(q.shape, device=dev()) for _ in range(3)]
+    dld, dks = torch.empty(B, H, L, device=dev()), torch.empty(B, H, device=dev())
+    _lib.selective_prefill_backward(*d, 1.0, None, to_dev(dy), None, *g, None, dld, dks)
+    torch.cuda.synchronize()
+    err = {}
+    for n, x, r in zip(("y", "S0", "S1", "S2", "K0", "K1", "K2", "dq", "dk", "dv", "dld", "dbeta"),
+                       (y, *st, *g, dld, dks), (ref, *st_ref, *(x.grad for x in t))):
+        r = r.detach().numpy()
+        err[n] = float(np.linalg.norm(to_np(x).astype(np.float64).reshape(r.shape) - r) / np.linalg.norm(r))
+    print({n: f"{e:.1e}" for n, e in err.items()})
+    assert err.pop("dld") < 1e-5 and max(err.values()) < 1e-6, err
