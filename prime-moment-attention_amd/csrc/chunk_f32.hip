@@ -201,21 +201,38 @@ __device__ __forceinline__ void load_rows(const ChunkF32Args &a, int b, int h, i
     if constexpr (SEL)
         if (tid < kWave) R.ld = (a.log_decay + static_cast<size_t>(seq) * a.L + t0)[min(tid, last)];
 }
-// the loaded rows in LDS as fp32 (k times kscale), zero past L and D
-template <int DP, bool VEC, bool STATE_ONLY, int PQ, int PK, int PV>
-__device__ __forceinline__ void put_rows(const ChunkF32Args &a, const Rows<DP> &R, int i, int d0, int nv, float kscale,
-                                         float (*sQ)[PQ], float (*sK)[PK], float (*sV)[PV]) {
-    float x[Dim<DP>::NE];
+// A masked score is 0, and 0 times an infinity or NaN is NaN: the tile on the diagonal, whose
+// product runs over 16 tokens, would carry such a value (or one whose square overflows) to
+// tokens that do not see it.  The sum of squares of the operands of those products tells
+// whether a chunk has one; it then takes the tiles token by token (diag_rows, diag_cols).
+// At D = 64 with vector rows (VEC) it does not.
+template <int DP>
+__device__ __forceinline__ float add_squares(const float (&x)[Dim<DP>::NE], float s) {
+#pragma unroll
+    for (int e = 0; e < Dim<DP>::NE; ++e) s = fmaf(x[e], x[e], s);
+    return s;
+}
+
+// the loaded rows in LDS as fp32 (k times kscale), zero past L and D; the sum of squares of
+// those of q, k and v that SQ names (bits 0, 1, 2)
+template <int DP, bool VEC, bool STATE_ONLY, int SQ, int PQ, int PK, int PV>
+__device__ __forceinline__ float put_rows(const ChunkF32Args &a, const Rows<DP> &R, int i, int d0, int nv, float kscale,
+                                          float (*sQ)[PQ], float (*sK)[PK], float (*sV)[PV]) {
+    float x[Dim<DP>::NE], sq = 0.f;
     if constexpr (!STATE_ONLY) {
         to_f32<DP, VEC>(R.q, VEC ? PRIME_F32 : a.dt_q, d0, a.D, i < nv, x);
         put_elems<DP>(sQ, i, d0, x);
+        if constexpr (!VEC && (SQ & 1)) sq = add_squares<DP>(x, sq);
     }
     to_f32<DP, VEC>(R.k, VEC ? PRIME_F32 : a.dt_k, d0, a.D, i < nv, x);
 #pragma unroll
     for (int e = 0; e < Dim<DP>::NE; ++e) x[e] *= kscale;
     put_elems<DP>(sK, i, d0, x);
+    if constexpr (!VEC && (SQ & 2)) sq = add_squares<DP>(x, sq);
     to_f32<DP, VEC>(R.v, VEC ? PRIME_F32 : a.dt_v, d0, a.D, i < nv, x);
     put_elems<DP>(sV, i, d0, x);
+    if constexpr (!VEC && (SQ & 4)) sq = add_squares<DP>(x, sq);
+    return sq;
 }
 
 // e^(a + b) for a in whole steps of kLogStep and |b| small: the rounding of the sum is put
@@ -488,6 +505,24 @@ __device__ __forceinline__ float k_readout(int i, int part, const float (*sQ)[PQ
     return rd;
 }
 
+// The diagonal tile of block tb token by token: x[r] += sum over j <= tok of a[tok][j] times
+// the row's column 16 xb + 4 g + r ...
+template <int PX, int PA>
+__device__ __forceinline__ void diag_rows(int tb, int xb, int g, int tok, const float (*sX)[PX], const float (*sA)[PA],
+                                          f32x4 &x) {
+    for (int j = 16 * tb; j <= tok; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = fmaf(sA[tok][j], sX[j][16 * xb + 4 * g + r], x[r]);
+}
+// ... or over i >= tok of a[i][tok]
+template <int PX, int PA>
+__device__ __forceinline__ void diag_cols(int tb, int xb, int g, int tok, const float (*sX)[PX], const float (*sA)[PA],
+                                          f32x4 &x) {
+    for (int i = tok; i < 16 * tb + 16; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = fmaf(sA[i][tok], sX[i][16 * xb + 4 * g + r], x[r]);
+}
+
 // num^T tile of (token block tb, value block dv): the state's part (needs no scores) ...
 template <int DP, int PQ, int PM>
 __device__ __forceinline__ f32x4 num_state(int tb, int dv, int g, int c16, float ec, const float (*sQ)[PQ],
@@ -509,10 +544,13 @@ __device__ __forceinline__ f32x4 num_state(int tb, int dv, int g, int c16, float
 // ... and the chunk's values (a is zero above token 16 tb + 15)
 template <int PV, int PA>
 __device__ __forceinline__ f32x4 num_values(int tb, int dv, int g, int c16, const float (*sV)[PV],
-                                            const float (*sA)[PA], f32x4 x) {
+                                            const float (*sA)[PA], f32x4 x, bool bad) {
     const int tok = 16 * tb + c16;
-    pipe<4, Op2>(tb + 1, [&](int s) { return Op2{sV[4 * s + g][16 * dv + c16], sA[tok][4 * s + g]}; },
-                 [&](const Op2 &o) { x = mfma4(o.a, o.b, x); });
+    const int n = bad ? tb : tb + 1;
+    if (n)
+        pipe<4, Op2>(n, [&](int s) { return Op2{sV[4 * s + g][16 * dv + c16], sA[tok][4 * s + g]}; },
+                     [&](const Op2 &o) { x = mfma4(o.a, o.b, x); });
+    if (bad) diag_rows(tb, dv, g, tok, sV, sA, x);
     return x;
 }
 
@@ -533,6 +571,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     __shared__ __attribute__((aligned(16))) float sA[STATE_ONLY ? 1 : kC][kPA];
     __shared__ __attribute__((aligned(16))) float sM[STATE_ONLY ? 1 : K::FP][K::PB];
     __shared__ float sKf[K::FP], sKin[K::FP], sS0[DP], sPw[kC + 1], sCum[2 * kC], sEc[kC], sW[kC], sDen[kC], sSc[2];
+    __shared__ int sBad;  // (!VEC) 1 + the last chunk with an infinite or NaN operand
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -567,11 +606,16 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
     if constexpr (DIN) l64 = int_pow(a.decay[h], kC);
     Rows<DP> R;
     load_rows<DP, VEC, SEL, false, STATE_ONLY>(a, b, h, seq, c_begin, tid, R);
-    if constexpr (!SEL) __syncthreads();  // sPw
+    if constexpr (!VEC) {
+        if (tid == 0) sBad = 0;
+    }
+    if constexpr (!SEL || !VEC) __syncthreads();  // sPw, sBad
     for (int c = c_begin; c < c_end; ++c) {
         const int nv = min(kC, a.L - c * kC);
         if constexpr (!STATE_ONLY) publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
-        put_rows<DP, VEC, STATE_ONLY>(a, R, i, d0, nv, SEL && !a.qk_norm ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        const float sq =
+            put_rows<DP, VEC, STATE_ONLY, 4>(a, R, i, d0, nv, SEL && !a.qk_norm ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        if (!VEC && !(sq < INFINITY)) sBad = c + 1;
         if (w == 0) {
             put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
             if (SEL && STATE_ONLY) seg_ld += wave_sum(lane < nv ? R.ld : 0.f);
@@ -617,7 +661,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_prefill_kernel(const ChunkF32
                 }
                 if (part == 0) sDen[i] = den;
             }
-            if (w < 4 * K::ND) acc = num_values(tb, dv, g, c16, sV, sA, acc);
+            if (w < 4 * K::ND) acc = num_values(tb, dv, g, c16, sV, sA, acc, !VEC && __builtin_amdgcn_readfirstlane(sBad) == c + 1);
             advance<DP>(C, 0.5f, e63, sumw, u, g, c16, tid, sK, sV, sW, sW);
             __syncthreads();
             if (w < 4 * K::ND && tok < nv) {
@@ -671,6 +715,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
     // l^(t+1) times the part of it the inner clamp withholds from the call's tokens
     __shared__ float sKin[K::FP], sHc[kC], sDh[kC];
     __shared__ float sFin[kNW];
+    __shared__ int sBad;  // (!VEC) 1 + the last chunk with an infinite or NaN operand
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -702,7 +747,10 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
     const int tb = w / K::ND, xb = w % K::ND, tok = 16 * tb + c16;  // this wave's unit of num and dFq
     Rows<DP> R;
     load_rows<DP, VEC, SEL, true>(a, b, h, seq, c_begin, tid, R);
-    if constexpr (!SEL) __syncthreads();
+    if constexpr (!VEC) {
+        if (tid == 0) sBad = 0;
+    }
+    if constexpr (!SEL || !VEC) __syncthreads();
     for (int c = c_begin; c < c_end; ++c) {
         const int nv = min(kC, a.L - c * kC);
         {
@@ -710,7 +758,8 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
             to_f32<DP, VEC>(R.dy, a.dt_dy, d0, a.D, i < nv, x);
             put_elems<DP>(sG, i, d0, x);
         }
-        put_rows<DP, VEC, false>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        const float sq = put_rows<DP, VEC, false, 6>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        if (!VEC && !(sq < INFINITY)) sBad = c + 1;
         publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
         if (w == 0) put_decays<SEL>(nv, lane, R.ld, sPw, sCum, sEc, sW, sSc);
         __syncthreads();
@@ -740,7 +789,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
             }
         }
         if (w < 4 * K::ND) {
-            num = num_values(tb, xb, g, c16, sV, sA, num);
+            num = num_values(tb, xb, g, c16, sV, sA, num, !VEC && __builtin_amdgcn_readfirstlane(sBad) == c + 1);
             const f32x4 dy = ld4(&sG[tok][16 * xb + 4 * g]);
             float dot = (dy[0] * num[0] + dy[1] * num[1]) + (dy[2] * num[2] + dy[3] * num[3]);
             dot = sum_lane32(sum_lane16(dot));
@@ -812,11 +861,23 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
         __syncthreads();
         // ---- dFq: the chunk's part -> dq
         if (w < 4 * K::ND) {
-            pipe<4, Op2>(tb + 1, [&](int s) { return Op2{sK[4 * s + g][16 * xb + c16], sA[tok][4 * s + g]}; },
-                         [&](const Op2 &o) {
-                             fx = mfma4(o.a, o.b, fx);
-                             fy = mfma4(0.5f * (o.a * o.a), o.b, fy);
-                         });
+            const bool bad = !VEC && __builtin_amdgcn_readfirstlane(sBad) == c + 1;
+            const int n = bad ? tb : tb + 1;
+            if (n)
+                pipe<4, Op2>(n, [&](int s) { return Op2{sK[4 * s + g][16 * xb + c16], sA[tok][4 * s + g]}; },
+                             [&](const Op2 &o) {
+                                 fx = mfma4(o.a, o.b, fx);
+                                 fy = mfma4(0.5f * (o.a * o.a), o.b, fy);
+                             });
+            if (bad) {
+                diag_rows(tb, xb, g, tok, sK, sA, fx);
+                for (int j = 16 * tb; j <= tok; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float k = sK[j][16 * xb + 4 * g + r];
+                        fy[r] = fmaf(0.5f * (k * k), sA[tok][j], fy[r]);
+                    }
+            }
             if (tok < nv) {
                 const int d = 16 * xb + 4 * g;
                 const f32x4 q = ld4(&sQ[tok][d]);
@@ -897,6 +958,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
     __shared__ float sKf[K::FP], sS0[DP], sPw[kC + 1], sCum[2 * kC], sEc[kC], sW[kC], sH[kC], sEh[kC], sSc[2];
     __shared__ float sPp[K::ND][kC], sPc[kC];  // SEL: the feature blocks' parts, the constant feature's
     __shared__ float sFin[kNW];
+    __shared__ int sBad;  // (!VEC) 1 + the last chunk with an infinite or NaN operand
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -937,7 +999,10 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
         hd = (a.g_den + o)[r];
     };
     load(c_end - 1);
-    if constexpr (!SEL) __syncthreads();
+    if constexpr (!VEC) {
+        if (tid == 0) sBad = 0;
+    }
+    if constexpr (!SEL || !VEC) __syncthreads();
     for (int c = c_end - 1; c >= c_begin; --c) {
         const int nv = min(kC, a.L - c * kC);
         float gr[K::NE];
@@ -945,7 +1010,8 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
 #pragma unroll
         for (int e = 0; e < K::NE; ++e) gr[e] = i < nv ? gr[e] * inv : 0.f;
         put_elems<DP>(sG, i, d0, gr);
-        put_rows<DP, VEC, false>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        const float sq = put_rows<DP, VEC, false, 1>(a, R, i, d0, nv, SEL ? a.k_scale[h] : 1.0f, sQ, sK, sV);
+        if (!VEC && !(add_squares<DP>(gr, sq) < INFINITY)) sBad = c + 1;
         publish<DP>(C, u, g, c16, tid, sM, sKf, sS0);
         if (part == 0) sH[i] = i < nv ? hd : 0.f;
         if (w == 0) {
@@ -984,10 +1050,13 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
         if constexpr (!DUAL) {
             if (w < 4 * K::ND) {
                 // dv: the chunk's part, sum_i a_ij g_i (a_ij = 0 for i < j)
-                pipe<4, Op2>(
-                    4 - jb,
-                    [&](int s) { return Op2{sG[16 * jb + 4 * s + g][16 * xb + c16], sA[16 * jb + 4 * s + g][tok]}; },
-                    [&](const Op2 &o) { ov = mfma4(o.a, o.b, ov); });
+                const bool bad = !VEC && __builtin_amdgcn_readfirstlane(sBad) == c + 1;
+                const int i0 = 16 * jb + (bad ? 16 : 0);
+                if (i0 < kC)
+                    pipe<4, Op2>(
+                        4 - i0 / 16, [&](int s) { return Op2{sG[i0 + 4 * s + g][16 * xb + c16], sA[i0 + 4 * s + g][tok]}; },
+                        [&](const Op2 &o) { ov = mfma4(o.a, o.b, ov); });
+                if (bad) diag_cols(jb, xb, g, tok, sG, sA, ov);
                 if (tok < nv) {
                     const int d = 16 * xb + 4 * g;
                     store_out(a.dv, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, ov, a.D - d, VEC);
@@ -1018,13 +1087,24 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
             __syncthreads();
             // ---- dFk: the chunk's part, sum_i da_ij Fq_i -> dk
             if (w < 4 * K::ND) {
-                pipe<4, Op2>(
-                    4 - jb,
-                    [&](int s) { return Op2{sQ[16 * jb + 4 * s + g][16 * xb + c16], sA[16 * jb + 4 * s + g][tok]}; },
-                    [&](const Op2 &o) {
-                        fx = mfma4(o.a, o.b, fx);
-                        fy = mfma4(o.a * o.a, o.b, fy);
-                    });
+                const bool bad = !VEC && __builtin_amdgcn_readfirstlane(sBad) == c + 1;
+                const int i0 = 16 * jb + (bad ? 16 : 0);
+                if (i0 < kC)
+                    pipe<4, Op2>(
+                        4 - i0 / 16, [&](int s) { return Op2{sQ[i0 + 4 * s + g][16 * xb + c16], sA[i0 + 4 * s + g][tok]}; },
+                        [&](const Op2 &o) {
+                            fx = mfma4(o.a, o.b, fx);
+                            fy = mfma4(o.a * o.a, o.b, fy);
+                        });
+                if (bad) {
+                    diag_cols(jb, xb, g, tok, sQ, sA, fx);
+                    for (int j = tok; j < 16 * jb + 16; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float q = sQ[j][16 * xb + 4 * g + r];
+                            fy[r] = fmaf(q * q, sA[j][tok], fy[r]);
+                        }
+                }
                 const int d = 16 * xb + 4 * g;
                 const f32x4 k = ld4(&sK[tok][d]);
                 f32x4 dk;

@@ -193,3 +193,42 @@ def test_chunk_f32_selective_strong_decays(D, share):
         err[n] = float(np.linalg.norm(to_np(x).astype(np.float64).reshape(r.shape) - r) / np.linalg.norm(r))
     print({n: f"{e:.1e}" for n, e in err.items()})
     assert err.pop("dld") < 1e-5 and max(err.values()) < 1e-6, err
+
+
+@pytest.mark.parametrize("selective", [False, True])
+@pytest.mark.parametrize("D,b", [(16, 0), (32, 37), (63, 79), (40, 64)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e25])
+def test_chunk_f32_unbounded_values_reach_only_tokens_that_see_them(selective, D, b, bad):
+    """Head dims below 64: NaN, infinity or a value whose square overflows in one token's
+    q, k, v or dy leaves every result that does not depend on that token as without it
+    (the order of a tile's sum apart: the file's tolerance)."""
+    B, H, L = 1, 2, 100
+    q, k, v, lam, rng = _case(B, H, L, D, 17)
+    dy = rng.standard_normal(q.shape).astype(np.float32)
+    ld, beta = to_dev(np.log(rng.uniform(0.9, 1.0, (B, H, L))).astype(np.float32)), to_dev(np.ones(H, np.float32))
+
+    def run(q, k, v, dy):
+        t = [to_dev(x) for x in (q, k, v)]
+        y, g = torch.empty_like(t[0]), [torch.empty_like(t[0]) for _ in range(3)]
+        if selective:
+            dld, dks = torch.empty(B, H, L, device=dev()), torch.empty(B, H, device=dev())
+            _lib.selective_prefill(*t, ld, beta, 1.0, None, y, None)
+            _lib.selective_prefill_backward(*t, ld, beta, 1.0, None, to_dev(dy), None, *g, None, dld, dks)
+        else:
+            _lib.chunked_prefill(*t, to_dev(lam), 1.0, 64, None, y, None)
+            _lib.chunked_prefill_backward(*t, to_dev(lam), 1.0, None, to_dev(dy), None, *g, None)
+        torch.cuda.synchronize()
+        return [to_np(x) for x in (y, *g)]
+    clean = run(q, k, v, dy)
+    before, after = np.arange(L) < b, np.arange(L) > b
+    other, none, every = before | after, np.zeros(L, bool), np.ones(L, bool)
+    # tokens of y, dq, dk, dv that do not depend on token b's q, k, v, dy
+    free = {"q": (other, other, after, after), "k": (before, before, none, none),
+            "v": (before, before, none, every), "dy": (every, other, after, after)}
+    for name, tokens in free.items():
+        x = {"q": q.copy(), "k": k.copy(), "v": v.copy(), "dy": dy.copy()}
+        x[name][:, :, b, D // 2] = bad
+        for what, got, want, n in zip(("y", "dq", "dk", "dv"), run(**x), clean, tokens):
+            if n.any():
+                e = np.abs(got[:, :, n] - want[:, :, n]).max() / np.abs(want).max()
+                assert e < TOL, (name, what, e)
