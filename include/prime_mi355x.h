@@ -21,10 +21,10 @@
  *
  * Head dim: D = 64 runs the MFMA chunk kernels; the base and selective forms
  * (prefill, decode step, backward, QK-norm) also take 1 <= D <= 63 (the
- * reference's own tests use 32 and 16), run in fp32 chunks (one token: one
- * wavefront per (sequence, head)) with no row-alignment requirement and no
- * workspace beyond the backward's per-token records.  The delta rule takes D <= 64
- * with any chunk (documented at prime_delta_prefill).  prime_accumulate and
+ * reference's own tests use 32 and 16), run in fp32 chunks (one token, and a
+ * few on many sequences: one wavefront per (sequence, head)) with no
+ * row-alignment requirement and no workspace beyond the backward's per-token
+ * records.  The delta rule takes D <= 64 with any chunk (documented at prime_delta_prefill).  prime_accumulate and
  * the split decode readout/update take D = 64 only.
  */
 #ifndef PRIME_MI355X_H

@@ -44,7 +44,8 @@
 // (8 waves, nothing loaded ahead, 2 segments: 187, 206, 72); a chunk is 16-18 us of which
 // its MFMAs are 8.4.  At D = 32, 8 sequences of 256 tokens: prefill 25 us, backward 71 us, against
 // 934 and 3580 us for one wavefront per sequence running the recurrence token by token
-// (one token costs the same either way, so a single token keeps that kernel).
+// (a single token, and a few tokens on many sequences, keep a kernel that goes token by token:
+// generic_d.hip).
 
 #include "head_row.h"
 #include "prefill_common.h"

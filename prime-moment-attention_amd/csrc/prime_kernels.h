@@ -276,8 +276,8 @@ struct DeltaArgs {
     int first, last;            // window is the first / last of the call
 };
 
-// Head dims below 64: one token (generic_d.hip, one wavefront per (sequence,
-// head)) and several (chunk_f32.hip).
+// Head dims below 64: one token, or a few on many sequences (generic_d.hip, one
+// wavefront per (sequence, head)), and the rest (chunk_f32.hip).
 struct GenericArgs {
     const void *q, *k, *v;
     int64_t q_sb, q_sh, q_sl, k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;

@@ -620,3 +620,41 @@ def test_generic_selective_module_head_dim_32():
         _, st = m(x.detach(), return_state=True)
         o1, _ = m(torch.randn(B, 1, 128, device=dev()), state=st)
     assert torch.isfinite(o1).all()
+
+
+@pytest.mark.parametrize("form", ["plain", "state", "inplace", "dense", "selective", "qknorm"])
+@pytest.mark.parametrize("D,L", [(1, 2), (16, 4), (31, 5), (32, 9), (48, 12), (63, 3)])
+def test_generic_few_tokens_on_many_sequences(form, D, L):
+    """Few tokens on several sequences a CU run token by token, the same call on a slice
+    of the batch in chunks: the same values, for the first and the last sequences, in every
+    form and with rows at odd strides, mixed dtypes and grouped heads.  1e-5 of each
+    tensor's largest value (fp32 sums in another order), 2^-7 with the LayerNorm's bf16
+    rows (a rounding at a tie)."""
+    B, H, Hkv = 1200, 4, 2  # 4800 sequences: 18 a CU of 256
+    g = torch.Generator().manual_seed(D * 100 + L)
+    dts = [torch.bfloat16] * 3 if form == "qknorm" else [torch.float32, torch.bfloat16, torch.float16]
+    big = [(torch.randn(B, h, L, D + 3, generator=g) * 0.3).to(dev(), dt) for h, dt in zip((H, Hkv, Hkv), dts)]
+    lam = torch.linspace(0.9, 0.999, H, device=dev())
+    st = [torch.rand(B, *x.shape[1:], generator=g).to(dev()) for x in _lib.new_state(1, H, D, "cpu")]
+    ld = -torch.rand(B, H, L, generator=g).to(dev())
+    ln = [torch.nn.LayerNorm(D).to(dev(), torch.bfloat16) for _ in range(2)]
+    print(f"[few tokens] {form} D={D} L={L}", flush=True)
+
+    def run(n):
+        q, k, v = (t[n][..., 2:2 + D] for t in big)
+        b = q.shape[0]
+        s_in = None if form == "plain" else tuple(x[n].clone() for x in st)
+        s_out = s_in if form == "inplace" else _lib.new_state(b, H, D, dev())
+        y = torch.empty(b, L, H, D, device=dev()).transpose(1, 2)
+        if form == "selective":
+            _lib.selective_prefill(q, k, v, ld[n].contiguous(), lam, 1.0, s_in, y, s_out)
+        else:
+            norm = _lib.qk_norm(*ln, 0.25, torch.bfloat16) if form == "qknorm" else None
+            _lib.chunked_prefill(q, k, v, lam, 2.0, 64, s_in, y, s_out, flags=1 if form == "dense" else 0,
+                                 qk_norm=norm)
+        return (y, *s_out)
+    whole = run(slice(0, B))
+    tol = 2 ** -7 if form == "qknorm" else 1e-5
+    for n in (slice(0, 8), slice(B - 8, B)):
+        for x, r in zip(whole, run(n)):
+            assert (x[n] - r).abs().max() <= tol * r.abs().max()
