@@ -54,6 +54,12 @@ constexpr int kPX = 3 * kD + 16; // X rows: scalar reads of 4 rows x 16 columns 
 constexpr int kPS = 32 + 4;      // the chain's state rows in operand order
 constexpr float kInvSqrt2 = 0.70710678118654752f;
 
+// four floats of a caller's state or gradient, which is only known to be 4-byte aligned
+// (one 16-byte access all the same: global memory takes any dword boundary)
+typedef f32x4 f32x4_dw __attribute__((aligned(4)));
+__device__ __forceinline__ f32x4 ld4_dw(const float *p) { return *reinterpret_cast<const f32x4_dw *>(p); }
+__device__ __forceinline__ void st4_dw(float *p, f32x4 v) { *reinterpret_cast<f32x4_dw *>(p) = v; }
+
 // Record of one (sequence, chunk), bytes.  The chains' 128 x 128 operands are
 // stored in the order they are read: [8 row blocks][64 lanes][32 k-steps], lane
 // l of block b holding row 16 b + l%16, columns 32 (l/16) + s; R0 and Q0 as
@@ -420,7 +426,7 @@ __global__ __launch_bounds__(kW *kWave, 1) void delta_bwd_chain_kernel(const Del
 
     f32x4 st[4];
 #pragma unroll
-    for (int dv = 0; dv < 4; ++dv) st[dv] = src ? ld4(src + sofs + so + 16 * dv * kP) : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dv = 0; dv < 4; ++dv) st[dv] = src ? ld4_dw(src + sofs + so + 16 * dv * kP) : f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto publish = [&](int buf) {
 #pragma unroll
@@ -527,7 +533,7 @@ __global__ __launch_bounds__(kW *kWave, 1) void delta_bwd_chain_kernel(const Del
         if (c == 0) step(0, ra, rb, fa, fb);
         if (a.dstate_in) {
 #pragma unroll
-            for (int dv = 0; dv < 4; ++dv) st4(a.dstate_in + sofs + so + 16 * dv * kP, st[dv]);
+            for (int dv = 0; dv < 4; ++dv) st4_dw(a.dstate_in + sofs + so + 16 * dv * kP, st[dv]);
         }
     }
 }
@@ -949,7 +955,7 @@ __global__ __launch_bounds__(kW *kWave, 1) void delta_bwd_grad_kernel(const Delt
             d2 = fmaf(p2[r], dphi[jj][1][r], d2);
             dq[r] = dpsi[jj][0][r] + 2.0f * kInvSqrt2 * q[r] * dpsi[jj][1][r];
         }
-        if (valid) st4(a.dq + (obase + tok) * kD + f0, dq);
+        if (valid) st4_dw(a.dq + (obase + tok) * kD + f0, dq);
     }
     d1 = sum_rows(d1);
     d2 = sum_rows(d2);
@@ -977,7 +983,7 @@ __global__ __launch_bounds__(kW *kWave, 1) void delta_bwd_grad_kernel(const Delt
                 const float g2 = r2 * (kInvSqrt2 * dphi[jj][1][r] - 1.4142135623730951f * p2[r] * n2);
                 dk[r] = g1 + 2.0f * kx * g2;
             }
-            if (valid) st4(a.dk + (obase + tok) * kD + f0, dk);
+            if (valid) st4_dw(a.dk + (obase + tok) * kD + f0, dk);
         }
     }
 }

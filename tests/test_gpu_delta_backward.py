@@ -245,3 +245,35 @@ def test_delta_module_trains_through_the_step_branch():
     for (name, p), (_, pc) in zip(m.named_parameters(), mc.named_parameters()):
         assert p.grad is not None, name
         assert _rel(p.grad, pc.grad) < TOL, (name, _rel(p.grad, pc.grad))
+
+
+def test_delta_backward_states_and_gradients_on_any_word():
+    """state_in, dstate_out and the fp32 outputs one, two and three words past a 16-byte
+    boundary: the same gradients, and nothing outside the outputs written."""
+    B, H, L, D = 1, 2, 130, 64
+    q, k, v, beta, alpha, s0, dy, ds = _case(B, H, H, L, 77, torch.float32)
+    t = [x.to(dev()).contiguous() for x in (q, k, v, dy)]
+    ws = torch.empty(_lib.delta_backward_workspace_size(B, H, L), dtype=torch.uint8, device=dev())
+    sizes = [B * H * L * D] * 3 + [B * H * L] * 2 + [B * H * D * 2 * D]
+    runs = []
+    for off in (0, 1, 2, 3):
+        def shifted(x):
+            buf = torch.zeros(x.numel() + 8, device=dev())
+            buf[off:off + x.numel()] = x.reshape(-1).to(dev())
+            return buf
+        si, so, be, al = (shifted(x) for x in (s0, ds, beta, alpha))
+        out = [torch.full((n + 8,), 7.0, device=dev()) for n in sizes]
+        d = [_lib.tensor_desc(x, True) for x in t]
+        p = lambda x: x.data_ptr() + 4 * off
+        r = _lib.ctypes.byref
+        rc = _lib.load().prime_delta_prefill_backward(
+            r(d[0]), r(d[1]), r(d[2]), p(be), p(al), B, H, H, L, D, 64, 0.9995, 1e-5, 2.0, p(si), r(d[3]), p(so),
+            *[p(x) for x in out], ws.data_ptr(), ws.numel(), _lib._stream(ws.device))
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        for x, n in zip(out, sizes):
+            assert (x[:off] == 7).all() and (x[off + n:] == 7).all()
+        runs.append([x[off:off + n].clone() for x, n in zip(out, sizes)])
+    for run in runs[1:]:
+        for x, r0 in zip(run, runs[0]):
+            assert torch.equal(x, r0)
