@@ -894,7 +894,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dq_kernel(const ChunkF32Args 
                     }
                     dq[r] = x1 + 2.0f * q[r] * y1;
                 }
-                store_out(a.dq, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, dq, a.D - d, VEC);
+                store_out(a.dq, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, dq, a.D - d, VEC && a.g_vec);
             }
         }
         __syncthreads();
@@ -1060,7 +1060,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
                 if (bad) diag_cols(jb, xb, g, tok, sG, sA, ov);
                 if (tok < nv) {
                     const int d = 16 * xb + 4 * g;
-                    store_out(a.dv, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, ov, a.D - d, VEC);
+                    store_out(a.dv, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, ov, a.D - d, VEC && a.g_vec);
                 }
                 // ---- dFk^T tiles (feature block xb and its squares; tokens of block jb): the carried part
                 pipe<4, Op3>(
@@ -1134,7 +1134,7 @@ __global__ __launch_bounds__(kT, 1) void chunk_f32_dkv_kernel(const ChunkF32Args
                             dk[r] *= ks;
                         }
                     }
-                    store_out(a.dk, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, dk, a.D - d, VEC);
+                    store_out(a.dk, a.dt_g, gbase + static_cast<int64_t>(c * kC + tok) * a.g_sl + d, dk, a.D - d, VEC && a.g_vec);
                 }
             }
             if constexpr (SEL) {
@@ -1350,6 +1350,7 @@ hipError_t launch_prefill_backward_f32(const BwdArgs &a, hipStream_t stream) {
     o.ds0 = a.ds0o; o.ds1 = a.ds1o; o.ds2 = a.ds2o; o.dk0 = a.dk0o; o.dk1 = a.dk1o; o.dk2 = a.dk2o;
     o.dsi0 = a.ds0i; o.dsi1 = a.ds1i; o.dsi2 = a.ds2i; o.dki0 = a.dk0i; o.dki1 = a.dk1i; o.dki2 = a.dk2i;
     o.dq = a.dq; o.dk = a.dk; o.dv = a.dv; o.dt_g = a.dt_g; o.g_sb = a.g_sb; o.g_sh = a.g_sh; o.g_sl = a.g_sl;
+    o.g_vec = gradient_rows_vec(a);
     o.inv_den = a.inv_den; o.g_den = a.g_den;
     o.kc1 = a.kcorr; o.kc2 = a.kcorr + kD; o.kc0 = a.kcorr + 2 * kD;
     o.kc_s = o.kc0_s = kBwdCorr;

@@ -1164,13 +1164,18 @@ void plan_backward_segments(int S, int L, int *G, int *cps, int per_cu) {
     *G = (NC + c - 1) / c;  // no empty segments
 }
 
+// gradient rows take one store of four elements if every row starts on such a boundary
+bool gradient_rows_vec(const BwdArgs &a) {
+    const uintptr_t four = (a.dt_g == PRIME_F32 ? 4 : 2) * 4;
+    return (reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) | reinterpret_cast<uintptr_t>(a.dv)) %
+                   four == 0 &&
+           a.g_sb % 4 == 0 && a.g_sh % 4 == 0 && a.g_sl % 4 == 0;
+}
+
 hipError_t launch_prefill_backward(const BwdArgs &args, hipStream_t stream) {
     if (args.dt_in == PRIME_F32) return launch_prefill_backward_f32(args, stream);
     BwdArgs a = args;
-    // gradient rows take one store of four elements if every row starts on such a boundary
-    const uintptr_t gsz = (a.dt_g == PRIME_F32 ? 4 : 2) * 4;
-    a.g_vec = !((reinterpret_cast<uintptr_t>(a.dq) | reinterpret_cast<uintptr_t>(a.dk) |
-                 reinterpret_cast<uintptr_t>(a.dv)) % gsz || a.g_sb % 4 || a.g_sh % 4 || a.g_sl % 4);
+    a.g_vec = gradient_rows_vec(a);
     const int S = a.B * a.H;
     hipError_t e;
     if (a.G > 1) {

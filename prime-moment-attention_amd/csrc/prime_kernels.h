@@ -205,7 +205,7 @@ struct BwdArgs {
     void *dq, *dk, *dv;
     int dt_g;
     int64_t g_sb, g_sh, g_sl;                               // strides of dq, dk, dv
-    bool g_vec;  // (bf16 passes) gradient rows on boundaries of four elements; set by the launch
+    bool g_vec;  // gradient rows on boundaries of four elements; set by the launch
     float *ds0i, *ds1i, *ds2i, *dk0i, *dk1i, *dk2i;         // adjoint of the incoming state (null => none)
     float *inv_den, *g_den;                                 // [B*H, L] fp32, written by the dq pass
     // the dense branch's double clamp with an incoming state (G == 1): the dq
@@ -226,6 +226,7 @@ struct BwdArgs {
 };
 constexpr int kBwdCorr = 132;  // floats per sequence in BwdArgs::kcorr (128 features, K0, padding)
 
+bool gradient_rows_vec(const BwdArgs &a);
 hipError_t launch_prefill_backward(const BwdArgs &a, hipStream_t stream);
 // fp32 inputs: the fp32 dq and dk/dv passes (chunk_f32.hip)
 hipError_t launch_prefill_backward_f32(const BwdArgs &a, hipStream_t stream);
@@ -303,6 +304,7 @@ struct GenericArgs {
     void *dq, *dk, *dv;
     int dt_g;
     int64_t g_sb, g_sh, g_sl;
+    bool g_vec;  // (D = 64) gradient rows on boundaries of four elements
     float *dsi0, *dsi1, *dsi2, *dki0, *dki1, *dki2;  // adjoint of the incoming state or null
     float *inv_den, *g_den;                           // [B*H][L]: 1/D and the denominator's adjoint
     // the dense clamp's share of the incoming K adjoint (dq pass to dk/dv pass), per

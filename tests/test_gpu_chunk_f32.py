@@ -232,3 +232,35 @@ def test_chunk_f32_unbounded_values_reach_only_tokens_that_see_them(selective, D
             if n.any():
                 e = np.abs(got[:, :, n] - want[:, :, n]).max() / np.abs(want).max()
                 assert e < TOL, (name, what, e)
+
+
+@pytest.mark.parametrize("form", ["base", "dense state", "selective"])
+def test_chunk_f32_gradient_rows_on_any_element(form):
+    """Head dim 64, fp32: gradient rows off the four-element boundary (element stores)
+    hold the bits of aligned ones (one store per four), and the padding between rows is
+    left alone, for every gradient dtype."""
+    B, H, L, D = 1, 2, 150, 64
+    q, k, v, lam, rng = _case(B, H, L, D, 60)
+    t = [to_dev(x) for x in (q, k, v)]
+    dy = to_dev(rng.standard_normal(q.shape).astype(np.float32))
+    ld = to_dev(np.log(rng.uniform(0.9, 1.0, (B, H, L))).astype(np.float32))
+    st = state_to_dev(random_state(B * H, D, 61), B, H, D) if form == "dense state" else None
+
+    def run(dtype, pitch):
+        buf = [torch.full((B, H, L, pitch), 7.0, device=dev(), dtype=dtype) for _ in range(3)]
+        g = [b[..., pitch - D:] for b in buf]
+        if form == "selective":
+            dld, dks = torch.empty(B, H, L, device=dev()), torch.empty(B, H, device=dev())
+            _lib.selective_prefill_backward(*t, ld, to_dev(lam), 1.0, None, dy, None, *g, None, dld, dks)
+        else:
+            _lib.chunked_prefill_backward(*t, to_dev(lam), 1.0, st, dy, None, *g,
+                                          _lib.new_state(B, H, D, dev()) if st else None, flags=1 if st else 0)
+        torch.cuda.synchronize()
+        assert all((b[..., :pitch - D] == 7).all() for b in buf)
+        return [x.contiguous() for x in g]
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+        ref = run(dtype, D)
+        for pitch in (D + 1, D + 2, D + 4):
+            print(f"[chunk f32 rows] {form} {dtype} pitch {pitch}", flush=True)
+            for x, r in zip(run(dtype, pitch), ref):
+                assert torch.equal(x, r)
