@@ -279,11 +279,13 @@ int prime_delta_gates(const void *erase, int64_t erase_sb, int64_t erase_sl, con
  *                  forward's clamp [1e-5, 1]
  *   dstate_in    : fp32 [B, H, D, 2D] or NULL
  *   workspace    : prime_delta_prefill_backward_workspace_size(B, H, L, D, chunk)
- *                  bytes (per chunk its transfer record, the state entering it
- *                  and the state's adjoint, in fp32, for as many (sequence,
- *                  head) pairs as 8 GiB hold and at least one; outside D = 64
- *                  with chunk 64 the state entering every chunk and one
- *                  chunk's token states per (sequence, head))
+ *                  bytes.  D = 64 with chunk 64: per chunk its transfer record,
+ *                  the state entering it and the state's adjoint, in fp32, for
+ *                  two (sequence, head) pairs a CU and at most 8 GiB; any size
+ *                  from one pair's (the same function at B = H = 1) works, the
+ *                  pairs then go in smaller groups.  Else the state entering
+ *                  every chunk and one chunk's token states per (sequence,
+ *                  head), which is the least
  * fp32 arithmetic throughout.
  */
 size_t prime_delta_prefill_backward_workspace_size(int B, int H, int L, int D, int chunk);

@@ -1368,9 +1368,9 @@ int prime_delta_prefill_backward(const prime_tensor_t *q, const prime_tensor_t *
     if (!rows_aligned(q, true) || !rows_aligned(k, true) || !rows_aligned(v, true) || !rows_aligned(dy, true))
         return fail(PRIME_ERR_MISALIGNED, "q/k/v/dy rows must start on 16-byte boundaries");
     if (!aligned16(workspace)) return fail(PRIME_ERR_MISALIGNED, "workspace must be 16-byte aligned");
-    if (workspace_bytes < prime_delta_prefill_backward_workspace_size(B, H, L, D, chunk))
-        return fail(PRIME_ERR_INVALID_ARG, "workspace of %zu bytes is below the %zu this shape needs", workspace_bytes,
-                    prime_delta_prefill_backward_workspace_size(B, H, L, D, chunk));
+    if (workspace_bytes < prime::delta_backward_ws_bytes(1, 1, L))
+        return fail(PRIME_ERR_INVALID_ARG, "workspace of %zu bytes is below the %zu that one sequence of this length needs",
+                    workspace_bytes, prime::delta_backward_ws_bytes(1, 1, L));
     prime::DeltaBwdArgs a{};
     a.q = q->data; a.k = k->data; a.v = v->data; a.dy = dy->data;
     a.q_sb = q->stride_b; a.q_sh = q->stride_h; a.q_sl = q->stride_l;
@@ -1384,6 +1384,7 @@ int prime_delta_prefill_backward(const prime_tensor_t *q, const prime_tensor_t *
     a.state_in = state_in; a.dstate_out = dstate_out;
     a.dq = dq; a.dk = dk; a.dv = dv; a.dbeta = dbeta; a.dalpha = dalpha; a.dstate_in = dstate_in;
     a.ws = static_cast<float *>(workspace);
+    a.ws_bytes = workspace_bytes;
     return check_hip(prime::launch_delta_backward(a, static_cast<hipStream_t>(stream)), "delta backward launch");
 }
 

@@ -41,6 +41,8 @@
 // MFMAs a wave are 3.4 us), grad 82 us: 0.37 ms.  As one kernel per sequence, fp32
 // on the VALU with the chunks in reverse and 24 of 256 CUs busy, it took 6.43 ms.
 
+#include <algorithm>
+
 #include "delta_f32_common.h"
 
 namespace prime {
@@ -988,14 +990,15 @@ __global__ __launch_bounds__(kW *kWave, 1) void delta_bwd_grad_kernel(const Delt
     }
 }
 
-// Sequences are taken in groups whose workspace stays within this (at least one
-// sequence): at 1024 tokens 2000 sequences at once, far more than the chains need
-// to fill the chip.
+// Sequences are taken in groups, as many as the workspace holds.  Its full size is for two a CU
+// (the chains' LDS lets two workgroups share one) and 8 GiB, at least one sequence: 2048
+// sequences of 1024 tokens take 12.6 ms in groups of 512 (2.3 GB), 12.4 in one (9.2), 13.4 in
+// groups of 192, 18.5 of 64; 192 of 2048 2.5 ms in one, 3.0 in two, 3.4 in three.
 constexpr size_t kDeltaBwdWsCap = size_t{8} << 30;
 
 size_t delta_backward_ws_bytes(int B, int H, int L) {
     const size_t per = seq_ws_bytes((L + kC - 1) / kC), n = static_cast<size_t>(B) * H;
-    const size_t fit = kDeltaBwdWsCap / per;
+    const size_t fit = std::min<size_t>(kDeltaBwdWsCap / per, 2 * static_cast<size_t>(device_cus()));
     return per * (fit < 1 ? 1 : fit < n ? fit : n);
 }
 
@@ -1015,7 +1018,7 @@ static hipError_t launch_group(const DeltaBwdArgs &a, int n, int NC, hipStream_t
 
 hipError_t launch_delta_backward(DeltaBwdArgs a, hipStream_t stream) {
     const int NC = (a.L + kC - 1) / kC, total = a.B * a.H;
-    const int group = static_cast<int>(delta_backward_ws_bytes(a.B, a.H, a.L) / seq_ws_bytes(NC));
+    const int group = static_cast<int>(std::min<size_t>(a.ws_bytes / seq_ws_bytes(NC), total));
     for (a.seq0 = 0; a.seq0 < total; a.seq0 += group) {
         const int n = group < total - a.seq0 ? group : total - a.seq0;
         const hipError_t e = a.dt_in == PRIME_BF16 ? launch_group<PRIME_BF16>(a, n, NC, stream)

@@ -353,7 +353,8 @@ struct DeltaBwdArgs {
     float *dq, *dk, *dv;        // [B, H, L, D]
     float *dbeta, *dalpha;      // [B, H, L]
     float *dstate_in;           // [B, H, D, 2D] or null
-    float *ws;                  // delta_backward_ws_bytes
+    float *ws;                  // at least one sequence's share (delta_backward_ws_bytes(1, 1, L))
+    size_t ws_bytes;
     int seq0;                   // first (sequence, head) of the group in the workspace
 };
 size_t delta_backward_ws_bytes(int B, int H, int L);

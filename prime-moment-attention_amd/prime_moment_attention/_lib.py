@@ -950,6 +950,20 @@ def delta_backward_workspace_size(B: int, H: int, L: int, D: int = 64, chunk: in
     return int(load().prime_delta_prefill_backward_workspace_size(B, H, L, D, chunk))
 
 
+def _delta_backward_workspace(B: int, H: int, L: int, D: int, chunk: int, dev) -> torch.Tensor:
+    """The delta backward's workspace; where memory is short, half of it and so on down
+    to one sequence's (D = 64, chunk 64: the sequences then go in smaller groups)."""
+    size = delta_backward_workspace_size(B, H, L, D, chunk)
+    least = delta_backward_workspace_size(1, 1, L) if D == 64 and chunk == 64 else size
+    while True:
+        try:
+            return torch.empty(size, dtype=torch.uint8, device=dev)
+        except torch.OutOfMemoryError:
+            if size <= least:
+                raise
+            size = max(size // 2, least)
+
+
 def delta_prefill_backward(q, k, v, beta, alpha, decay_pad: float, feat_eps: float, bound: float, state_in, dy,
                            dstate_out, workspace: Optional[torch.Tensor] = None, chunk: int = 64):
     """Gradients of the chunked delta-rule prefill (prime_delta_prefill_backward)
@@ -975,7 +989,7 @@ def delta_prefill_backward(q, k, v, beta, alpha, decay_pad: float, feat_eps: flo
     dalpha = torch.empty(B, H, Lq, **f32)
     dstate = torch.empty(B, H, D, 2 * D, **f32) if state_in is not None else None
     if workspace is None:
-        workspace = torch.empty(delta_backward_workspace_size(B, H, Lq, D, chunk), dtype=torch.uint8, device=dev)
+        workspace = _delta_backward_workspace(B, H, Lq, D, chunk, dev)
     qd, kd, vd, yd = tensor_desc(q, True), tensor_desc(k, True), tensor_desc(v, True), tensor_desc(dy, True)
     ptr = lambda t: ctypes.c_void_p(t.data_ptr()) if t is not None else None
     rc = load().prime_delta_prefill_backward(

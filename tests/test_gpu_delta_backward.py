@@ -90,7 +90,7 @@ def test_delta_backward_sequence_groups():
     """More sequences than one workspace group holds: the later group's results
     equal those of a call with its sequences alone."""
     H, L = 120, 3
-    B = 235  # 28200 (sequence, head) pairs; 8 GiB hold about 27000 of one chunk each
+    B = 235  # 28200 (sequence, head) pairs, two a CU in a group
     per = _lib.delta_backward_workspace_size(1, 1, L)
     assert _lib.delta_backward_workspace_size(B, H, L) < per * B * H
     q, k, v, beta, alpha, s0, dy, ds = (t.to(dev()).contiguous() for t in _case(B, H, H, L, 9, torch.float32))
@@ -277,3 +277,35 @@ def test_delta_backward_states_and_gradients_on_any_word():
     for run in runs[1:]:
         for x, r0 in zip(run, runs[0]):
             assert torch.equal(x, r0)
+
+
+def test_delta_backward_in_small_workspaces(monkeypatch):
+    """A workspace for one, two and all but one sequence gives the bits of the full one;
+    less than one sequence's is refused; a wrapper that cannot get the full size takes
+    what it can."""
+    B, H, L = 1, 5, 150
+    q, k, v, beta, alpha, s0, dy, ds = (t.to(dev()).contiguous() for t in _case(B, H, H, L, 21, torch.float32))
+    per = _lib.delta_backward_workspace_size(1, 1, L)
+    assert _lib.delta_backward_workspace_size(B, H, L) == per * B * H
+
+    def run(size=None):
+        ws = None if size is None else torch.empty(size, dtype=torch.uint8, device=dev())
+        out = _lib.delta_prefill_backward(q, k, v, beta, alpha, 0.9995, 1e-5, 2.0, s0, dy, ds, workspace=ws)
+        torch.cuda.synchronize()
+        return out
+    ref = run(per * B * H)
+    for size in (per, 2 * per, 4 * per, 2 * per + 100, 20 * per):
+        assert all(torch.equal(x, r) for x, r in zip(run(size), ref))
+    with pytest.raises(RuntimeError, match="below"):
+        run(per - 1)
+    sizes, empty = [], torch.empty
+
+    def scarce(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            sizes.append(a[0])
+            if a[0] > 2 * per:
+                raise torch.OutOfMemoryError("no memory")
+        return empty(*a, **kw)
+    monkeypatch.setattr(torch, "empty", scarce)
+    assert all(torch.equal(x, r) for x, r in zip(run(), ref))
+    assert sizes == [5 * per, 5 * per // 2, 5 * per // 4]
