@@ -580,7 +580,8 @@ int prime_accumulate_noalloc(const prime_tensor_t *k, const prime_tensor_t *v, i
  * as the reference differentiates in fp32).
  * workspace (16-byte aligned): at least B*H*L*8 bytes (per-token
  * denominators; rounded up to 256), plus B*H*528 bytes for
- * PRIME_FLAG_DENSE_CLAMP with a state; with prime_chunked_prefill_backward_workspace_size()
+ * PRIME_FLAG_DENSE_CLAMP with a state (below D = 64 the first suffice unless
+ * dstate_in and dstate_out share memory); with prime_chunked_prefill_backward_workspace_size()
  * bytes, few long sequences are split into segments that run in parallel
  * (segment-entry states by the forward's state-only pass, dual states by a
  * reverse scan).  Results agree either way.

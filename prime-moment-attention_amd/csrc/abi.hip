@@ -141,20 +141,34 @@ int generic_args(prime::GenericArgs &a, const prime_tensor_t *q, const prime_ten
 
 // The backward's per-token scratch at the start of the workspace, and the dense
 // clamp's incoming-K correction: behind it where the workspace holds it, else in
-// the incoming state's adjoint itself (which the dk/dv pass writes last).
-void generic_bwd_scratch(prime::GenericArgs &a, void *workspace, size_t workspace_bytes, size_t token_bytes) {
+// the incoming state's adjoint itself (which the dk/dv pass writes last).  The dk/dv
+// pass reads the final state's adjoint after the correction is written, so then the
+// two may not share memory.
+int generic_bwd_scratch(prime::GenericArgs &a, void *workspace, size_t workspace_bytes, size_t token_bytes) {
+    const size_t S = static_cast<size_t>(a.B) * a.H;
     a.inv_den = static_cast<float *>(workspace);
-    a.g_den = a.inv_den + static_cast<size_t>(a.B) * a.H * a.L;
-    if (workspace_bytes >= token_bytes + static_cast<size_t>(a.B) * a.H * prime::kBwdCorr * sizeof(float)) {
+    a.g_den = a.inv_den + S * a.L;
+    const size_t full = token_bytes + S * prime::kBwdCorr * sizeof(float);
+    if (workspace_bytes >= full) {
         a.kc1 = reinterpret_cast<float *>(static_cast<char *>(workspace) + token_bytes);
         a.kc2 = a.kc1 + prime::kD;
         a.kc0 = a.kc2 + prime::kD;
         a.kc_s = a.kc0_s = prime::kBwdCorr;
-    } else {
-        a.kc1 = a.dki1; a.kc2 = a.dki2; a.kc0 = a.dki0;
-        a.kc_s = a.D;
-        a.kc0_s = 1;
+        return PRIME_OK;
     }
+    a.kc1 = a.dki1; a.kc2 = a.dki2; a.kc0 = a.dki0;
+    a.kc_s = a.D;
+    a.kc0_s = 1;
+    if (a.dense_clamp && a.s1i && a.dsi1 && a.ds1) {
+        const float *out[3] = {a.kc1, a.kc2, a.kc0}, *in[6] = {a.ds0, a.ds1, a.ds2, a.dk0, a.dk1, a.dk2};
+        const size_t D = a.D, no[3] = {S * D, S * D, S}, ni[6] = {S * D, S * D * D, S * D * D, S, S * D, S * D};
+        for (int i = 0; i < 3; ++i)
+            for (int j = 0; j < 6; ++j)
+                if (overlap(out[i], no[i] * sizeof(float), in[j], ni[j] * sizeof(float)))
+                    return fail(PRIME_ERR_ALIAS, "dstate_in overlaps dstate_out: the dense clamp then needs a workspace "
+                                "of %zu bytes", full);
+    }
+    return PRIME_OK;
 }
 
 int generic_norm(prime::GenericArgs &a, const prime_qk_norm_t *norm) {
@@ -917,7 +931,7 @@ int prime_chunked_prefill_backward(const prime_tensor_t *q, const prime_tensor_t
             g.dsi0 = dstate_in->s0; g.dsi1 = dstate_in->s1; g.dsi2 = dstate_in->s2;
             g.dki0 = dstate_in->k0; g.dki1 = dstate_in->k1; g.dki2 = dstate_in->k2;
         }
-        generic_bwd_scratch(g, workspace, workspace_bytes, bwd_token_bytes(B, H, L));
+        if ((rc = generic_bwd_scratch(g, workspace, workspace_bytes, bwd_token_bytes(B, H, L)))) return rc;
         return check_hip(prime::launch_chunk_f32_backward(g, static_cast<hipStream_t>(stream)), "backward launch");
     }
     if (B <= 0 || H <= 0 || L <= 0) return fail(PRIME_ERR_INVALID_ARG, "bad sizes B=%d H=%d L=%d", B, H, L);
@@ -1054,7 +1068,8 @@ int prime_selective_prefill_backward(const prime_tensor_t *q, const prime_tensor
             g.dsi0 = dstate_in->s0; g.dsi1 = dstate_in->s1; g.dsi2 = dstate_in->s2;
             g.dki0 = dstate_in->k0; g.dki1 = dstate_in->k1; g.dki2 = dstate_in->k2;
         }
-        generic_bwd_scratch(g, workspace, bwd_token_bytes(B, H, L), bwd_token_bytes(B, H, L));
+        // (no dense clamp here, so no correction)
+        if ((rc = generic_bwd_scratch(g, workspace, bwd_token_bytes(B, H, L), bwd_token_bytes(B, H, L)))) return rc;
         g.pq = reinterpret_cast<float *>(static_cast<char *>(workspace) + bwd_token_bytes(B, H, L));
         g.fin = g.pq + static_cast<size_t>(B) * H * L;
         g.dlogd = d_log_decay;

@@ -264,3 +264,29 @@ def test_chunk_f32_gradient_rows_on_any_element(form):
             print(f"[chunk f32 rows] {form} {dtype} pitch {pitch}", flush=True)
             for x, r in zip(run(dtype, pitch), ref):
                 assert torch.equal(x, r)
+
+
+def test_chunk_f32_dense_clamp_backward_in_place_state_adjoint():
+    """dstate_in on the buffers of dstate_out: the same result with the correction in the
+    workspace; refused where the workspace holds the per-token scratch alone (the
+    correction would replace an adjoint that is still to be read)."""
+    B, H, L, D = 1, 2, 90, 32
+    q, k, v, lam, rng = _case(B, H, L, D, 13)
+    st = state_to_dev(random_state(B * H, D, 14), B, H, D)
+    ds = [0.1 * rng.standard_normal(x.shape) for x in O.zero_state(B * H, D)]
+    t, dy = [to_dev(x) for x in (q, k, v)], to_dev(rng.standard_normal(q.shape).astype(np.float32))
+    small = (B * H * L * 8 + 255) // 256 * 256
+
+    def run(inplace, size):
+        g, dso = [torch.empty_like(t[0]) for _ in range(3)], state_to_dev(ds, B, H, D)
+        dsi = dso if inplace else _lib.new_state(B, H, D, dev())
+        _lib.chunked_prefill_backward(*t, to_dev(lam), 2.5, st, dy, dso, *g, dsi, flags=1,
+                                      workspace=torch.empty(size, dtype=torch.uint8, device=dev()))
+        torch.cuda.synchronize()
+        return (*g, *dsi)
+    full = _lib.backward_workspace_size(B, H, L)
+    ref = run(False, full)
+    for out in (run(True, full), run(False, small)):
+        assert all(torch.equal(a, b) for a, b in zip(out, ref))
+    with pytest.raises(RuntimeError, match="overlaps"):
+        run(True, small)
