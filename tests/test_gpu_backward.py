@@ -407,8 +407,8 @@ def test_backward_row_alignment_and_dy_dtype(L, dense_state):
 
 @pytest.mark.parametrize("L", [129, 256, 513, 1000])
 def test_backward_short_segments_equal_one_segment(L):
-    """The bf16 plan splits down to one chunk per segment (a ragged last one too):
-    against one segment per sequence (minimum workspace), with an incoming state and
+    """From below the length where the bf16 plan begins to split (test_backward_short_
+    segments_match_float64 names it): against one segment per sequence (minimum workspace), with an incoming state and
     a final-state adjoint; the tolerance of the segmented test of longer sequences."""
     B, H = 1, 6
     q, k, v = (to_dev(x, torch.bfloat16) for x in O.make_inputs((B, H, L, D), seed=520, bf16=True))
@@ -428,3 +428,34 @@ def test_backward_short_segments_equal_one_segment(L):
     for x, y, n in zip(outs[0][0], outs[1][0], ("dq", "dk", "dv")):
         assert_close(x, y, 5e-3, n)
     assert_state_close(outs[0][1], outs[1][1], 5e-3, "dstate_in")
+
+
+@pytest.mark.parametrize("L", [64 * 3 + 1, 250, 513])
+def test_backward_short_segments_match_float64(L):
+    """bf16, lengths from the first that the plan splits at this batch (one chunk per
+    segment, a ragged last one): the dual-state pass is launched, and not in the minimum
+    workspace, and both agree with float64."""
+    B, H = 1, 6
+    q, k, v = O.make_inputs((B, H, L, D), seed=530, bf16=True)
+    dy = O.bf16_round(np.random.default_rng(531).standard_normal((B, H, L, D)).astype(np.float32))
+    lam = np.linspace(0.99, 0.9999, H).astype(np.float32)
+    st0, ds = random_state(B * H, D, 532), random_state(B * H, D, 533)
+    ref = O.recurrent_vjp(*(x.reshape(H, L, D) for x in (q, k, v)), lam.astype(np.float64), dy.reshape(H, L, D), eps=1.0,
+                          state=st0, dstate=ds)
+    t = [to_dev(x, torch.bfloat16) for x in (q, k, v, dy)]
+    sd = [state_to_dev(x, B, H, D) for x in (st0, ds)]
+    small = (B * H * L * 8 + 255) // 256 * 256
+    for split, nbytes in ((1, _lib.backward_workspace_size(B, H, L)), (0, small)):
+        g, dsi = [torch.empty(B, H, L, D, device=dev()) for _ in range(3)], _lib.new_state(B, H, D, dev())
+        _lib.timer_enable(_lib.KERNEL_BWD_DUAL)
+        _lib.timer_reset()
+        try:
+            _lib.chunked_prefill_backward(*t[:3], to_dev(lam), 1.0, sd[0], t[3], sd[1], *g, dsi,
+                                          workspace=torch.empty(nbytes, dtype=torch.uint8, device=dev()))
+            torch.cuda.synchronize()
+            assert _lib.timer_read(_lib.KERNEL_BWD_DUAL)[1] == split
+        finally:
+            _lib.timer_enable()
+        for x, r, n in zip(g, ref[:3], ("dq", "dk", "dv")):
+            assert_close(to_np(x).reshape(r.shape), r, TOL_BF16, n)
+        assert_state_close(state_to_np(dsi, B * H, D), ref[3], TOL_BF16, "dstate_in")

@@ -1,5 +1,6 @@
-"""GPU parity of the head dims below 64 (generic_d.hip: one wavefront per
-(sequence, head), the recurrence token by token) against the oracle, whose
+"""GPU parity of the head dims below 64 (one token, or a few on many sequences:
+generic_d.hip, one wavefront per (sequence, head); else and the backward:
+chunk_f32.hip, fp32 chunks) against the oracle, whose
 restatement takes any D: the chunked prefill (chunked_ssd.py:48-184, with its
 own chunk size or none -- the result does not depend on it) and the dense
 branch's double clamp (attention.py:160-202), the decode step

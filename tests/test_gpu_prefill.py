@@ -6,6 +6,7 @@ import torch
 
 from oracle import oracle as O
 from prime_moment_attention import _lib
+from selective_ref import selective_forward
 from prime_moment_attention.chunked_ssd import chunked_prime_ssd_core, prime_prefill
 
 from gpu_util import (TOL_BF16, TOL_F32, assert_close, assert_state_close, random_state,
@@ -184,9 +185,9 @@ def test_prefill_segmented_equals_one_segment(with_state):
 @pytest.mark.parametrize("selective", [False, True])
 @pytest.mark.parametrize("L", [64, 65, 129, 513, 1000])
 def test_prefill_short_segments_equal_one_segment(L, selective, dtype):
-    """The plan splits down to one chunk per segment (a ragged last one too): with
-    the workspace it asks for against one segment per sequence, grouped k/v and an
-    incoming state.  The two differ by the rounding of a state that is summed per
+    """Around the lengths where the plan begins to split (test_prefill_short_segments_
+    match_float64 names them): with the workspace it asks for against one segment per
+    sequence, grouped k/v and an incoming state.  Where it splits the two differ by the rounding of a state that is summed per
     segment: the tolerances of the segmented tests of longer sequences."""
     B, H, Hkv = 1, 6, 2
     q, _, _ = O.make_inputs((B, H, L, D), seed=70, bf16=True)
@@ -207,3 +208,49 @@ def test_prefill_short_segments_equal_one_segment(L, selective, dtype):
     tol = 2e-3 if dtype == torch.bfloat16 else 1e-4
     assert_close(outs[0][0], outs[1][0], tol, "y")
     assert_state_close(outs[0][1], outs[1][1], tol)
+
+
+@pytest.mark.parametrize("dtype,selective,L", [
+    (torch.bfloat16, False, 64 * 9 + 1), (torch.bfloat16, False, 1000), (torch.float32, False, 64 * 3 + 1),
+    (torch.float32, False, 250), (torch.float32, False, 513), (torch.bfloat16, True, 64 * 7 + 1),
+    (torch.bfloat16, True, 1000), (torch.float32, True, 129), (torch.float32, True, 190), (torch.float32, True, 513)])
+def test_prefill_short_segments_match_float64(dtype, selective, L):
+    """Lengths from the first that each kernel's plan splits at this batch (one chunk per
+    segment, a ragged last one): the state-only pass is launched, and not without a
+    workspace, and both agree with float64."""
+    B, H, Hkv = 1, 6, 2
+    q, _, _ = O.make_inputs((B, H, L, D), seed=80, bf16=True)
+    _, k, v = O.make_inputs((B, Hkv, L, D), seed=81, bf16=True)
+    st0 = random_state(B * H, D, 82)
+    lam = np.linspace(0.99, 0.9999, H).astype(np.float32)
+    ld = (-0.02 * np.random.default_rng(83).random((B, H, L))).astype(np.float32)
+    ke, ve = np.repeat(k, H // Hkv, 1), np.repeat(v, H // Hkv, 1)
+    if selective:
+        t64 = lambda x: torch.from_numpy(np.asarray(x, np.float64))
+        shapes = [(B, H, D), (B, H, D, D), (B, H, D, D), (B, H, 1), (B, H, D), (B, H, D)]
+        yo, so = selective_forward(t64(q), t64(ke), t64(ve), t64(ld), torch.full((B, H), 0.7, dtype=torch.float64),
+                                   1.0, tuple(t64(x).reshape(s) for x, s in zip(st0, shapes)))
+        yo, so = yo.numpy(), [x.numpy() for x in so]
+    else:
+        yo, so = O.chunked(*(x.reshape(H, L, D) for x in (q, ke, ve)), lam.astype(np.float64), eps=1.0, chunk=64,
+                           state=st0)
+    tq, tk, tv = (to_dev(x, dtype) for x in (q, k, v))
+    st_in = state_to_dev(st0, B, H, D)
+    tol = TOL_BF16 if dtype == torch.bfloat16 else TOL_F32
+    for split, ws in ((1, None), (0, torch.empty(0, dtype=torch.uint8, device=dev()))):
+        y, st = torch.empty(B, H, L, D, device=dev()), _lib.new_state(B, H, D, dev())
+        _lib.timer_enable(_lib.KERNEL_PREFILL_SEGMENTS)
+        _lib.timer_reset()
+        try:
+            if selective:
+                _lib.selective_prefill(tq, tk, tv, to_dev(ld), torch.full((H,), 0.7, device=dev()), 1.0, st_in, y, st,
+                                       workspace=ws)
+            else:
+                _lib.chunked_prefill(tq, tk, tv, to_dev(lam), 1.0, 64, st_in, y, st, 0, workspace=ws)
+            torch.cuda.synchronize()
+            assert _lib.timer_read(_lib.KERNEL_PREFILL_SEGMENTS)[1] == split
+        finally:
+            _lib.timer_enable()
+        assert_close(to_np(y).reshape(yo.shape), yo, tol, "y")
+        for x, r in zip(st, so):
+            assert_close(to_np(x).reshape(r.shape), r, tol, "state")
