@@ -47,19 +47,13 @@
 // (a single token, and a few tokens on many sequences, keep a kernel that goes token by token:
 // generic_d.hip).
 
+#include "f32_common.h"
 #include "head_row.h"
-#include "prefill_common.h"
 
 namespace prime {
 namespace {
 
 constexpr int kT = 1024, kNW = kT / kWave;
-
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
-__device__ __forceinline__ void st4(float *p, f32x4 v) { *reinterpret_cast<f32x4 *>(p) = v; }
 
 template <int DP>
 struct Dim {
@@ -112,12 +106,6 @@ struct Op3 {
 struct OpV {
     f32x4 a, b;
 };
-
-// lower 16x16 tile t (0..9) -> (row block, column block)
-__device__ __forceinline__ void lower_tile(int t, int &ib, int &jb) {
-    ib = t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3;
-    jb = t - ib * (ib + 1) / 2;
-}
 
 // NE consecutive elements of a row from column d0 as stored, from clamped addresses:
 // nothing is masked or converted here, so that no wait sits between a load and the

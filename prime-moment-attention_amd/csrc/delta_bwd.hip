@@ -43,7 +43,7 @@
 
 #include <algorithm>
 
-#include "delta_f32_common.h"
+#include "f32_common.h"
 
 namespace prime {
 namespace {

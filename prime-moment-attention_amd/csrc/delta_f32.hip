@@ -24,7 +24,7 @@
 //   R0 [8 fb][4 dv][64 lanes]   R0^T accumulator tiles (4 floats per lane)
 //   Y0 [4 dv][4 tb][64 lanes]   Y0^T accumulator tiles
 
-#include "delta_f32_common.h"
+#include "f32_common.h"
 
 namespace prime {
 namespace {

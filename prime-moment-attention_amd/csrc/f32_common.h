@@ -1,6 +1,6 @@
-// Device helpers shared by the fp32 delta-rule kernels (delta_f32.hip and
+// Device helpers shared by the fp32 kernels (chunk_f32.hip, delta_f32.hip and
 // delta_bwd.hip): the fp32 MFMA, 16-byte accesses, the lower tiles of a chunk's
-// 64 x 64 blocks and the chunk's triangular solve.
+// 64 x 64 blocks and the delta chunk's triangular solve.
 #pragma once
 
 #include "prefill_common.h"
