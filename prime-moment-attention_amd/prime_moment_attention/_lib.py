@@ -526,10 +526,11 @@ def plain_eager(*ts: torch.Tensor) -> bool:
     forward-mode level or functorch transform (their tensors look plain), no dispatch or
     function mode or tracer that has to see the call.  (1.2 us)"""
     C = torch._C
-    return (not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+    return (not torch.compiler.is_compiling()  # (first: a compiler's tracer goes no further)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
             and forward_ad._current_level < 0 and C._functorch.peek_interpreter_stack() is None
             and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
-            and C._get_tracing_state() is None and not torch.compiler.is_compiling())
+            and C._get_tracing_state() is None)
 
 
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
