@@ -521,16 +521,18 @@ def linear_fused(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, epilogue: 
 ROWS_LINEAR_MAX = 512
 
 
-def plain_eager(*ts: torch.Tensor) -> bool:
-    """Whether torch would only compute an operation over ts: no autograd recording, no
+_functorch_level = torch._C._functorch.peek_interpreter_stack
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_is_tracing = torch._C._is_tracing
+
+
+def plain_eager(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether torch would only compute an operation over a and b: no autograd recording, no
     forward-mode level or functorch transform (their tensors look plain), no dispatch or
-    function mode or tracer that has to see the call.  (1.2 us)"""
-    C = torch._C
-    return (not torch.compiler.is_compiling()  # (first: a compiler's tracer goes no further)
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
-            and forward_ad._current_level < 0 and C._functorch.peek_interpreter_stack() is None
-            and C._len_torch_dispatch_stack() == 0 and C._len_torch_function_stack() == 0
-            and C._get_tracing_state() is None)
+    function mode or tracer that has to see the call.  (1 us)"""
+    return (not ((a.requires_grad or b.requires_grad) and torch.is_grad_enabled())
+            and forward_ad._current_level < 0 and _functorch_level() is None
+            and _dispatch_modes() == 0 and _function_modes() == 0 and not _is_tracing())
 
 
 def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -538,12 +540,13 @@ def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     measured, 16-byte rows, plain dense tensors of one device, and nothing recording,
     transforming or recasting the call (``plain_eager``).  An x of another width is left to
     torch, which refuses it."""
-    K = x.shape[-1]
-    return (w.shape[1] == K and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.is_cuda and w.device == x.device
-            and 0 < x.numel() <= ROWS_LINEAR_MAX * K and K % 128 == 0 and K <= 1024 and w.shape[0] % 32 == 0
-            and w.shape[0] <= 3072 and x.is_contiguous() and w.is_contiguous()
+    if x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or w.dim() != 2:
+        return False
+    N, K = w.shape
+    return (x.shape[-1] == K and K % 128 == 0 and K <= 1024 and N % 32 == 0 and N <= 3072
+            and 0 < x.numel() <= ROWS_LINEAR_MAX * K and x.is_cuda and w.get_device() == x.get_device()
             and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
-            and plain_eager(x, w) and not torch.is_autocast_enabled()
+            and x.is_contiguous() and w.is_contiguous() and plain_eager(x, w) and not torch.is_autocast_enabled()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
@@ -551,7 +554,7 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w.T by prime_linear_fused (``rows_linear_ok``): x [..., K] -> [..., N]."""
     N, K = w.shape
     M = x.numel() // K
-    out = torch.empty(*x.shape[:-1], N, device=x.device, dtype=x.dtype)
+    out = x.new_empty((*x.shape[:-1], N))
     rc = load().prime_linear_fused(x.data_ptr(), w.data_ptr(), None, out.data_ptr(), M, N, K, K, K, N, N, PRIME_BF16,
                                    EPILOGUE_NONE, 0.0, _stream(x.device))
     _check(rc, "prime_linear_fused")
