@@ -211,8 +211,9 @@ int device_cus() {
 // before they slow each other), the scan and launches (`fixed`) and each slot's
 // traffic (`slot`).  The five figures of each kernel are fitted to 13 shapes from
 // 12 x 128 to 96 x 8192 tokens with every G (times within 10 % of the model at the
-// chosen G): the plan is within 0.5 % of the best G on fp32 and bf16, 13 % at worst
-// (selective bf16, 12 x 1000).  12 x 512 fp32: 8 segments 25.9 us, 2 segments 44.3;
+// chosen G): there the plan is within 0.5 % of the best G on fp32 and bf16, 6 % at worst
+// (selective bf16, 12 x 1000).  Over 4 to 48 sequences of 1024 to 32,768 tokens it is within 8 %
+// (bf16, 4 x 1024: 19.3 us against 17.9), 14 % for selective bf16 (4 x 4096: 31.0 against 26.9).  12 x 512 fp32: 8 segments 25.9 us, 2 segments 44.3;
 // 12 x 512 bf16: one 20.1, 2 segments 27.3; 96 x 2048 bf16: one 59.8, 2 68.5;
 // 96 x 8192 bf16: 8 160.5, 7 169.8; 48 x 777 selective fp32: 5 56.8, 3 78.8.
 namespace {
@@ -821,12 +822,18 @@ __global__ __launch_bounds__(256) void segment_scan_kernel(const PrefillArgs a) 
     for (int s0 = 0; s0 < ns; s0 += 8) {
         float d[8], f[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int s = s0 + t < ns ? s0 + t : ns - 1;  // clamped (unused past ns)
-            d[t] = slot[static_cast<size_t>(s) * kWsStride];
-            // selective: segment s's own decay, stored beside its slot's state
-            f[t] = sel ? exp2f(slot[static_cast<size_t>(s) * kWsStride + kWsDecay - e])
-                       : (s == a.G - 1 ? lLast : lT);
+        for (int t = 0; t < 8; ++t) d[t] = slot[static_cast<size_t>(min(s0 + t, ns - 1)) * kWsStride];
+        if (sel) {
+            // segment s's own decay, stored beside its slot's state (the loads apart from what is
+            // done with them: with exp2f behind each the wave waited for one after the other,
+            // 0.25 us a segment)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) f[t] = slot[static_cast<size_t>(min(s0 + t, ns - 1)) * kWsStride + kWsDecay - e];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) f[t] = exp2f(f[t]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) f[t] = s0 + t >= a.G - 1 ? lLast : lT;
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {

@@ -213,10 +213,11 @@ def test_prefill_short_segments_equal_one_segment(L, selective, dtype):
 @pytest.mark.parametrize("dtype,selective,L", [
     (torch.bfloat16, False, 64 * 9 + 1), (torch.bfloat16, False, 1000), (torch.float32, False, 64 * 3 + 1),
     (torch.float32, False, 250), (torch.float32, False, 513), (torch.bfloat16, True, 64 * 7 + 1),
-    (torch.bfloat16, True, 1000), (torch.float32, True, 129), (torch.float32, True, 190), (torch.float32, True, 513)])
+    (torch.bfloat16, True, 1000), (torch.bfloat16, True, 64 * 41 + 5), (torch.float32, True, 129),
+    (torch.float32, True, 190), (torch.float32, True, 513), (torch.float32, True, 64 * 41 + 5)])
 def test_prefill_short_segments_match_float64(dtype, selective, L):
     """Lengths from the first that each kernel's plan splits at this batch (one chunk per
-    segment, a ragged last one): the state-only pass is launched, and not without a
+    segment, a ragged last one; then more segments than the scan takes at a time): the state-only pass is launched, and not without a
     workspace, and both agree with float64."""
     B, H, Hkv = 1, 6, 2
     q, _, _ = O.make_inputs((B, H, L, D), seed=80, bf16=True)
