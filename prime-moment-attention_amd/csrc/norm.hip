@@ -336,7 +336,8 @@ hipError_t launch_add_rmsnorm(const RmsNormArgs &a, hipStream_t stream) {
 // Bound by its read of both projections (403 MB at 131,072 tokens x 12 heads of 64 in
 // bf16); as torch ops that read was sigmoid, cast, mean and transposes, 1.36 ms there.
 // A workgroup takes 64 tokens x 4 heads, 8 lanes a row, and turns the sums round in LDS so
-// that each head's tokens are written together.  bf16 and fp16 take the hardware's exp2
+// that each head's tokens are written together.  The tokens of all sequences are numbered
+// through (a workgroup per sequence made a decode batch of 600 one token in 64 each: 40 us).  bf16 and fp16 take the hardware's exp2
 // and reciprocal: after the rounding to 16 bits every input gives torch's sigmoid, but for
 // the three bf16 values near -88 whose sigmoid is subnormal (5e-39), which give 0; fp32 the
 // full forms.
@@ -352,8 +353,8 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict
     __shared__ float sSum[2][kGateHeads][kGateTok + 1];
     constexpr int ES = DT == PRIME_F32 ? 4 : 2;
     const int tid = threadIdx.x, part = tid & 7;
-    const int t0 = blockIdx.x * kGateTok, h0 = blockIdx.y * kGateHeads;
-    const int nt = min(kGateTok, L - t0), nh = min(kGateHeads, H - h0);
+    const int h0 = blockIdx.y * kGateHeads, nh = min(kGateHeads, H - h0);
+    const int64_t ntok = static_cast<int64_t>(B) * L;
     auto sig = [](float x) {
         if constexpr (DT == PRIME_F32) return 1.0f / (1.0f + expf(-x));
         const float s = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * x));
@@ -377,15 +378,32 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict
         }
         return a;
     };
-    for (int64_t b = blockIdx.z; b < B; b += gridDim.z) {
-        const char *eb = static_cast<const char *>(erase) + (b * e_sb + static_cast<int64_t>(t0) * e_sl) * ES;
-        const char *wb = static_cast<const char *>(write) + (b * w_sb + static_cast<int64_t>(t0) * w_sl) * ES;
-        // row rr = 4 token + head: 8 rounds of 32 rows
+    for (int64_t n0 = static_cast<int64_t>(blockIdx.x) * kGateTok; n0 < ntok;
+         n0 += static_cast<int64_t>(gridDim.x) * kGateTok) {
+        const int64_t b0 = n0 / L;
+        const uint32_t t0 = static_cast<uint32_t>(n0 - b0 * L);
+        const int nt = static_cast<int>(min(static_cast<int64_t>(kGateTok), ntok - n0));
+        const bool one = t0 + kGateTok <= static_cast<uint32_t>(L);  // the tile lies in sequence b0
+        // token tk of the tile: sequence b, token t
+        auto place = [&](int tk, int64_t &b, uint32_t &t) {
+            b = b0;
+            t = t0 + tk;
+            if (!one) {
+                const uint32_t d = t / static_cast<uint32_t>(L);
+                b += d;
+                t -= d * L;
+            }
+        };
+        // row rr = 4 token + head: up to 8 rounds of 32 rows
 #pragma unroll 4
-        for (int it = 0; it < kGateTok * kGateHeads / 32; ++it) {
+        for (int it = 0; it < (nt + 7) / 8; ++it) {
             const int rr = it * 32 + (tid >> 3), tk = rr / kGateHeads, hh = rr % kGateHeads;
-            const int64_t t = min(tk, nt - 1), h = h0 + min(hh, nh - 1);
-            const char *pe = eb + (t * e_sl + h * D) * ES, *pw = wb + (t * w_sl + h * D) * ES;
+            int64_t b;
+            uint32_t t;
+            place(min(tk, nt - 1), b, t);
+            const int64_t h = h0 + min(hh, nh - 1);
+            const char *pe = static_cast<const char *>(erase) + (b * e_sb + t * e_sl + h * D) * ES;
+            const char *pw = static_cast<const char *>(write) + (b * w_sb + t * w_sl + h * D) * ES;
             float se = 0.f, sw = 0.f;
             if constexpr (VEC) {
                 u32x4 re[DT == PRIME_F32 ? 2 : 1], rw[DT == PRIME_F32 ? 2 : 1];
@@ -416,7 +434,10 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict
         __syncthreads();
         const int tk = tid & 63, hh = tid >> 6;
         if (tk < nt && hh < nh) {
-            const int64_t o = (b * H + h0 + hh) * L + t0 + tk;
+            int64_t b;
+            uint32_t t;
+            place(tk, b, t);
+            const int64_t o = (b * H + h0 + hh) * L + t;
             beta[o] = sSum[1][hh][tk] * 0.5f;
             alpha[o] = decay * (1.0f - sSum[0][hh][tk] * 0.5f);
         }
@@ -425,8 +446,9 @@ __global__ __launch_bounds__(256) void delta_gates_kernel(const void *__restrict
 }
 
 hipError_t launch_delta_gates(const DeltaGateArgs &a, hipStream_t stream) {
-    // (a grid's z ends at 65,535: workgroups take further sequences in turn)
-    const dim3 g((a.L + kGateTok - 1) / kGateTok, (a.H + kGateHeads - 1) / kGateHeads, std::min(a.B, 65535)), blk(256);
+    // (a grid of 2^22 workgroups at most: they take further tiles in turn)
+    const int64_t tiles = (static_cast<int64_t>(a.B) * a.L + kGateTok - 1) / kGateTok;
+    const dim3 g(static_cast<uint32_t>(std::min<int64_t>(tiles, 1 << 22)), (a.H + kGateHeads - 1) / kGateHeads), blk(256);
     auto al = [](const void *p, int64_t sb, int64_t sl, int64_t es) {
         return reinterpret_cast<uintptr_t>(p) % 16 == 0 && sb * es % 16 == 0 && sl * es % 16 == 0;
     };

@@ -384,3 +384,17 @@ def test_delta_gates_sigmoid_is_torchs_for_every_value(dtype):
     ra = (0.9995 * (1.0 - s * 0.5)).view(1, 512, 128).transpose(1, 2)
     for got, want in ((beta, rb), (alpha, ra)):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,H,L,D", [(130, 5, 1, 64), (9, 4, 7, 64), (70, 3, 3, 64), (3, 6, 63, 64), (5, 2, 65, 64),
+                                     (2, 4, 96, 64), (100, 3, 2, 8), (1, 4, 200, 64)])
+def test_delta_gates_tiles_over_sequences(dtype, B, H, L, D):
+    """Tiles of 64 tokens that hold many short sequences, or the end of one and the start
+    of the next, at batch and token strides of a wider buffer: torch's values for each."""
+    g = torch.Generator().manual_seed(B * L)
+    pre = [(torch.randn(B, L + 2, H * D + 8, generator=g) * 2).to(dev(), dtype)[:, 1:1 + L, :H * D] for _ in range(2)]
+    beta, alpha = _lib.delta_gates(pre[0], pre[1], 0.9995, H, D)
+    mean = lambda t: torch.sigmoid(t).reshape(B, L, H, D).float().mean(-1).transpose(1, 2)
+    assert (beta - mean(pre[1]) * 0.5).abs().max() <= 2e-7  # (the order of D fp32 additions)
+    assert (alpha - 0.9995 * (1.0 - mean(pre[0]) * 0.5)).abs().max() <= 2e-7
