@@ -30,31 +30,34 @@ namespace {
 constexpr int kGD = 64;     // lanes: value columns 0 .. D-1 and the ones column D (D < 64)
 constexpr int kGC = 64;     // rows per workgroup of the head LayerNorm
 constexpr int kGP = kGD + 1;
+constexpr int kFew = 16;    // tokens of a call that goes token by token, at most
 
 }  // namespace
 
-// MULTI: a.L tokens in order, else one.
-template <bool MULTI>
+// T: tokens staged (one, or up to T = kFew of a call), taken in order.
+template <int T>
 __global__ __launch_bounds__(kGD) void generic_step_kernel(const GenericArgs a) {
-    __shared__ float sq[kGP], sk[kGP], sdec[1];
+    __shared__ float sq[T][kGP], sk[T][kGP], sv[T][kGP], sdec[T];
     __shared__ float sKin[3][kGP];  // incoming K1, K2 (dense clamp), K0 at [2][0]
     const int lane = threadIdx.x, bh = blockIdx.x;
     const int b = bh / a.H, h = bh - b * a.H, hk = h / a.group, D = a.D;
+    const int L = T == 1 ? 1 : a.L;
     const bool col = lane <= D;
     const bool sel = a.selective != 0;
     // the second-order weights: k*k and q*q/2 (base), (beta k)*(beta k)/2 and q*q (selective)
     const float ck2 = sel ? 0.5f : 1.0f, cq2 = sel ? 1.0f : 0.5f;
     const size_t o1 = static_cast<size_t>(bh) * D * D, o0 = static_cast<size_t>(bh) * D;
-    // ---- a token: q and k for LDS, v in its lane
-    float qx, kx, vx;
-    auto load_token = [&](int t) {
-        qx = lane < D ? load_elem(a.q, b * a.q_sb + h * a.q_sh + t * a.q_sl + lane, a.dt_q) : 0.f;
-        kx = lane < D ? load_elem(a.k, b * a.k_sb + hk * a.k_sh + t * a.k_sl + lane, a.dt_k) : 0.f;
-        vx = lane < D ? load_elem(a.v, b * a.v_sb + hk * a.v_sh + t * a.v_sl + lane, a.dt_v) : (lane == D ? 1.0f : 0.0f);
-    };
-    load_token(0);
-    sq[lane] = qx;
-    sk[lane] = kx;
+    // ---- the tokens' rows in LDS, v with the ones column
+    {
+        const int64_t qo = b * a.q_sb + h * a.q_sh + lane, ko = b * a.k_sb + hk * a.k_sh + lane,
+                      vo = b * a.v_sb + hk * a.v_sh + lane;
+#pragma unroll 4
+        for (int t = 0; t < L; ++t) {
+            sq[t][lane] = lane < D ? load_elem(a.q, qo + t * a.q_sl, a.dt_q) : 0.f;
+            sk[t][lane] = lane < D ? load_elem(a.k, ko + t * a.k_sl, a.dt_k) : 0.f;
+            sv[t][lane] = lane < D ? load_elem(a.v, vo + t * a.v_sl, a.dt_v) : (lane == D ? 1.0f : 0.0f);
+        }
+    }
     float S0 = 0.f, S1[kGD - 1], S2[kGD - 1];
 #pragma unroll
     for (int i = 0; i < kGD - 1; ++i) {
@@ -73,49 +76,47 @@ __global__ __launch_bounds__(kGD) void generic_step_kernel(const GenericArgs a) 
         }
         if (lane == 0) sKin[2][0] = a.k0i[bh];
     }
-    float lin = 1.f;  // the incoming state's decay
-    for (int t = 0; t < (MULTI ? a.L : 1); ++t) {
-        if (MULTI && t) {
-            __syncthreads();  // (the last token's reads)
-            sq[lane] = qx;
-            sk[lane] = kx;
+    __syncthreads();
+    if (a.qk_norm) {  // a row per lane
+        const int t = lane & 31;
+        if (t < L) {
+            if (lane < 32) generic_ln_row(sq[t], D, a.qn_w, a.qn_b, a.dt_norm, a.ln_eps, a.q_scale, a.dt_q);
+            else generic_ln_row(sk[t], D, a.kn_w, a.kn_b, a.dt_norm, a.ln_eps, 1.0f, a.dt_k);
         }
-        const float vj = vx;
-        if (MULTI && t + 1 < a.L) load_token(t + 1);
         __syncthreads();
-        if (a.qk_norm) {
-            if (lane == 0) generic_ln_row(sq, D, a.qn_w, a.qn_b, a.dt_norm, a.ln_eps, a.q_scale, a.dt_q);
-            if (lane == 1) generic_ln_row(sk, D, a.kn_w, a.kn_b, a.dt_norm, a.ln_eps, 1.0f, a.dt_k);
-            __syncthreads();
-        }
-        if (sel) {
-            sk[lane] *= a.k_scale[h];
-            if (lane == 0) {
-                float lam_t;
-                if (a.log_decay) {
-                    lam_t = expf(a.log_decay[MULTI ? static_cast<size_t>(bh) * a.L + t : bh]);
-                } else if (a.decay_bh) {
-                    lam_t = a.decay_bh[bh];
-                } else {
-                    // selective.py:368, 386: Delta = clamp(softplus(s)), each stage
-                    // rounded to the step's dtype as the module's tensors are
-                    const float sv0 = load_elem(a.step, b * a.step_sb + h, a.dt_step);
-                    float d = sv0 > 20.f ? sv0 : log1pf(expf(sv0));
-                    d = round_dt(d, a.dt_step);
-                    d = round_dt(fminf(fmaxf(d, a.step_min), a.step_max), a.dt_step);
-                    lam_t = expf(-d / a.tau[h]);
-                }
-                sdec[0] = lam_t;
+    }
+    if (sel) {
+        const float ks = a.k_scale[h];
+        for (int t = 0; t < L; ++t) sk[t][lane] *= ks;
+        if (lane < L) {
+            float lam_t;
+            if (a.log_decay) {
+                lam_t = expf(a.log_decay[static_cast<size_t>(bh) * L + lane]);
+            } else if (a.decay_bh) {
+                lam_t = a.decay_bh[bh];
+            } else {
+                // selective.py:368, 386: Delta = clamp(softplus(s)), each stage
+                // rounded to the step's dtype as the module's tensors are
+                const float sv0 = load_elem(a.step, b * a.step_sb + h, a.dt_step);
+                float d = sv0 > 20.f ? sv0 : log1pf(expf(sv0));
+                d = round_dt(d, a.dt_step);
+                d = round_dt(fminf(fmaxf(d, a.step_min), a.step_max), a.dt_step);
+                lam_t = expf(-d / a.tau[h]);
             }
-            __syncthreads();
+            sdec[lane] = lam_t;
         }
-        const float lt = sel ? sdec[0] : a.decay[h];
+        __syncthreads();
+    }
+    const float lh = sel ? 0.f : a.decay[h];
+    float lin = 1.f;  // the incoming state's decay
+    for (int t = 0; t < L; ++t) {
+        const float lt = sel ? sdec[t] : lh, vj = sv[t][lane];
         S0 = lt * S0 + vj;
         float num = S0;
 #pragma unroll
         for (int i = 0; i < kGD - 1; ++i) {
             if (i < D) {
-                const float ki = sk[i], qi = sq[i];
+                const float ki = sk[t][i], qi = sq[t][i];
                 S1[i] = fmaf(lt, S1[i], ki * vj);
                 S2[i] = fmaf(lt, S2[i], ck2 * ki * ki * vj);
                 num = fmaf(qi, S1[i], num);
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(kGD) void generic_step_kernel(const GenericArgs a) 
             lin *= lt;
             float di = sKin[2][0];
             for (int i = 0; i < D; ++i) {
-                const float qi = sq[i];
+                const float qi = sq[t][i];
                 di = fmaf(qi, sKin[0][i], di);
                 di = fmaf(0.5f * qi * qi, sKin[1][i], di);
             }
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(kGD) void generic_step_kernel(const GenericArgs a) 
             den_c = fmaxf(den, a.eps);
         }
         if (lane < D && a.y)
-            store_elem(a.y, b * a.y_sb + h * a.y_sh + (MULTI ? t * a.y_sl : 0) + lane, a.dt_y, num / den_c);
+            store_elem(a.y, b * a.y_sb + h * a.y_sh + (T == 1 ? 0 : t * a.y_sl) + lane, a.dt_y, num / den_c);
     }
     if (a.s1o && col) {
 #pragma unroll
@@ -159,23 +160,31 @@ __global__ __launch_bounds__(kGD) void generic_step_kernel(const GenericArgs a) 
 }
 
 // Few tokens on many sequences go token by token: a chunk costs its workgroup the same for
-// 2 tokens as for 64, and with several workgroups a CU those add up.  With s sequences a CU
-// the line lies at s + 1 tokens, 12 at most: at D = 32 with states, the times of the token
-// kernel over the chunk kernel are 1.00 at s = 3 and 4 tokens (1.28 at 2 sequences and 3
-// tokens), 0.84 at 4 and 4 (1.02 at 6 tokens), 0.86 at 16 and 12 (1.07 at 16); at D = 48 0.79,
-// 0.66 and 0.65.  A QK LayerNorm on load is one lane's work per token here and one lane a
-// token there: (s + 1) / 2 tokens, 5 at most (D = 32: 0.98 at 3 and 2, 0.79 at 4 and 2 and 1.09
-// at 3, 0.75 at 8 and 4, 0.89 at 16 and 5 and 1.04 at 6).  16,384 sequences of 2 tokens: 608 us in
-// chunks, 204 token by token (D = 32); 4096 of 2 at D = 48 236 and 65.
+// 2 tokens as for 64, and the chunk kernel runs r = ceil(sequences / CUs) rounds of them.  The
+// lines (tokens up to which this kernel was the faster one, at head dims 8 to 63 and 64 to 8192
+// sequences) by what a call carries:
+//   no state in or out   2 r - 1  from r = 2 (D = 32, r = 2: 15.1 us against 17.1 at 3 tokens, 18.5 at 4);
+//                        above D = 32, whose chunks cost more, 3 r - 3
+//   states               2 r - 2  from r = 3, 14 at most (D = 32, r = 3: 28.3 against 29.2 at 4, 34.7 at 6)
+//   the dense clamp's    2 r - 4, 10 at most (the incoming denominator is read once per token)
+//   a QK LayerNorm on load, whose serial row each lane does once here and there:
+//                        4 r - 4, with states 4 r - 6, with the dense clamp's 4 r - 8 and 10 at most
+// 8192 sequences of 2 tokens at D = 32: 294 us in chunks, 81 token by token; 600 of 2 at D = 48
+// without states 40 and 13.
 static bool token_by_token(const GenericArgs &a) {
-    const int64_t s = static_cast<int64_t>(a.B) * a.H / device_cus();
-    return s >= 3 && a.L <= (a.qk_norm ? std::min<int64_t>((s + 1) / 2, 5) : std::min<int64_t>(s + 1, 12));
+    const int64_t cus = device_cus(), r = (static_cast<int64_t>(a.B) * a.H + cus - 1) / cus;
+    const bool state = a.s1i || a.s1o, dense = a.dense_clamp && a.s1i;
+    const int64_t line = a.qk_norm ? 4 * r - (dense ? 8 : state ? 6 : 4)
+                         : dense   ? 2 * r - 4
+                         : state   ? (r < 3 ? 0 : 2 * r - 2)
+                                   : (a.D > 32 ? 3 * r - 3 : 2 * r - 1);
+    return a.L <= std::min<int64_t>(line, dense ? 10 : state && !a.qk_norm ? 14 : kFew);
 }
 
 hipError_t launch_generic_prefill(GenericArgs a, hipStream_t stream) {
     const dim3 grid(a.B * a.H), block(kGD);
-    if (a.L == 1) hipLaunchKernelGGL(generic_step_kernel<false>, grid, block, 0, stream, a);
-    else if (token_by_token(a)) hipLaunchKernelGGL(generic_step_kernel<true>, grid, block, 0, stream, a);
+    if (a.L == 1) hipLaunchKernelGGL(generic_step_kernel<1>, grid, block, 0, stream, a);
+    else if (token_by_token(a)) hipLaunchKernelGGL(generic_step_kernel<kFew>, grid, block, 0, stream, a);
     else return launch_chunk_f32_prefill(a, stream);
     return hipGetLastError();
 }
