@@ -593,7 +593,7 @@ def _prefill_args(q, k, v, decay, eps, chunk, state_in, y, state_out, flags, wor
     _check_state(state_in, B, H, D, "state_in")
     _check_state(state_out, B, H, D, "state_out")
     if workspace is None:
-        nbytes = workspace_size(B, H, Lq, flags)
+        nbytes = workspace_size(B, H, Lq, flags) if D == 64 else 0  # (below 64 no call is split)
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
     elif workspace.numel() == 0:
         workspace = None

@@ -659,3 +659,31 @@ def test_generic_few_tokens_on_many_sequences(form, D, L):
     for n in (slice(0, 8), slice(B - 8, B)):
         for x, r in zip(whole, run(n)):
             assert (x[n] - r).abs().max() <= tol * r.abs().max()
+
+
+@pytest.mark.parametrize("selective", [False, True])
+def test_generic_prefill_allocates_no_workspace(monkeypatch, selective):
+    """Head dims below 64 run one segment a sequence: where D = 64 gets segment slots by
+    default, they get none, and the outputs are those of an explicit empty workspace."""
+    B, H, L, D = 1, 4, 1000, 32
+    assert _lib.workspace_size(B, H, L) > 0
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(B, H, L, D, generator=g).to(dev()) for _ in range(3))
+    lam, ld = torch.linspace(0.9, 0.999, H, device=dev()), -torch.rand(B, H, L, generator=g).to(dev())
+    byte_buffers, empty = [], torch.empty
+
+    def run(ws):
+        y = empty(B, H, L, D, device=dev())
+        if selective:
+            _lib.selective_prefill(q, k, v, ld, lam, 1.0, None, y, None, workspace=ws)
+        else:
+            _lib.chunked_prefill(q, k, v, lam, 1.0, 64, None, y, None, workspace=ws)
+        return y
+    ref = run(empty(0, dtype=torch.uint8, device=dev()))
+
+    def watched(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            byte_buffers.append(a)
+        return empty(*a, **kw)
+    monkeypatch.setattr(torch, "empty", watched)
+    assert torch.equal(run(None), ref) and not byte_buffers
