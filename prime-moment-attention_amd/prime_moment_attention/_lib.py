@@ -523,7 +523,8 @@ ROWS_LINEAR_MAX = 512
 
 _functorch_level = torch._C._functorch.peek_interpreter_stack
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
-_is_tracing = torch._C._is_tracing
+_is_tracing, _is_autocast_enabled = torch._C._is_tracing, torch.is_autocast_enabled
+_BF16 = torch.bfloat16
 
 
 def plain_eager(a: torch.Tensor, b: torch.Tensor) -> bool:
@@ -540,14 +541,15 @@ def rows_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     measured, 16-byte rows, plain dense tensors of one device, and nothing recording,
     transforming or recasting the call (``plain_eager``).  An x of another width is left to
     torch, which refuses it."""
-    if x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or w.dim() != 2:
+    if x.dtype is not _BF16 or w.dtype is not _BF16 or w.dim() != 2:
         return False
     N, K = w.shape
+    tw = type(w)
     return (x.shape[-1] == K and K % 128 == 0 and K <= 1024 and N % 32 == 0 and N <= 3072
             and 0 < x.numel() <= ROWS_LINEAR_MAX * K and x.is_cuda and w.get_device() == x.get_device()
-            and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
-            and x.is_contiguous() and w.is_contiguous() and plain_eager(x, w) and not torch.is_autocast_enabled()
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and type(x) is torch.Tensor and (tw is torch.nn.Parameter or tw is torch.Tensor)
+            and x.is_contiguous() and w.is_contiguous() and plain_eager(x, w) and not _is_autocast_enabled()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -91,9 +91,10 @@ _LINEAR_FORWARD = nn.Linear.forward
 def _plain_linear(m: nn.Module) -> bool:
     """Whether m(x) is x @ weight.T and nothing else: an nn.Linear without bias or hooks
     whose ``forward`` nobody has replaced, on the instance (offloading, adapter and
-    quantisation wrappers do) or on the class."""
-    g = torch.nn.modules.module
-    return (type(m) is nn.Linear and m.bias is None and "forward" not in m.__dict__
+    quantisation wrappers do) or on the class.  (The bias is looked up where an nn.Linear keeps
+    it: nn.Module's own attribute lookup takes 0.5 us.)"""
+    g, d = torch.nn.modules.module, m.__dict__
+    return (type(m) is nn.Linear and m._parameters.get("bias", m) is None and "bias" not in d and "forward" not in d
             and nn.Linear.forward is _LINEAR_FORWARD
             and not (m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks
                      or g._global_forward_pre_hooks))
@@ -102,8 +103,10 @@ def _plain_linear(m: nn.Module) -> bool:
 def project_out(proj: nn.Module, y: torch.Tensor) -> torch.Tensor:
     """``proj(y)``: for few rows through the row kernel, where the module is a plain
     nn.Linear and torch has nothing to record or transform."""
-    if _plain_linear(proj) and _lib.rows_linear_ok(y, proj.weight):
-        return _lib.rows_linear(y, proj.weight)
+    if _plain_linear(proj):
+        w = proj.weight
+        if _lib.rows_linear_ok(y, w):
+            return _lib.rows_linear(y, w)
     return proj(y)
 
 

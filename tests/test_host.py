@@ -147,3 +147,29 @@ def test_selective_gate_constants_follow_parameters():
     assert tau2 is not tau and torch.equal(tau2, m.get_tau(torch.device("cpu")).float())
     assert torch.equal(beta2, m.get_beta(torch.device("cpu")).float())
     assert not tau2.requires_grad
+
+
+def test_plain_linear_is_a_linear_as_it_comes():
+    """What the few-row projection may take the place of: an nn.Linear without bias,
+    wherever that is held, without hooks and with its own ``forward``."""
+    from prime_moment_attention.attention import _plain_linear
+    make = lambda bias=False: torch.nn.Linear(8, 8, bias=bias)
+    assert _plain_linear(make()) and not _plain_linear(make(True))
+    class Sub(torch.nn.Linear):
+        pass
+    assert not _plain_linear(Sub(8, 8, bias=False))
+    m = make()
+    del m._parameters["bias"]
+    assert not _plain_linear(m)
+    m.bias = torch.ones(8)  # a plain attribute, which forward adds as any other
+    assert not _plain_linear(m)
+    m = make()
+    m.__dict__["bias"] = torch.ones(8)  # ... in front of the parameter's None
+    assert not _plain_linear(m)
+    m = make()
+    handle = m.register_forward_hook(lambda *a: None)
+    assert not _plain_linear(m)
+    handle.remove()
+    assert _plain_linear(m)
+    m.forward = lambda x: x
+    assert not _plain_linear(m)
