@@ -36,21 +36,37 @@ def _same_storage(a, b) -> bool:
     return all(x.data_ptr() == y.data_ptr() for x, y in zip(a, b))
 
 
+_LINEAR_FORWARD = nn.Linear.forward
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """Whether m(x) is x @ weight.T and nothing else: an nn.Linear without bias or hooks
+    whose ``forward`` nobody has replaced, on the instance (offloading, adapter and
+    quantisation wrappers do) or on the class.  (The bias is looked up where an nn.Linear keeps
+    it: nn.Module's own attribute lookup takes 0.5 us.)"""
+    g, d = torch.nn.modules.module, m.__dict__
+    return (type(m) is nn.Linear and m._parameters.get("bias", m) is None and "bias" not in d and "forward" not in d
+            and nn.Linear.forward is _LINEAR_FORWARD
+            and not (m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks
+                     or g._global_forward_pre_hooks))
+
+
 def _stacked_qkv(mod: nn.Module) -> Optional[torch.Tensor]:
     """The q, k and v weights of an attention module stacked into one
     [(H + 2 Hk) D, hidden] matrix, so that inference projects with one GEMM
     instead of three (the same products: each output column is the same dot
     product).  Cached on the module outside its state dict and rebuilt when a
     weight's storage or version counter changes; None while autograd records
-    through the weights (training keeps the three nn.Linear calls) or when the
-    three differ in dtype or device or carry a bias."""
-    lins = (mod.q_proj, mod.k_proj, mod.v_proj)
-    ws = tuple(m.weight for m in lins)
-    if torch.is_grad_enabled() and any(w.requires_grad for w in ws):
+    through the weights (training keeps the three nn.Linear calls), when the
+    three differ in dtype or device, or when one is more than its weight
+    (_plain_linear: a bias, a hook, a replaced forward, another module)."""
+    mq, mk, mv = mod.q_proj, mod.k_proj, mod.v_proj
+    if not (_plain_linear(mq) and _plain_linear(mk) and _plain_linear(mv)):
         return None
-    q, k, v = ws
-    if (any(m.bias is not None for m in lins) or not q.dtype == k.dtype == v.dtype
-            or not q.device == k.device == v.device):
+    q, k, v = ws = (mq.weight, mk.weight, mv.weight)
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return None
+    if not q.dtype == k.dtype == v.dtype or not q.device == k.device == v.device:
         return None
     # the cache holds the weight tensors themselves, so their storage
     # cannot be freed and reused by a new weight at the same address
@@ -83,21 +99,6 @@ def project_qkv(mod: nn.Module, hidden_states: torch.Tensor):
     linear = _lib.rows_linear if _lib.rows_linear_ok(hidden_states, w) else torch.nn.functional.linear
     qkv = linear(hidden_states, w).view(B, L, H + 2 * Hk, D).transpose(1, 2)
     return qkv[:, :H], qkv[:, H:H + Hk], qkv[:, H + Hk:]
-
-
-_LINEAR_FORWARD = nn.Linear.forward
-
-
-def _plain_linear(m: nn.Module) -> bool:
-    """Whether m(x) is x @ weight.T and nothing else: an nn.Linear without bias or hooks
-    whose ``forward`` nobody has replaced, on the instance (offloading, adapter and
-    quantisation wrappers do) or on the class.  (The bias is looked up where an nn.Linear keeps
-    it: nn.Module's own attribute lookup takes 0.5 us.)"""
-    g, d = torch.nn.modules.module, m.__dict__
-    return (type(m) is nn.Linear and m._parameters.get("bias", m) is None and "bias" not in d and "forward" not in d
-            and nn.Linear.forward is _LINEAR_FORWARD
-            and not (m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks
-                     or g._global_forward_pre_hooks))
 
 
 def project_out(proj: nn.Module, y: torch.Tensor) -> torch.Tensor:

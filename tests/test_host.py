@@ -173,3 +173,26 @@ def test_plain_linear_is_a_linear_as_it_comes():
     assert _plain_linear(m)
     m.forward = lambda x: x
     assert not _plain_linear(m)
+
+
+def test_stacked_qkv_leaves_changed_projections_alone():
+    """A projection that is more than its weight (a hook, a forward set on the instance,
+    another module, with or without a ``weight``) runs as the module it is: no stacked
+    copy, also when one was made before the change."""
+    from prime_moment_attention.attention import PrimeMomentAttention, _stacked_qkv, project_qkv
+    x = torch.randn(1, 3, 64)
+    with torch.no_grad():
+        for name, n in (("q_proj", 0), ("k_proj", 1), ("v_proj", 2)):
+            m = PrimeMomentAttention(64, 2, 32, num_kv_heads=1)
+            assert _stacked_qkv(m) is not None
+            plain = project_qkv(m, x)
+            lin = getattr(m, name)
+            handle = lin.register_forward_hook(lambda mod, i, o: 2 * o)
+            assert _stacked_qkv(m) is None and torch.allclose(project_qkv(m, x)[n], 2 * plain[n], rtol=1e-5)
+            handle.remove()
+            lin.forward = lambda y, lin=lin: 3 * torch.nn.functional.linear(y, lin.weight)
+            assert torch.allclose(project_qkv(m, x)[n], 3 * plain[n], rtol=1e-5)
+            del lin.forward
+            assert _stacked_qkv(m) is not None
+            setattr(m, name, torch.nn.Sequential(lin, torch.nn.Tanh()))
+            assert torch.allclose(project_qkv(m, x)[n], plain[n].tanh(), atol=1e-6)
