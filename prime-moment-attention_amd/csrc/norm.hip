@@ -337,10 +337,11 @@ hipError_t launch_add_rmsnorm(const RmsNormArgs &a, hipStream_t stream) {
 // bf16); as torch ops that read was sigmoid, cast, mean and transposes, 1.36 ms there.
 // A workgroup takes 64 tokens x 4 heads, 8 lanes a row, and turns the sums round in LDS so
 // that each head's tokens are written together.  The tokens of all sequences are numbered
-// through (a workgroup per sequence made a decode batch of 600 one token in 64 each: 40 us).  bf16 and fp16 take the hardware's exp2
-// and reciprocal: after the rounding to 16 bits every input gives torch's sigmoid, but for
-// the three bf16 values near -88 whose sigmoid is subnormal (5e-39), which give 0; fp32 the
-// full forms.
+// through: with a tile per sequence a decode batch worked through 64 rows for each token (600
+// sequences 26 us, 4096 176; now 9 and 8.6).  bf16 and fp16 take the hardware's exp2 and
+// reciprocal: after the rounding to 16 bits every input gives torch's sigmoid, but for the
+// three bf16 values near -88 whose sigmoid is subnormal (5e-39), which give 0; fp32 the full
+// forms.
 namespace {
 constexpr int kGateTok = 64, kGateHeads = 4;
 }

@@ -213,9 +213,10 @@ int device_cus() {
 // 12 x 128 to 96 x 8192 tokens with every G (times within 10 % of the model at the
 // chosen G): there the plan is within 0.5 % of the best G on fp32 and bf16, 6 % at worst
 // (selective bf16, 12 x 1000).  Over 4 to 48 sequences of 1024 to 32,768 tokens it is within 8 %
-// (bf16, 4 x 1024: 19.3 us against 17.9), 14 % for selective bf16 (4 x 4096: 31.0 against 26.9).  12 x 512 fp32: 8 segments 25.9 us, 2 segments 44.3;
-// 12 x 512 bf16: one 20.1, 2 segments 27.3; 96 x 2048 bf16: one 59.8, 2 68.5;
-// 96 x 8192 bf16: 8 160.5, 7 169.8; 48 x 777 selective fp32: 5 56.8, 3 78.8.
+// (bf16, 4 x 1024: 19.3 us against 17.9), 14 % for selective bf16 (4 x 4096: 31.0 against
+// 26.9).  12 x 512 fp32: 8 segments 25.9 us, 2 segments 44.3; 12 x 512 bf16: one 20.1, 2
+// segments 27.3; 96 x 2048 bf16: one 59.8, 2 68.5; 96 x 8192 bf16: 8 160.5, 7 169.8; 48 x 777
+// selective fp32: 5 56.8, 3 78.8.
 namespace {
 
 struct PlanCost {
